@@ -79,32 +79,17 @@ __device__ __forceinline__ T vpick3(int a, T v0, T v1, T v2)
     return a == 0 ? v0 : (a == 1 ? v1 : v2);
 }
 
-// the reference in the frame (a, t1, t2) of a boundary face whose element
-// state is permuted that way (momentum components and slopes): frame
-// component 0 = axis a, 1 = the lower other axis, 2 = the upper one
-__device__ __forceinline__ DevRef permute_ref(const DevRef &R, int a)
+// the reference with its velocity and momentum in the frame (a, t1, t2) of a
+// boundary face normal to axis a (t1 the lower other axis)
+__device__ __forceinline__ DevRef frame_ref(const DevRef &R, int a)
 {
-    DevRef Q;
-    Q.r = R.r; Q.p = R.p; Q.E = R.E; Q.Epp = R.Epp;
-    Q.gam = R.gam; Q.gm1 = R.gm1; Q.gq = R.gq;
-    Q.c0[3] = R.c0[3]; Q.c0[4] = R.c0[4];
-    #pragma unroll
-    for (int i = 3; i < 5; i++) { Q.c0h[i] = R.c0h[i]; Q.c0l[i] = R.c0l[i]; }
-    Q.c0h[0] = vpick3(a, R.c0h[0], R.c0h[1], R.c0h[2]);
-    Q.c0h[1] = vpick3(a, R.c0h[1], R.c0h[0], R.c0h[0]);
-    Q.c0h[2] = vpick3(a, R.c0h[2], R.c0h[2], R.c0h[1]);
-    Q.c0l[0] = vpick3(a, R.c0l[0], R.c0l[1], R.c0l[2]);
-    Q.c0l[1] = vpick3(a, R.c0l[1], R.c0l[0], R.c0l[0]);
-    Q.c0l[2] = vpick3(a, R.c0l[2], R.c0l[2], R.c0l[1]);
+    DevRef Q = R;
     Q.u[0] = vpick3(a, R.u[0], R.u[1], R.u[2]);
     Q.u[1] = vpick3(a, R.u[1], R.u[0], R.u[0]);
     Q.u[2] = vpick3(a, R.u[2], R.u[2], R.u[1]);
     Q.m[0] = vpick3(a, R.m[0], R.m[1], R.m[2]);
     Q.m[1] = vpick3(a, R.m[1], R.m[0], R.m[0]);
     Q.m[2] = vpick3(a, R.m[2], R.m[2], R.m[1]);
-    Q.c0[0] = vpick3(a, R.c0[0], R.c0[1], R.c0[2]);
-    Q.c0[1] = vpick3(a, R.c0[1], R.c0[0], R.c0[0]);
-    Q.c0[2] = vpick3(a, R.c0[2], R.c0[2], R.c0[1]);
     return Q;
 }
 
@@ -125,28 +110,40 @@ __device__ __forceinline__ void load_dev(const S *__restrict__ U, int64_t n, int
     }
 }
 
-// state at a point from its deviation trace t = (dm[3], dE, drho)
+// The pointwise functions below spell out their fused multiply-adds and let
+// the compiler form no others: the result of a point then does not depend on
+// the kernel it is inlined into, and a mesh gives the same bits however its
+// chunks are cut and whichever kernel runs them.
+
+// state at a point from its deviation trace t = (dm[3], dE, drho); x = dE less
+// the kinetic-energy deviation, dp = (gamma - 1) x
 struct DPrim {
     float r, ri, u[3], p, E, cz;
-    float dr, dm[3], du[3], dE, dp;
+    float dr, dm[3], du[3], dE, dp, x;
 };
 
 __device__ __forceinline__ void dev_prim(const DevRef &R, const float *t, DPrim &q)
 {
+    #pragma clang fp contract(off)
     q.dm[0] = t[0]; q.dm[1] = t[1]; q.dm[2] = t[2]; q.dE = t[3]; q.dr = t[4];
     q.r = R.r + q.dr;
     q.ri = rcp(q.r);
     #pragma unroll
     for (int d = 0; d < 3; d++) {
-        q.du[d] = (q.dm[d] - R.u[d] * q.dr) * q.ri;
-        q.u[d] = R.u[d] + q.du[d];
+        const float w = fmaf(-q.dr, R.u[d], q.dm[d]);
+        q.du[d] = w * q.ri;
+        q.u[d] = fmaf(q.ri, w, R.u[d]);
     }
-    const float dk = 0.5f * (q.dm[0] * q.u[0] + q.dm[1] * q.u[1] + q.dm[2] * q.u[2]
-                             + R.m[0] * q.du[0] + R.m[1] * q.du[1] + R.m[2] * q.du[2]);
-    q.dp = R.gm1 * (q.dE - dk);
-    q.p = R.p + q.dp;
+    float k = q.dm[1] * q.u[1];
+    k = fmaf(q.dm[0], q.u[0], k);
+    k = fmaf(q.dm[2], q.u[2], k);
+    #pragma unroll
+    for (int d = 0; d < 3; d++) k = fmaf(q.du[d], R.m[d], k);
+    q.x = fmaf(-0.5f, k, q.dE);
+    q.dp = R.gm1 * q.x;
+    q.p = fmaf(R.gm1, q.x, R.p);
     q.E = R.E + q.dE;
-    q.cz = dsqrt(R.gam * q.p * q.ri);
+    q.cz = dsqrt(q.ri * (R.gam * q.p));
 }
 
 // deviation state of a full primitive state (exterior states of boundary
@@ -179,123 +176,113 @@ __device__ __forceinline__ void prim_of_dev(const DevParams &P, const DevRef &R,
     p.c[0] = 1.f;
 }
 
-// face-frame view (normal axis AX with sign s, tangents T1 < T2)
-struct DFrame {
-    float r, ri, un, ut1, ut2, p, E, cz;
-    float dr, dmn, dmt1, dmt2, dun, dE, dp;
-};
+// Fluxes of two point states across a face normal to axis ax, minus F(U_r);
+// q in the states' component order.  The axis may differ between lanes: the
+// normal components are picked by selects, so that one code path serves the
+// three axes with the components' sums in one order.  (On an interior face
+// dp_R - dp_L is one fused step from the states' x.)
 
-template <int AX>
-__device__ __forceinline__ DFrame dev_frame(const DPrim &q, float s)
-{
-    constexpr int T1 = (AX == 0) ? 1 : 0, T2 = (AX == 2) ? 1 : 2;
-    DFrame f;
-    f.r = q.r; f.ri = q.ri; f.p = q.p; f.E = q.E; f.cz = q.cz;
-    f.un = s * q.u[AX]; f.ut1 = q.u[T1]; f.ut2 = q.u[T2];
-    f.dr = q.dr; f.dE = q.dE; f.dp = q.dp;
-    f.dmn = s * q.dm[AX]; f.dmt1 = q.dm[T1]; f.dmt2 = q.dm[T2];
-    f.dun = s * q.du[AX];
-    return f;
-}
-
-// reference values in the same frame
-struct DRefFrame {
-    float mn, mt1, mt2, Epp, gq, gam;
-};
-
-template <int AX>
-__device__ __forceinline__ DRefFrame dev_ref_frame(const DevRef &R, float s)
-{
-    constexpr int T1 = (AX == 0) ? 1 : 0, T2 = (AX == 2) ? 1 : 2;
-    DRefFrame f;
-    f.mn = s * R.m[AX]; f.mt1 = R.m[T1]; f.mt2 = R.m[T2]; f.Epp = R.Epp; f.gq = R.gq; f.gam = R.gam;
-    return f;
-}
-
-__device__ __forceinline__ DFrame sel_dframe(bool c, const DFrame &a, const DFrame &b)
-{
-    DFrame o;
-    o.r = sel(c, a.r, b.r); o.ri = sel(c, a.ri, b.ri); o.un = sel(c, a.un, b.un); o.ut1 = sel(c, a.ut1, b.ut1); o.ut2 = sel(c, a.ut2, b.ut2);
-    o.p = sel(c, a.p, b.p); o.E = sel(c, a.E, b.E); o.cz = sel(c, a.cz, b.cz);
-    o.dr = sel(c, a.dr, b.dr); o.dmn = sel(c, a.dmn, b.dmn); o.dmt1 = sel(c, a.dmt1, b.dmt1);
-    o.dmt2 = sel(c, a.dmt2, b.dmt2); o.dun = sel(c, a.dun, b.dun); o.dE = sel(c, a.dE, b.dE);
-    o.dp = sel(c, a.dp, b.dp);
-    return o;
-}
-
-// physical flux deviation F_n(U) - F_n(U_r) in the face frame
-// (q = (normal momentum, t1, t2, energy, mass))
-__device__ __forceinline__ void dev_phys(const DFrame &K, const DRefFrame &R, float *q)
-{
-    q[0] = K.dmn * K.un + R.mn * K.dun + K.dp;
-    q[1] = K.dmt1 * K.un + R.mt1 * K.dun;
-    q[2] = K.dmt2 * K.un + R.mt2 * K.dun;
-    q[3] = (K.dE + K.dp) * K.un + R.Epp * K.dun;
-    q[4] = K.dmn;
-}
-
-// HLLC (src/charm_fluxes.c:319-437) minus F(U_r): the upwind branches are
-// the physical flux deviation, the star branch adds S_K (U*_K - U_K) =
+// HLLC (src/charm_fluxes.c:319-437): the upwind branches are the physical flux
+// deviation, the star branch adds S_K (U*_K - U_K) =
 // S_K g (rho_K S_K, rho_K ut1, rho_K ut2, E_K + a_K S* + p_K, rho_K),
 // g = (S* - u_K) / (S_K - S*)
-__device__ __forceinline__ bool hllc_dev(const DFrame &L, const DFrame &Rt, const DRefFrame &rf, float *q)
+template <bool BND>
+__device__ __forceinline__ bool hllc_dev(const DPrim &L, const DPrim &Rt, const DevRef &rf, int ax, float *q)
 {
-    const float p_pvrs = 0.5f * (L.p + Rt.p) - 0.5f * (Rt.un - L.un) * 0.25f * (L.r + Rt.r) * (L.cz + Rt.cz);
-    const float p_star = p_pvrs > 0.f ? p_pvrs : 0.f;
+    #pragma clang fp contract(off)
+    const float unl = vpick3(ax, L.u[0], L.u[1], L.u[2]), unr = vpick3(ax, Rt.u[0], Rt.u[1], Rt.u[2]);
+    const float dnl = vpick3(ax, L.du[0], L.du[1], L.du[2]), dnr = vpick3(ax, Rt.du[0], Rt.du[1], Rt.du[2]);
+    const float pv = 0.5f * (unr - unl) * -0.25f * (L.r + Rt.r) * (L.cz + Rt.cz);
+    const float p_star = fmaxf(0.f, fmaf(0.5f, L.p + Rt.p, pv));
     // c_K q_K with q_K = sqrt(1 + gq (p* / p_K - 1)) for p* > p_K, else 1, as
     // one root: c_K q_K = sqrt(gamma / rho_K (p_K + gq max(p* - p_K, 0)))
-    float sl = L.un - dsqrt(rf.gam * L.ri * (L.p + rf.gq * fmaxf(p_star - L.p, 0.f)));
-    float sr = Rt.un + dsqrt(rf.gam * Rt.ri * (Rt.p + rf.gq * fmaxf(p_star - Rt.p, 0.f)));
+    float sl = unl - dsqrt(rf.gam * L.ri * fmaf(rf.gq, fmaxf(0.f, p_star - L.p), L.p));
+    float sr = unr + dsqrt(rf.gam * Rt.ri * fmaf(rf.gq, fmaxf(0.f, p_star - Rt.p), Rt.p));
     if (sl > sr) { const float t = sl; sl = sr; sr = t; }
-    const float al = L.r * (sl - L.un), ar = Rt.r * (sr - Rt.un);
-    const float dpn = Rt.dp - L.dp, dun = Rt.dun - L.dun;
-    const float den = rcp(al - ar);
-    float dl = (dpn - ar * dun) * den;              // S* - u_L
-    float dr = (dpn - al * dun) * den;              // S* - u_R
-    float s_star = L.un + dl;
-    if (s_star < sl) { s_star = sl; dl = sl - L.un; dr = sl - Rt.un; }
-    if (s_star > sr) { s_star = sr; dl = sr - L.un; dr = sr - Rt.un; }
+    const float wl = sl - unl, wr = sr - unr, al = L.r * wl, ar = Rt.r * wr;
+    const float dpn = BND ? Rt.dp - L.dp : fmaf(rf.gm1, Rt.x, -L.dp), dun = dnr - dnl;
+    const float den = rcp(fmaf(L.r, wl, -ar));
+    const float nl = fmaf(-dun, ar, dpn);
+    float dl = nl * den;                            // S* - u_L
+    float dr = fmaf(-dun, al, dpn) * den;           // S* - u_R
+    float s_star = fmaf(nl, den, unl);
+    if (s_star < sl) { s_star = sl; dl = wl; dr = sl - unr; }
+    if (s_star > sr) { s_star = sr; dl = sr - unl; dr = wr; }
     const bool ok = (sl <= s_star) && (s_star <= sr);
     // one branch-free body: the upwind side of a supersonic face (sl >= 0:
     // left, sr <= 0: right) with no star term, else the star region of the
     // side s* falls on
     const bool sup = (sl >= 0.f) || (sr <= 0.f);
     const bool left = (sl >= 0.f) || (!(sr <= 0.f) && s_star >= 0.f);
-    const DFrame K = sel_dframe(left, L, Rt);
+    const float un = sel(left, unl, unr), dn = sel(left, dnl, dnr), r = sel(left, L.r, Rt.r), p = sel(left, L.p, Rt.p);
+    const float E = sel(left, L.E, Rt.E), dE = sel(left, L.dE, Rt.dE), dp = sel(left, L.dp, Rt.dp);
     const float sk = left ? sl : sr, dk = left ? dl : dr;
-    dev_phys(K, rf, q);
     const float sg = sup ? 0.f : sk * dk * rcp(sk - s_star);          // S_K g
-    const float ak = K.r * (sk - K.un);
-    q[0] += sg * (K.r * sk);
-    q[1] += sg * (K.r * K.ut1);
-    q[2] += sg * (K.r * K.ut2);
-    q[3] += sg * (K.E + ak * s_star + K.p);
-    q[4] += sg * K.r;
+    float dm[3];
+    #pragma unroll
+    for (int j = 0; j < 3; j++) dm[j] = sel(left, L.dm[j], Rt.dm[j]);
+    const float dmn = vpick3(ax, dm[0], dm[1], dm[2]);
+    const float mn = vpick3(ax, rf.m[0], rf.m[1], rf.m[2]);
+    const float qn = fmaf(r * sk, sg, fmaf(mn, dn, un * dmn) + dp);
+    #pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const float u = sel(left, L.u[j], Rt.u[j]);
+        const float qt = fmaf(r * u, sg, fmaf(un, dm[j], dn * rf.m[j]));
+        q[j] = ax == j ? qn : qt;
+    }
+    q[3] = fmaf(dn, rf.Epp, un * (dp + dE));
+    q[3] = fmaf(sg, p + fmaf(s_star, r * (sk - un), E), q[3]);
+    q[4] = fmaf(r, sg, dmn);
     return ok;
 }
 
-// Lax-Friedrichs / central (src/charm_fluxes.c:255-315, 513-559) minus F(U_r)
-__device__ __forceinline__ void lf_dev(const DFrame &L, const DFrame &Rt, const DRefFrame &rf, float *q,
+// Lax-Friedrichs / central (src/charm_fluxes.c:255-315, 513-559)
+__device__ __forceinline__ void lf_dev(const DPrim &L, const DPrim &Rt, const DevRef &rf, int ax, float *q,
                                        bool central)
 {
-    float fl[5], fr[5];
-    dev_phys(L, rf, fl);
-    dev_phys(Rt, rf, fr);
-    const float alpha = central ? 0.f : fmaxf(fabsf(L.un) + L.cz, fabsf(Rt.un) + Rt.cz);
-    q[0] = 0.5f * (fr[0] + fl[0] - alpha * (Rt.dmn - L.dmn));
-    q[1] = 0.5f * (fr[1] + fl[1] - alpha * (Rt.dmt1 - L.dmt1));
-    q[2] = 0.5f * (fr[2] + fl[2] - alpha * (Rt.dmt2 - L.dmt2));
-    q[3] = 0.5f * (fr[3] + fl[3] - alpha * (Rt.dE - L.dE));
-    q[4] = 0.5f * (fr[4] + fl[4] - alpha * (Rt.dr - L.dr));
+    #pragma clang fp contract(off)
+    float f[2][5], un[2];
+    #pragma unroll
+    for (int s = 0; s < 2; s++) {
+        const DPrim &K = s ? Rt : L;
+        un[s] = vpick3(ax, K.u[0], K.u[1], K.u[2]);
+        const float dn = vpick3(ax, K.du[0], K.du[1], K.du[2]);
+        #pragma unroll
+        for (int j = 0; j < 3; j++) f[s][j] = fmaf(K.dm[j], un[s], rf.m[j] * dn) + (ax == j ? K.dp : 0.f);
+        f[s][3] = fmaf(rf.Epp, dn, un[s] * (K.dE + K.dp));
+        f[s][4] = vpick3(ax, K.dm[0], K.dm[1], K.dm[2]);
+    }
+    const float alpha = central ? 0.f : fmaxf(fabsf(un[0]) + L.cz, fabsf(un[1]) + Rt.cz);
+    #pragma unroll
+    for (int j = 0; j < 3; j++) q[j] = 0.5f * fmaf(-alpha, Rt.dm[j] - L.dm[j], f[1][j] + f[0][j]);
+    q[3] = 0.5f * fmaf(-alpha, Rt.dE - L.dE, f[1][3] + f[0][3]);
+    q[4] = 0.5f * fmaf(-alpha, Rt.dr - L.dr, f[1][4] + f[0][4]);
 }
 
-template <int FLUX>
-__device__ __forceinline__ bool flux_dev(const DFrame &L, const DFrame &Rt, const DRefFrame &rf, float *q)
+// flux deviations along the three axes at a volume point
+__device__ __forceinline__ void phys_dev(const DPrim &q, const DevRef &rf, float (*F)[5])
+{
+    #pragma clang fp contract(off)
+    const float h = fmaf(rf.gm1, q.x, q.dE);               // dE + dp
+    #pragma unroll
+    for (int d = 0; d < 3; d++) {
+        #pragma unroll
+        for (int j = 0; j < 3; j++) {
+            F[d][j] = fmaf(q.du[j], rf.m[d], q.dm[d] * q.u[j]);
+            if (d == j) F[d][j] = fmaf(rf.gm1, q.x, F[d][j]);
+        }
+        F[d][3] = fmaf(q.du[d], rf.Epp, q.u[d] * h);
+        F[d][4] = q.dm[d];
+    }
+}
+
+template <int FLUX, bool BND>
+__device__ __forceinline__ bool flux_dev(const DPrim &L, const DPrim &Rt, const DevRef &rf, int ax, float *q)
 {
     if constexpr (FLUX == FLUX_HLLC) {
-        return hllc_dev(L, Rt, rf, q);
+        return hllc_dev<BND>(L, Rt, rf, ax, q);
     } else {
-        lf_dev(L, Rt, rf, q, FLUX == FLUX_CD);
+        lf_dev(L, Rt, rf, ax, q, FLUX == FLUX_CD);
         return true;
     }
 }

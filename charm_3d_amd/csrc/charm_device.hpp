@@ -98,6 +98,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t var_rsrc(const S *U, int64_t n
                                              0x00020000);
 }
 
+// the value at byte offset `off` of variable v's planes (the lane picks the plane)
+template <typename S>
+__device__ __forceinline__ S ldo(const S *U, int64_t n, int v, int off)
+{
+    const __amdgpu_buffer_rsrc_t r = var_rsrc(U, n, v);
+    if constexpr (sizeof(S) == 8) return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    else return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+
 // i = 4 v + k
 template <typename S>
 __device__ __forceinline__ S ldp(const S *U, int64_t n, int i, int e)
@@ -464,6 +473,18 @@ __device__ __forceinline__ Frame<R, NC> to_frame(const Prim<R, NC> &p, R n0, R n
     f.un = p.u * n0 + p.v * n1 + p.w * n2;
     f.ut1 = p.u * t10 + p.v * t11 + p.w * t12;
     f.ut2 = p.u * t20 + p.v * t21 + p.w * t22;
+    #pragma unroll
+    for (int i = 0; i < NC; i++) f.c[i] = p.c[i];
+    return f;
+}
+
+// the flux's view of a state whose velocity is already in the face's frame
+template <typename R, int NC>
+__device__ __forceinline__ Frame<R, NC> frame_state(const Prim<R, NC> &p)
+{
+    Frame<R, NC> f;
+    f.r = p.r; f.e_tot = p.e_tot; f.p = p.p; f.cz = p.cz; f.gam = p.gam;
+    f.un = p.u; f.ut1 = p.v; f.ut2 = p.w;
     #pragma unroll
     for (int i = 0; i < NC; i++) f.c[i] = p.c[i];
     return f;

@@ -73,108 +73,158 @@ __device__ __forceinline__ void to_xyz(int a, R n, R t1, R t2, R &x, R &y, R &z)
     z = (a == 2) ? n : t2;
 }
 
-// Moments of one face normal to axis AX from the two element states u0, u1
-// (u1 unused on a boundary face):
-// out[3][NV] = wJ * (sum q, sum q phi_t1, sum q phi_t2) over the six points,
-// phi_t the tangential Taylor coordinates of the small (or side-0) face.
-// DEV: u0, u1 hold deviations from the chunk reference *rf (coefficient 0
-// minus the reference) and q is F - F(U_r) (charm_dev.hpp).
-// tl / tr (PH = 1, may be null): the EOS closure of side 0 / 1 at point k
-// from the point pass starts at tl[k * ts] / tr[k * ts], its planes
-// kMemoRows * ts apart (global memory: the point loop is not unrolled, so a
-// local array would sit in scratch)
-template <typename R, int NC, int FLUX, int AX, bool BND, int PH, bool DEV = false>
-__device__ __forceinline__ bool face_core(const DevParams &P, const R *u0, const R *u1, int info,
-                                          int lown, R *out, int bnd_axis, const DevRef &rf,
-                                          const R *tl = nullptr, const R *tr = nullptr,
-                                          int64_t ts = 0)
+// Element coefficients for a face normal to axis ax: the slopes in the face's
+// order (n, t1 < t2), so that one code path serves the faces of all three
+// axes and a wave that straddles two orientations does not run the face code
+// twice (with the axis as a template argument 0.84 of the lanes were active at
+// level 7 in FP32, 0.65 at level 6 in FP64).  The kernel is bound by VALU
+// issue: 458 -> 422 us at 2,097,152 leaves in FP32, 152 -> 141 us at 262,144
+// in FP64.  The planes are picked by the lane's byte offset.  The momentum components keep their order in the
+// deviation form (DEV; deviations from the reference, as load_dev), whose
+// flux picks the normal ones; else they follow into the frame by selects.
+template <typename R>
+__device__ __forceinline__ void frame_momentum(int ax, R *u)
+{
+    #pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const R x = u[k], y = u[4 + k], z = u[8 + k];
+        u[k] = vpick3(ax, x, y, z);
+        u[4 + k] = ax == 0 ? y : x;
+        u[8 + k] = ax == 2 ? y : z;
+    }
+}
+
+template <typename S, typename R, int NC, bool DEV>
+__device__ __forceinline__ void load_frame(const S *__restrict__ U, int64_t n, int e, int ax, const DevRef &rf, R *u)
 {
     constexpr int NV = 4 + NC;
-    constexpr int T1 = (AX == 0) ? 1 : 0, T2 = (AX == 2) ? 1 : 2;
-    const int dir0 = info & 7, kind = (info >> 3) & 3, sub = (info >> 5) & 3;
-    const R s = (dir0 & 1) ? R(1) : R(-1);              // outward normal of side 0
+    const int np = (int) (n * (int64_t) sizeof(S)), o0 = e * (int) sizeof(S);
+    const int off[4] = {o0, o0 + (ax == 0 ? np : (ax == 1 ? 2 * np : 3 * np)), o0 + (ax == 0 ? 2 * np : np),
+                        o0 + (ax == 2 ? 2 * np : 3 * np)};
+    #pragma unroll
+    for (int v = 0; v < NV; v++)
+        #pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const S x = ldo<S>(U, n, v, off[k]);
+            if constexpr (DEV && sizeof(S) == 4) u[4 * v + k] = k ? x : (x - rf.c0h[v]) - rf.c0l[v];
+            else if constexpr (DEV) u[4 * v + k] = k ? (float) x : (float) ((double) x - rf.c0[v]);
+            else u[4 * v + k] = (R) x;
+        }
+    if constexpr (!DEV) frame_momentum<R>(ax, u);
+}
+
+// The points of a face in its two sides' coordinates: scale and tangential
+// offsets.  The big side of a hanging face sees the small face's points at
+// delta + offset / 2 in its own units.
+template <typename R>
+struct FaceMap {
+    R m0, o01, o02, m1, o11, o12;
+    __device__ __forceinline__ FaceMap(int kind, int sub)
+    {
+        const R d1 = (sub & 1) ? R(0.25) : R(-0.25), d2 = (sub & 2) ? R(0.25) : R(-0.25);
+        const bool big0 = kind == FACE_HANG1, big1 = kind == FACE_HANG0;
+        m0 = big0 ? R(0.5) : R(1); m1 = big1 ? R(0.5) : R(1);
+        o01 = big0 ? d1 : R(0); o02 = big0 ? d2 : R(0);
+        o11 = big1 ? d1 : R(0); o12 = big1 ? d2 : R(0);
+    }
+};
+
+// the value on the face (its normal-direction part is the same at all points)
+// takes coefficient 0's place
+template <typename R, int NV>
+__device__ __forceinline__ void to_face(R pn, R *u)
+{
+    #pragma unroll
+    for (int v = 0; v < NV; v++) u[4*v] = fma(pn, u[4*v+1], u[4*v]);
+}
+
+template <typename R, int NV>
+__device__ __forceinline__ void face_trace(const R *u, R q1, R q2, R *t)
+{
+    #pragma unroll
+    for (int v = 0; v < NV; v++) t[v] = fma(q2, u[4*v+3], fma(q1, u[4*v+2], u[4*v]));
+}
+
+// The flux q at the face point of offsets g1, g2 from the two sides (to_face;
+// u1 unused on a boundary face, whose state and normal are mirrored so that
+// the outward normal is +n), in the frame; DEV: q is F - F(U_r) (charm_dev.hpp),
+// in the frame on a boundary face, in global order (normal axis ax) on others.
+// dir0, s: the boundary face's direction and outward sign along its axis.
+// tl / tr (PH = 1, may be null): each side's EOS closure at this point from
+// the point pass, its planes kMemoRows * ts apart
+template <typename R, int NC, int FLUX, bool BND, int PH, bool DEV>
+__device__ __forceinline__ bool point_flux(const DevParams &P, const R *u0, const R *u1, const FaceMap<R> &fm, R g1, R g2, int dir0, R s,
+                                           const DevRef &rf, const R *tl, const R *tr, int64_t ts, R *q)
+{
+    constexpr int NV = 4 + NC;
+    R t[NV];
+    face_trace<R, NV>(u0, BND ? g1 : fma(fm.m0, g1, fm.o01), BND ? g2 : fma(fm.m0, g2, fm.o02), t);
+    if constexpr (DEV) {
+        DPrim dl, dr;
+        dev_prim(rf, t, dl);
+        if (BND) {
+            if (P.bnd_type[dir0] == BND_OUTLET) {
+                dr = dl;                   // transmissive: the exterior state is the interior one
+            } else {
+                Prim<float, 1> pl, pr;
+                prim_of_dev(P, rf, dl, pl);
+                pl.u *= s;
+                bnd_state<float, 1, 0>(P, dir0, 0, s, pl, pr, dir0 >> 1);
+                pr.u *= s;
+                dev_from_prim(rf, pr, dr);
+            }
+        } else {
+            face_trace<R, NV>(u1, fma(fm.m1, g1, fm.o11), fma(fm.m1, g2, fm.o12), t);
+            dev_prim(rf, t, dr);
+        }
+        return flux_dev<FLUX, BND>(dl, dr, rf, BND ? 0 : dir0 >> 1, q);
+    } else {
+        Prim<R, NC> pl, pr;
+        cons_to_prim<R, NC, PH>(P, t, pl, tl, kMemoRows * ts);
+        if (BND) {
+            pl.u *= s;
+            bnd_state<R, NC, PH>(P, dir0, 0, s, pl, pr, dir0 >> 1);
+            pl.u *= s;
+            pr.u *= s;
+        } else {
+            face_trace<R, NV>(u1, fma(fm.m1, g1, fm.o11), fma(fm.m1, g2, fm.o12), t);
+            cons_to_prim<R, NC, PH>(P, t, pr, tr, kMemoRows * ts);
+        }
+        return flux_x<R, NC, FLUX>(frame_state(pl), frame_state(pr), q);
+    }
+}
+
+// Moments of one face from its two element states in the face's frame
+// (load_frame): out[3][NV] = wJ * (sum q, sum q phi_t1, sum q phi_t2) over the
+// six points, q and phi in the frame, phi_t the tangential Taylor coordinates
+// of the small (or side-0) face.  tl / tr as point_flux's for point k at
+// tl[k * ts] (global memory: the point loop is not unrolled, so a local array
+// would sit in scratch).
+template <typename R, int NC, int FLUX, bool BND, int PH, bool DEV>
+__device__ __forceinline__ bool face_core(const DevParams &P, R *u0, R *u1, int kind, int sub, int dir0, R s,
+                                          int lown, R *out, const DevRef &rf, const R *tl = nullptr,
+                                          const R *tr = nullptr, int64_t ts = 0)
+{
+    constexpr int NV = 4 + NC;
     const R h = ldexp(R(1), -lown);
     const R wj = h * h * R(1.0 / 6.0);
-    // normal-basis values on the face: side 0 at +-1/2 by its face parity
-    const R pa0 = R(0.5) * s, pa1 = -pa0;
-    // the big side of a hanging face sees the small face's points at
-    // delta + offset / 2 in its own units
-    const R d1 = (sub & 1) ? R(0.25) : R(-0.25);
-    const R d2 = (sub & 2) ? R(0.25) : R(-0.25);
-    const bool big0 = (kind == FACE_HANG1), big1 = (kind == FACE_HANG0);
-    const R m0 = big0 ? R(0.5) : R(1), m1 = big1 ? R(0.5) : R(1);
-    const R o01 = big0 ? d1 : R(0), o02 = big0 ? d2 : R(0);
-    const R o11 = big1 ? d1 : R(0), o12 = big1 ? d2 : R(0);
     R S0[NV], S1[NV], S2[NV];
     #pragma unroll
     for (int v = 0; v < NV; v++) { S0[v] = R(0); S1[v] = R(0); S2[v] = R(0); }
-    // the normal-direction part of each trace is the same at all six points
-    R c0[NV], c1[NV];
-    #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        c0[v] = u0[4*v] + pa0 * u0[4*v+1+AX];
-        c1[v] = BND ? R(0) : u1[4*v] + pa1 * u1[4*v+1+AX];
-    }
+    to_face<R, NV>(R(0.5), u0);
+    if (!BND) to_face<R, NV>(R(-0.5), u1);
+    const FaceMap<R> fm(kind, sub);
     bool ok = true;
     // a rolled loop over the points (k is wave-uniform: the point's constants
     // are scalar selects): a fifth of the unrolled code and fewer registers
     #pragma unroll 1
     for (int k = 0; k < 6; k++) {
         const R g1 = gp_t1<R>(k), g2 = gp_t2<R>(k);
-        R t[NV];
+        R q[NV];
+        ok &= point_flux<R, NC, FLUX, BND, PH, DEV>(P, u0, u1, fm, g1, g2, dir0, s, rf, tl ? tl + k * ts : nullptr,
+                                                    tr ? tr + k * ts : nullptr, ts, q);
         #pragma unroll
-        for (int v = 0; v < NV; v++)
-            t[v] = c0[v] + (o01 + m0 * g1) * u0[4*v+1+T1] + (o02 + m0 * g2) * u0[4*v+1+T2];
-        R q[NV], qg[NV];
-        if constexpr (DEV) {
-            DPrim dl, dr;
-            dev_prim(rf, t, dl);
-            if (BND) {
-                if (P.bnd_type[dir0] == BND_OUTLET) {
-                    dr = dl;                   // transmissive: the exterior state is the interior one
-                } else {
-                    Prim<float, 1> pl, pr;
-                    prim_of_dev(P, rf, dl, pl);
-                    bnd_state<float, 1, 0>(P, dir0, AX, s, pl, pr, bnd_axis);
-                    dev_from_prim(rf, pr, dr);
-                }
-            } else {
-                #pragma unroll
-                for (int v = 0; v < NV; v++)
-                    t[v] = c1[v] + (o11 + m1 * g1) * u1[4*v+1+T1] + (o12 + m1 * g2) * u1[4*v+1+T2];
-                dev_prim(rf, t, dr);
-            }
-            ok &= flux_dev<FLUX>(dev_frame<AX>(dl, s), dev_frame<AX>(dr, s), dev_ref_frame<AX>(rf, s), q);
-        } else {
-        Prim<R, NC> pl, pr;
-        cons_to_prim<R, NC, PH>(P, t, pl, tl ? tl + k * ts : nullptr, kMemoRows * ts);
-        if (BND) {
-            bnd_state<R, NC, PH>(P, dir0, AX, s, pl, pr, bnd_axis);
-        } else {
-            #pragma unroll
-            for (int v = 0; v < NV; v++)
-                t[v] = c1[v] + (o11 + m1 * g1) * u1[4*v+1+T1] + (o12 + m1 * g2) * u1[4*v+1+T2];
-            cons_to_prim<R, NC, PH>(P, t, pr, tr ? tr + k * ts : nullptr, kMemoRows * ts);
-        }
-        // face frame (s e_AX, e_T1, e_T2)
-        Frame<R, NC> fl, fr;
-        {
-            const R vl[3] = {pl.u, pl.v, pl.w}, vr[3] = {pr.u, pr.v, pr.w};
-            fl.r = pl.r; fl.e_tot = pl.e_tot; fl.p = pl.p; fl.cz = pl.cz; fl.gam = pl.gam;
-            fr.r = pr.r; fr.e_tot = pr.e_tot; fr.p = pr.p; fr.cz = pr.cz; fr.gam = pr.gam;
-            fl.un = s * vl[AX]; fr.un = s * vr[AX];
-            fl.ut1 = vl[T1]; fr.ut1 = vr[T1];
-            fl.ut2 = vl[T2]; fr.ut2 = vr[T2];
-            #pragma unroll
-            for (int i = 0; i < NC; i++) { fl.c[i] = pl.c[i]; fr.c[i] = pr.c[i]; }
-        }
-        ok &= flux_x<R, NC, FLUX>(fl, fr, q);
-        }
-        qg[AX] = s * q[0]; qg[T1] = q[1]; qg[T2] = q[2];
-        #pragma unroll
-        for (int v = 3; v < NV; v++) qg[v] = q[v];
-        #pragma unroll
-        for (int v = 0; v < NV; v++) { S0[v] += qg[v]; S1[v] += qg[v] * g1; S2[v] += qg[v] * g2; }
+        for (int v = 0; v < NV; v++) { S0[v] += q[v]; S1[v] = fma(q[v], g1, S1[v]); S2[v] = fma(q[v], g2, S2[v]); }
     }
     #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -182,87 +232,133 @@ __device__ __forceinline__ bool face_core(const DevParams &P, const R *u0, const
         out[NV + v] = S1[v] * wj;
         out[2 * NV + v] = S2[v] * wj;
     }
+    if (BND) {
+        #pragma unroll
+        for (int m = 0; m < 3; m++) out[m * NV] *= s;
+    }
     return ok;
 }
 
-// interior face from the two preloaded element states; the small side's
-// level sets the face size
-template <typename R, int NC, int FLUX, int AX, int PH, bool DEV = false>
-__device__ __forceinline__ bool face_moments(const DevParams &P, const R *u0, const R *u1, int info,
-                                             int lev0, R *out, const DevRef &rf, const R *tl = nullptr,
-                                             const R *tr = nullptr, int64_t ts = 0)
+// a boundary face's state and reference in its frame, mirrored to the outward
+// normal +n
+template <typename R, int NV, bool DEV>
+__device__ __forceinline__ void mirror_side(int ax, R s, R *u, DevRef &rf)
 {
-    const int kind = (info >> 3) & 3;
-    return face_core<R, NC, FLUX, AX, false, PH, DEV>(P, u0, u1, info, kind == FACE_HANG1 ? lev0 + 1 : lev0, out,
-                                                      AX, rf, tl, tr, ts);
+    if constexpr (DEV) {
+        frame_momentum<R>(ax, u);
+        rf = frame_ref(rf, ax);
+    }
+    #pragma unroll
+    for (int v = 0; v < NV; v++) u[4*v+1] *= s;
+    #pragma unroll
+    for (int k = 0; k < 4; k++) u[k] *= s;
+    if constexpr (DEV) { rf.u[0] *= s; rf.m[0] *= s; }
 }
 
-// Boundary faces: the element state is rotated into the frame (a, t1, t2)
-// of its face (Taylor slopes and momentum components permuted), evaluated
-// with the x-normal code, and the momentum moments are rotated back; one
-// code path serves the three axes.
-template <typename R, int NC, int FLUX, int PH, bool DEV = false>
-__device__ __forceinline__ bool face_moments_bnd(const DevParams &P, const R *u, int info, int lev, R *out,
-                                                 const DevRef &rf, const R *tl = nullptr, int64_t ts = 0)
+// PH = 1: each side's point EOS closures from the point pass, at the side's
+// own (sub)face slot 4 d + j (point k at k * n), or null
+template <typename R, int PH>
+__device__ __forceinline__ void face_closures(const StageArgs &A, int4 rec, const R *&tl, const R *&tr)
+{
+    tl = tr = nullptr;
+    if (PH == 1 && A.tpt) {
+        const R *TP = reinterpret_cast<const R *>(A.tpt);
+        const int64_t n = A.n_elem;
+        const int dir0 = rec.z & 7, kind = (rec.z >> 3) & 3, sub = (rec.z >> 5) & 3;
+        const int s0 = 4 * dir0 + (kind == FACE_HANG1 ? sub : 0);
+        const int s1 = 4 * (dir0 ^ 1) + (kind == FACE_HANG0 ? sub : 0);
+        tl = TP + (int64_t) 6 * s0 * n + rec.x;
+        if (kind != FACE_BND) tr = TP + (int64_t) 6 * s1 * n + rec.y;
+    }
+}
+
+// One face record of a chunk: its moments into dst[3][NV] (global momentum
+// order)
+template <typename S, typename R, int NC, int FLUX, int PH, bool DEV>
+__device__ __forceinline__ bool face_record(const DevParams &P, const S *__restrict__ U, int64_t n, int4 rec,
+                                            int lev0, const DevRef &rf, R *dst, const R *tl, const R *tr)
 {
     constexpr int NV = 4 + NC;
-    const int ax = (info & 7) >> 1;
-    R w[4 * NV];
-    #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        // source variable: momentum components follow the axis permutation
-        R c[4];
-        #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (v < 3) {
-                const R x0 = u[4 * 0 + k], x1 = u[4 * 1 + k], x2 = u[4 * 2 + k];
-                // frame var v -> global var: v=0 -> ax, v=1 -> t1, v=2 -> t2
-                const int gv = (v == 0) ? ax : ((v == 1) ? (ax == 0 ? 1 : 0) : (ax == 2 ? 1 : 2));
-                c[k] = (gv == 0) ? x0 : ((gv == 1) ? x1 : x2);
-            } else {
-                c[k] = u[4 * v + k];
-            }
-        }
-        const R ca = (ax == 0) ? c[1] : ((ax == 1) ? c[2] : c[3]);
-        const R ct1 = (ax == 0) ? c[2] : c[1];
-        const R ct2 = (ax == 2) ? c[2] : c[3];
-        w[4 * v] = c[0]; w[4 * v + 1] = ca; w[4 * v + 2] = ct1; w[4 * v + 3] = ct2;
-    }
-    R o[3 * NV];
+    const int dir0 = rec.z & 7, kind = (rec.z >> 3) & 3, sub = (rec.z >> 5) & 3, ax = dir0 >> 1;
+    R ua[4 * NV], o[3 * NV];
+    load_frame<S, R, NC, DEV>(U, n, rec.x, ax, rf, ua);
     bool ok;
-    if constexpr (DEV) {
-        // the chunk reference in the face's frame, like the state
-        ok = face_core<R, NC, FLUX, 0, true, PH, true>(P, w, w, info, lev, o, ax, permute_ref(rf, ax));
+    if (kind == FACE_BND) {
+        const R s = (dir0 & 1) ? R(1) : R(-1);
+        DevRef rx = rf;
+        mirror_side<R, NV, DEV>(ax, s, ua, rx);
+        ok = face_core<R, NC, FLUX, true, PH, DEV>(P, ua, ua, kind, sub, dir0, s, lev0, o, rx, tl, nullptr, n);
     } else {
-        ok = face_core<R, NC, FLUX, 0, true, PH>(P, w, w, info, lev, o, ax, rf, tl, nullptr, ts);
+        // side 0 of an interior face is the leaf on the lower side: s = +1
+        R ub[4 * NV];
+        load_frame<S, R, NC, DEV>(U, n, rec.y, ax, rf, ub);
+        ok = face_core<R, NC, FLUX, false, PH, DEV>(P, ua, ub, kind, sub, dir0, R(1),
+                                                    kind == FACE_HANG1 ? lev0 + 1 : lev0, o, rf, tl, tr, n);
     }
+    // the frame's momentum moments back to global order by the LDS address
+    const bool fr = !DEV || kind == FACE_BND;
+    const int g0 = fr ? ax : 0, g1 = fr ? (ax == 0 ? 1 : 0) : 1, g2 = fr ? (ax == 2 ? 1 : 2) : 2;
     #pragma unroll
     for (int m = 0; m < 3; m++) {
-        const R f0 = o[m * NV + 0], f1 = o[m * NV + 1], f2 = o[m * NV + 2];
-        // global var g takes frame var: g == ax -> 0, g == t1 -> 1, g == t2 -> 2
-        out[m * NV + 0] = (ax == 0) ? f0 : f1;
-        out[m * NV + 1] = (ax == 1) ? f0 : ((ax == 0) ? f1 : f2);
-        out[m * NV + 2] = (ax == 2) ? f0 : f2;
+        dst[m * NV + g0] = o[m * NV];
+        dst[m * NV + g1] = o[m * NV + 1];
+        dst[m * NV + g2] = o[m * NV + 2];
         #pragma unroll
-        for (int v = 3; v < NV; v++) out[m * NV + v] = o[m * NV + v];
+        for (int v = 3; v < NV; v++) dst[m * NV + v] = o[m * NV + v];
     }
     return ok;
 }
 
-// volume integral, src/models/euler/charm_model.c:66-132: with the Taylor
+// The volume integral, src/models/euler/charm_model.c:66-132: with the Taylor
 // basis on a cube, grad phi_k = e_k / h and phi_k(gp) = +-1/(2 sqrt 3), so
 // int[v][1+d] -= (wJ/h) sum_gp F_d,v and the gravity term adds
 // -g_v sum_gp rho phi_k wJ.
-// tv (PH = 1, may be null): the EOS closure at volume point g starts at
-// tv[g * ts], its planes kMemoRows * ts apart
-template <typename R, int NC, int PH>
-__device__ __forceinline__ void volume_integral(const DevParams &P, const R *u, R h, R *res,
-                                                const R *tv = nullptr, int64_t ts = 0)
+// volume_terms: the fluxes F_d at one Gauss point (signs of g) and the density
+// there.  DEV: u holds deviation coefficients and F is F - F(U_r), the
+// momentum, energy and mass fluxes along each axis as in dev_phys; the gravity
+// term takes the full density.
+// tk (PH = 1, may be null): the point's EOS closure, its planes kMemoRows * ts
+// apart
+template <typename R, int NC, int PH, bool DEV>
+__device__ __forceinline__ R volume_terms(const DevParams &P, const R *u, int g, const DevRef &rf, const R *tk,
+                                          int64_t ts, R (*F)[4 + NC])
 {
     constexpr int NV = 4 + NC;
     const R ph = R(0.28867513459481288225);           // 1/(2 sqrt 3)
-    const R hinv = rcp(h);
-    const R wj = h * h * h * R(0.125);
+    const R px = (g & 1) ? ph : -ph, py = (g & 2) ? ph : -ph, pz = (g & 4) ? ph : -ph;
+    R t[NV];
+    trace<R, NV>(u, px, py, pz, t);
+    if constexpr (DEV) {
+        DPrim q;
+        dev_prim(rf, t, q);
+        phys_dev(q, rf, F);
+        return q.r;
+    } else {
+        Prim<R, NC> p;
+        cons_to_prim<R, NC, PH>(P, t, p, tk, kMemoRows * ts);
+        const R vel[3] = {p.u, p.v, p.w};
+        #pragma unroll
+        for (int d = 0; d < 3; d++) {
+            F[d][0] = t[d] * p.u + (d == 0 ? p.p : R(0));
+            F[d][1] = t[d] * p.v + (d == 1 ? p.p : R(0));
+            F[d][2] = t[d] * p.w + (d == 2 ? p.p : R(0));
+            F[d][3] = t[d] * p.e_tot + p.p * vel[d];
+            #pragma unroll
+            for (int i = 0; i < NC; i++) F[d][4 + i] = t[d] * p.c[i];
+        }
+        return p.r;
+    }
+}
+
+// tv (PH = 1, may be null): the EOS closure at volume point g starts at
+// tv[g * ts]
+template <typename R, int NC, int PH, bool DEV>
+__device__ __forceinline__ void volume_integral(const DevParams &P, const R *u, R h, const DevRef &rf, R *res,
+                                                const R *tv = nullptr, int64_t ts = 0)
+{
+    constexpr int NV = 4 + NC;
+    const R ph = R(0.28867513459481288225);
+    const R wj = h * h * h * R(0.125), f = wj * rcp(h);
     R SF[3][NV];
     R G[4] = {R(0), R(0), R(0), R(0)};
     #pragma unroll
@@ -271,25 +367,15 @@ __device__ __forceinline__ void volume_integral(const DevParams &P, const R *u, 
         for (int v = 0; v < NV; v++) SF[d][v] = R(0);
     #pragma unroll
     for (int g = 0; g < 8; g++) {
-        const R px = (g & 1) ? ph : -ph, py = (g & 2) ? ph : -ph, pz = (g & 4) ? ph : -ph;
-        R t[NV];
-        trace<R, NV>(u, px, py, pz, t);
-        Prim<R, NC> p;
-        cons_to_prim<R, NC, PH>(P, t, p, tv ? tv + g * ts : nullptr, kMemoRows * ts);
-        const R m[3] = {t[0], t[1], t[2]};
-        const R vel[3] = {p.u, p.v, p.w};
+        R F[3][NV];
+        const R r = volume_terms<R, NC, PH, DEV>(P, u, g, rf, tv ? tv + g * ts : nullptr, ts, F);
         #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            SF[d][0] += m[d] * p.u + (d == 0 ? p.p : R(0));
-            SF[d][1] += m[d] * p.v + (d == 1 ? p.p : R(0));
-            SF[d][2] += m[d] * p.w + (d == 2 ? p.p : R(0));
-            SF[d][3] += m[d] * p.e_tot + p.p * vel[d];
+        for (int d = 0; d < 3; d++)
             #pragma unroll
-            for (int i = 0; i < NC; i++) SF[d][4 + i] += m[d] * p.c[i];
-        }
-        G[0] += p.r; G[1] += p.r * px; G[2] += p.r * py; G[3] += p.r * pz;
+            for (int v = 0; v < NV; v++) SF[d][v] += F[d][v];
+        G[0] += r; G[1] += r * ((g & 1) ? ph : -ph); G[2] += r * ((g & 2) ? ph : -ph);
+        G[3] += r * ((g & 4) ? ph : -ph);
     }
-    const R f = wj * hinv;
     #pragma unroll
     for (int v = 0; v < NV; v++) {
         res[4*v+0] = R(0);
@@ -305,51 +391,25 @@ __device__ __forceinline__ void volume_integral(const DevParams &P, const R *u, 
     }
 }
 
-// the volume integral of F - F(U_r) from deviation coefficients u (one
-// species): the momentum, energy and mass fluxes along each axis d as in
-// dev_phys; the gravity term takes the full density
-__device__ __forceinline__ void volume_integral_dev(const DevParams &P, const DevRef &rf, const float *u, float h,
-                                                    float *res)
+// the moments (M0, M1, M2) of one variable of a face record added to its
+// leaf's integrals res[4] of that variable, from the given side
+template <typename R>
+__device__ __forceinline__ void slot_add(int info, int side, R M0, R M1, R M2, R *res)
 {
-    const float ph = 0.28867513459481288225f;          // 1/(2 sqrt 3)
-    const float hinv = rcp(h);
-    const float wj = h * h * h * 0.125f;
-    float SF[3][5];
-    float G[4] = {0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-    for (int d = 0; d < 3; d++)
-        #pragma unroll
-        for (int v = 0; v < 5; v++) SF[d][v] = 0.f;
-    #pragma unroll
-    for (int g = 0; g < 8; g++) {
-        const float px = (g & 1) ? ph : -ph, py = (g & 2) ? ph : -ph, pz = (g & 4) ? ph : -ph;
-        float t[5];
-        trace<float, 5>(u, px, py, pz, t);
-        DPrim q;
-        dev_prim(rf, t, q);
-        #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            #pragma unroll
-            for (int j = 0; j < 3; j++) SF[d][j] += q.dm[d] * q.u[j] + rf.m[d] * q.du[j] + (d == j ? q.dp : 0.f);
-            SF[d][3] += (q.dE + q.dp) * q.u[d] + rf.Epp * q.du[d];
-            SF[d][4] += q.dm[d];
-        }
-        G[0] += q.r; G[1] += q.r * px; G[2] += q.r * py; G[3] += q.r * pz;
-    }
-    const float f = wj * hinv;
-    #pragma unroll
-    for (int v = 0; v < 5; v++) {
-        res[4*v+0] = 0.f;
-        res[4*v+1] = -SF[0][v] * f;
-        res[4*v+2] = -SF[1][v] * f;
-        res[4*v+3] = -SF[2][v] * f;
-    }
-    #pragma unroll
-    for (int v = 0; v < 3; v++) {
-        const float gv = P.grav_f[v];
-        #pragma unroll
-        for (int k = 0; k < 4; k++) res[4*v+k] -= gv * G[k] * wj;
-    }
+    const int dir0 = info & 7, kind = (info >> 3) & 3, sub = (info >> 5) & 3;
+    const R sg = side ? R(-1) : R(1);
+    const R pa = ((dir0 & 1) ^ side) ? R(0.5) : R(-0.5);
+    const bool big = (kind == FACE_HANG0 && side == 1) || (kind == FACE_HANG1 && side == 0);
+    const R mu = big ? R(0.5) : R(1);
+    const R d1 = big ? ((sub & 1) ? R(0.25) : R(-0.25)) : R(0);
+    const R d2 = big ? ((sub & 2) ? R(0.25) : R(-0.25)) : R(0);
+    const R m0 = sg * M0, m1 = sg * M1, m2 = sg * M2;
+    R cx, cy, cz;
+    to_xyz<R>(dir0 >> 1, pa * m0, mu * m1 + d1 * m0, mu * m2 + d2 * m0, cx, cy, cz);
+    res[0] += m0;
+    res[1] += cx;
+    res[2] += cy;
+    res[3] += cz;
 }
 
 // S: storage type of the state; R: arithmetic type of the residual (S = R,
@@ -368,12 +428,13 @@ __device__ __forceinline__ const DevParams &stage_params(const StageArgs &A, con
 
 // The FP32 deviation-form instances are held to at most 168 VGPRs (three
 // waves per SIMD) so that a change of the code cannot drop them below the
-// occupancy their LDS allows; with the rolled point loop they need 117, and
-// four 40 KB workgroups share a CU
+// occupancy their LDS allows; with the rolled point loop they need 114, and
+// four 40 KB workgroups share a CU.  The FP64 ones are held to two waves (the
+// exact Riemann solver with two species took 264 registers and ran at one).
 template <typename R, int NC, int FLUX, int PH>
 constexpr int stage_min_waves()
 {
-    return uses_dev<R, NC, FLUX, PH>() ? 3 : 1;
+    return uses_dev<R, NC, FLUX, PH>() ? 3 : (sizeof(R) == 8 && PH == 0 ? 2 : 1);
 }
 
 template <typename S, typename R, int NC, int FLUX, int BS, int PH>
@@ -403,37 +464,10 @@ void k_stage(StageArgs A, DevParams Pv)
     for (int f = fb + (int) threadIdx.x; f < fe; f += BS) {
         const int4 rec = A.cf4[f];
         R *dst = mom + (size_t) (f - fb) * 3 * NV;
-        R ua[4 * NV];
-        if constexpr (DEV) load_dev<S>(U, n, rec.x, rf, ua);
-        else load_conv<S, R, NV>(U, n, rec.x, ua);
         const int lev0 = A.level[rec.x];
-        // faces of a chunk are sorted by (axis, kind): waves are mostly
-        // uniform in the branch taken here
-        const int ax = (rec.z & 7) >> 1;
-        // PH = 1: each side's point EOS closures from the point pass, at
-        // the side's own (sub)face slot 4 d + j (point k at k * n)
-        const R *pl = nullptr, *pr = nullptr;
-        if (PH == 1 && A.tpt) {
-            const R *TP = reinterpret_cast<const R *>(A.tpt);
-            const int dir0 = rec.z & 7, kind = (rec.z >> 3) & 3, sub = (rec.z >> 5) & 3;
-            const int s0 = 4 * dir0 + (kind == FACE_HANG1 ? sub : 0);
-            const int s1 = 4 * (dir0 ^ 1) + (kind == FACE_HANG0 ? sub : 0);
-            pl = TP + (int64_t) 6 * s0 * n + rec.x;
-            if (kind != FACE_BND) pr = TP + (int64_t) 6 * s1 * n + rec.y;
-        }
-        if (((rec.z >> 3) & 3) == FACE_BND) {
-            ok &= face_moments_bnd<R, NC, FLUX, PH, DEV>(P, ua, rec.z, lev0, dst, rf, pl, n);
-        } else {
-            R ub[4 * NV];
-            if constexpr (DEV) load_dev<S>(U, n, rec.y, rf, ub);
-            else load_conv<S, R, NV>(U, n, rec.y, ub);
-            if (ax == 0)
-                ok &= face_moments<R, NC, FLUX, 0, PH, DEV>(P, ua, ub, rec.z, lev0, dst, rf, pl, pr, n);
-            else if (ax == 1)
-                ok &= face_moments<R, NC, FLUX, 1, PH, DEV>(P, ua, ub, rec.z, lev0, dst, rf, pl, pr, n);
-            else
-                ok &= face_moments<R, NC, FLUX, 2, PH, DEV>(P, ua, ub, rec.z, lev0, dst, rf, pl, pr, n);
-        }
+        const R *pl, *pr;
+        face_closures<R, PH>(A, rec, pl, pr);
+        ok &= face_record<S, R, NC, FLUX, PH, DEV>(P, U, n, rec, lev0, rf, dst, pl, pr);
         finfo[f - fb] = rec.z;
     }
     __syncthreads();
@@ -442,15 +476,17 @@ void k_stage(StageArgs A, DevParams Pv)
         R u[4 * NV], res[4 * NV];
         const int lev = A.level[e];
         const R h = ldexp(R(1), -lev);
-        if constexpr (DEV) {
-            load_dev<S>(U, n, e, rf, u);
-            volume_integral_dev(P, rf, u, h, res);
-        } else {
-            load_conv<S, R, NV>(U, n, e, u);
-            volume_integral<R, NC, PH>(P, u, h, res,
-                                       (PH == 1 && A.tpt) ? reinterpret_cast<const R *>(A.tpt) + (int64_t) kMemoVolRow * n + e
-                                                          : nullptr, n);
-        }
+        // a leaf has at least six slots: their loads are in flight during the
+        // volume integral (one dependent load per slot before)
+        const int s_beg = A.slot_ptr[e], s_end = A.slot_ptr[e + 1];
+        int sl6[6];
+        #pragma unroll
+        for (int k = 0; k < 6; k++) sl6[k] = A.slots[s_beg + k];
+        if constexpr (DEV) load_dev<S>(U, n, e, rf, u);
+        else load_conv<S, R, NV>(U, n, e, u);
+        volume_integral<R, NC, PH, DEV>(P, u, h, rf, res,
+                                        (PH == 1 && A.tpt) ? reinterpret_cast<const R *>(A.tpt) + (int64_t) kMemoVolRow * n + e
+                                                           : nullptr, n);
         if constexpr (PH == 1) {
             if (A.visc) {
                 const S *__restrict__ VI = reinterpret_cast<const S *>(A.visc);
@@ -458,31 +494,15 @@ void k_stage(StageArgs A, DevParams Pv)
                 for (int i = 0; i < 16; i++) res[i] += (R) (VI + i * A.n_elem)[e];
             }
         }
-        const int s_end = A.slot_ptr[e + 1];
-        for (int si = A.slot_ptr[e]; si < s_end; si++) {
-            const int sl = A.slots[si];
+        auto gather = [&](int sl) {
             const int fl = sl >> 1, side = sl & 1;
-            const int info = finfo[fl];
-            const int dir0 = info & 7, kind = (info >> 3) & 3, sub = (info >> 5) & 3;
-            const int a = dir0 >> 1;
-            const R sg = side ? R(-1) : R(1);
-            const R pa = ((dir0 & 1) ^ side) ? R(0.5) : R(-0.5);
-            const bool big = (kind == FACE_HANG0 && side == 1) || (kind == FACE_HANG1 && side == 0);
-            const R mu = big ? R(0.5) : R(1);
-            const R d1 = big ? ((sub & 1) ? R(0.25) : R(-0.25)) : R(0);
-            const R d2 = big ? ((sub & 2) ? R(0.25) : R(-0.25)) : R(0);
             const R *m = mom + (size_t) fl * 3 * NV;
             #pragma unroll
-            for (int v = 0; v < NV; v++) {
-                const R M0 = sg * m[v], M1 = sg * m[NV + v], M2 = sg * m[2 * NV + v];
-                R cx, cy, cz;
-                to_xyz<R>(a, pa * M0, mu * M1 + d1 * M0, mu * M2 + d2 * M0, cx, cy, cz);
-                res[4*v+0] += M0;
-                res[4*v+1] += cx;
-                res[4*v+2] += cy;
-                res[4*v+3] += cz;
-            }
-        }
+            for (int v = 0; v < NV; v++) slot_add<R>(finfo[fl], side, m[v], m[NV + v], m[2 * NV + v], &res[4*v]);
+        };
+        #pragma unroll
+        for (int k = 0; k < 6; k++) gather(sl6[k]);
+        for (int si = s_beg + 6; si < s_end; si++) gather(A.slots[si]);
         S *out = reinterpret_cast<S *>(A.out);
         if (A.mode == 0) {
             #pragma unroll
