@@ -1053,6 +1053,72 @@ done:
     return rc;
 }
 
+void charm_pieces_free(charm_pieces_t *p)
+{
+    free(p->ch_ebeg); free(p->ch_fbeg); free(p->ch_ref); free(p->cf4); free(p->slots);
+    memset(p, 0, sizeof(*p));
+}
+
+/* A piece's faces keep their chunk's order (by axis and kind) and a leaf its
+ * slot order, so the sums of a leaf run as in the chunk. */
+int charm_mesh_cut(const charm_mesh_t *m, int max_e, int max_f, charm_pieces_t *out)
+{
+    int64_t c, e, k, cap = 0;
+    int32_t *mark = (int32_t *) malloc((size_t) (m->chunk_faces + 1) * sizeof(int32_t));
+    int32_t *rank = (int32_t *) malloc((size_t) (m->chunk_faces + 1) * sizeof(int32_t));
+    memset(out, 0, sizeof(*out));
+    /* every slot names a face of its piece, so the slots bound the face copies */
+    out->ch_ebeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->ch_fbeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->ch_ref = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->cf4 = (int32_t *) malloc((size_t) (m->nslot + 1) * 4 * sizeof(int32_t));
+    out->slots = (uint16_t *) malloc((size_t) (m->nslot + 1) * sizeof(uint16_t));
+    if (!mark || !rank || !out->ch_ebeg || !out->ch_fbeg || !out->ch_ref || !out->cf4 || !out->slots) {
+        free(mark); free(rank);
+        charm_pieces_free(out);
+        charm_set_error("mesh_cut: out of memory");
+        return CHARM_ERR_MEM;
+    }
+    for (c = 0; c < m->nch; c++) {
+        const int64_t eb = m->ch_ebeg[c], ee = m->ch_ebeg[c + 1], fb = m->ch_fbeg[c], nf = m->ch_fbeg[c + 1] - fb;
+        int64_t pb = eb, f;
+        for (f = 0; f < nf; f++) mark[f] = -1;          /* the last piece (by its first leaf) that took the face */
+        for (e = eb, cap = 0; e <= ee; e++) {
+            int64_t nnew = 0;
+            if (e < ee)
+                /* (a leaf that is its own periodic neighbour holds both sides
+                 * of the face in adjacent slots) */
+                for (k = m->slot_ptr[e]; k < m->slot_ptr[e + 1]; k++)
+                    nnew += mark[m->slots[k] >> 1] != pb &&
+                            !(k > m->slot_ptr[e] && m->slots[k - 1] >> 1 == m->slots[k] >> 1);
+            if (e == ee || (e > pb && (e - pb >= max_e || cap + nnew > max_f))) {
+                const int64_t p = out->nch++;
+                int64_t q;
+                out->ch_ebeg[p] = (int32_t) pb;
+                out->ch_fbeg[p] = (int32_t) out->ncf;
+                out->ch_ref[p] = (int32_t) eb;
+                for (f = 0; f < nf; f++)
+                    if (mark[f] == pb) {
+                        rank[f] = (int32_t) (out->ncf - out->ch_fbeg[p]);
+                        memcpy(&out->cf4[4 * out->ncf], &m->cf4[4 * (fb + f)], 4 * sizeof(int32_t));
+                        out->ncf++;
+                    }
+                for (q = m->slot_ptr[pb]; q < m->slot_ptr[e]; q++)
+                    out->slots[q] = (uint16_t) ((rank[m->slots[q] >> 1] << 1) | (m->slots[q] & 1));
+                pb = e;
+                cap = 0;
+            }
+            if (e < ee)
+                for (k = m->slot_ptr[e]; k < m->slot_ptr[e + 1]; k++)
+                    if (mark[m->slots[k] >> 1] != pb) { mark[m->slots[k] >> 1] = (int32_t) pb; cap++; }
+        }
+    }
+    out->ch_ebeg[out->nch] = (int32_t) m->n;
+    out->ch_fbeg[out->nch] = (int32_t) out->ncf;
+    free(mark); free(rank);
+    return CHARM_OK;
+}
+
 int charm_forest_flatten(const charm_forest_t *f, int chunk_elems, int chunk_faces,
                          charm_mesh_t **out)
 {

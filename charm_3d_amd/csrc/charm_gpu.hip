@@ -34,7 +34,9 @@ struct charm_gpu_ctx {
     int n_xcd;
     uint8_t *d_level;
     int4 *d_cf4, *d_aux;
-    int *d_ch_ebeg, *d_ch_fbeg, *d_slot_ptr, *d_nbr;
+    int *d_ch_ebeg, *d_ch_fbeg, *d_ch_ref, *d_slot_ptr, *d_nbr;
+    int points;               // small mesh: stages with one thread per quadrature point
+    int block;                // threads of a chunk's workgroup
     uint16_t *d_slots;
     int4 *d_q;                // leaves (x, y, z, level): adaptation
     int32_t *hq;              // host copy of the leaves of the uploaded mesh
@@ -87,7 +89,7 @@ extern "C" int charm_gpu_device_count(int *n)
 static void free_mesh(charm_gpu_ctx_t *c)
 {
     void **p[] = {(void **) &c->d_level, (void **) &c->d_cf4, (void **) &c->d_aux,
-                  (void **) &c->d_ch_ebeg, (void **) &c->d_ch_fbeg, (void **) &c->d_slot_ptr,
+                  (void **) &c->d_ch_ebeg, (void **) &c->d_ch_fbeg, (void **) &c->d_ch_ref, (void **) &c->d_slot_ptr,
                   (void **) &c->d_nbr, (void **) &c->d_slots, &c->B[0], &c->B[1], &c->B[2],
                   (void **) &c->d_stage64, (void **) &c->d_partial, (void **) &c->d_q,
                   &c->d_auxf, &c->d_vi, &c->d_auxo, &c->d_lift, (void **) &c->d_dcoef, (void **) &c->d_chem,
@@ -276,6 +278,45 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
         }                                                                           \
     } while (0)
 
+// The chunks a context runs a mesh on.  With the flattening's chunks, sized
+// for meshes of many, a small mesh would occupy a few of the 256 CUs and a
+// stage would last as long as one workgroup's serial passes, so its chunks
+// are cut into pieces; every piece keeps its chunk's reference leaf, so the
+// cut changes no bit of the FP32 deviation form.  Stage times (us), uncut and
+// as chosen:
+//   up to 6,000 leaves, pieces of 8 on k_stage_pt: 512 leaves FP64 22 -> 8,
+//     4,096 leaves FP32 21 -> 11, four species 64 -> 47;
+//   up to 12,000 (exact Riemann solver: 24,000), pieces of 16 on k_stage_pt:
+//     9,192 leaves FP64 37 -> 27, exact solver 54 -> 22;
+//   else, one to three species of constant cp: FP32 up to 65,536 pieces of 64
+//     on 256 threads (40,328 leaves 32 -> 25, exact solver 59 -> 44; 86,864
+//     37 -> 36), FP64 up to 24,000 pieces of 48 (19,104 leaves 37 -> 30;
+//     at 32,768 the pieces lose, 34 -> 40).
+// A viscous or real-gas mesh beyond the point kernel's sizes stays uncut (104
+// and 105 at 32,768 leaves).
+struct Pieces {
+    charm_pieces_t p;
+    int rc, cut, points;
+    Pieces(const charm_gpu_ctx_t *c, const charm_mesh_t *m) : rc(CHARM_OK), cut(0), points(0)
+    {
+        const bool fp64 = c->prec == CHARM_FP64;
+        int e = 0, f = 0;
+        if (m->n <= 6000) { e = 8; f = 48; points = 1; }
+        else if (m->n <= 12000 || (m->n <= 24000 && c->cfg.flux == CHARM_FLUX_GODUNOV)) { e = 16; f = 80; points = 1; }
+        if (points && stage_points_smem_bytes(c->prec, c->nc, f, e) > 65536) { e = f = points = 0; }
+        if (!points && !c->ph) {
+            if (!fp64 && m->n <= 65536) { e = 64; f = 256; }
+            if (fp64 && m->n <= 24000) { e = 48; f = 192; }
+        }
+        cut = e && (m->chunk_elems > e || m->chunk_faces > f);
+        memset(&p, 0, sizeof(p));
+        if (cut) { rc = charm_mesh_cut(m, e, f, &p); return; }
+        p.nch = m->nch; p.ncf = m->ncf;
+        p.ch_ebeg = m->ch_ebeg; p.ch_fbeg = m->ch_fbeg; p.ch_ref = m->ch_ebeg; p.cf4 = m->cf4; p.slots = m->slots;
+    }
+    ~Pieces() { if (cut) charm_pieces_free(&p); }
+};
+
 extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
 {
     if (!c || !m) { charm_set_error("upload_mesh: null argument"); return CHARM_ERR_ARG; }
@@ -306,10 +347,13 @@ extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
     HIPCHK(hipStreamSynchronize(c->st));
     free_mesh(c);
     const size_t ssz = (size_t) m->n * 4 * c->nv * c->esz;
+    Pieces pc(c, m);
+    if (pc.rc) return pc.rc;
     DMALLOC(c->d_level, (size_t) m->n);
-    DMALLOC(c->d_cf4, (size_t) m->ncf * sizeof(int4));
-    DMALLOC(c->d_ch_ebeg, (size_t) (m->nch + 1) * sizeof(int));
-    DMALLOC(c->d_ch_fbeg, (size_t) (m->nch + 1) * sizeof(int));
+    DMALLOC(c->d_cf4, (size_t) pc.p.ncf * sizeof(int4));
+    DMALLOC(c->d_ch_ebeg, (size_t) (pc.p.nch + 1) * sizeof(int));
+    DMALLOC(c->d_ch_fbeg, (size_t) (pc.p.nch + 1) * sizeof(int));
+    DMALLOC(c->d_ch_ref, (size_t) pc.p.nch * sizeof(int));
     DMALLOC(c->d_slot_ptr, (size_t) (m->n + 1) * sizeof(int));
     DMALLOC(c->d_slots, (size_t) m->nslot * sizeof(uint16_t));
     DMALLOC(c->d_nbr, (size_t) m->n * 6 * sizeof(int));
@@ -338,11 +382,12 @@ extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
     memcpy(c->hq, m->q, (size_t) m->n * 4 * sizeof(int32_t));
     HIPCHK(hipMemcpyAsync(c->d_q, m->q, (size_t) m->n * sizeof(int4), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_level, m->level, (size_t) m->n, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_cf4, m->cf4, (size_t) m->ncf * sizeof(int4), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_ch_ebeg, m->ch_ebeg, (size_t) (m->nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_ch_fbeg, m->ch_fbeg, (size_t) (m->nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_cf4, pc.p.cf4, (size_t) pc.p.ncf * sizeof(int4), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_ch_ebeg, pc.p.ch_ebeg, (size_t) (pc.p.nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_ch_fbeg, pc.p.ch_fbeg, (size_t) (pc.p.nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_ch_ref, pc.p.ch_ref, (size_t) pc.p.nch * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_slot_ptr, m->slot_ptr, (size_t) (m->n + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_slots, m->slots, (size_t) m->nslot * sizeof(uint16_t), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_slots, pc.p.slots, (size_t) m->nslot * sizeof(uint16_t), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_nbr, m->nbr, (size_t) m->n * 6 * sizeof(int), hipMemcpyHostToDevice, c->st));
     if (m->naux)
         HIPCHK(hipMemcpyAsync(c->d_aux, m->aux, (size_t) m->naux * sizeof(int4), hipMemcpyHostToDevice, c->st));
@@ -352,9 +397,16 @@ extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
         HIPCHK(hipMemsetAsync(c->d_chem, 0, (size_t) m->n * sizeof(double), c->st));
     }
     HIPCHK(hipStreamSynchronize(c->st));
-    c->n = m->n; c->nch = m->nch; c->ncf = m->ncf; c->nslot = m->nslot; c->naux = m->naux;
-    c->max_faces = m->chunk_faces;
-    c->chunk_elems = m->chunk_elems;
+    c->n = m->n; c->nch = pc.p.nch; c->ncf = pc.p.ncf; c->nslot = m->nslot; c->naux = m->naux;
+    // the largest chunk there is sizes the workgroups and their LDS
+    c->max_faces = c->chunk_elems = 1;
+    for (int64_t i = 0; i < c->nch; i++) {
+        const int ne = pc.p.ch_ebeg[i + 1] - pc.p.ch_ebeg[i], nf = pc.p.ch_fbeg[i + 1] - pc.p.ch_fbeg[i];
+        if (ne > c->chunk_elems) c->chunk_elems = ne;
+        if (nf > c->max_faces) c->max_faces = nf;
+    }
+    c->points = pc.points && stage_points_smem_bytes(c->prec, c->nc, c->max_faces, c->chunk_elems) <= 65536;
+    c->block = c->chunk_elems > 128 || (pc.cut && c->max_faces > 128) ? 256 : 128;
     return CHARM_OK;
 }
 
@@ -473,8 +525,9 @@ static StageArgs stage_args(charm_gpu_ctx_t *c, const void *U, const void *U0, v
     StageArgs A;
     A.U = U; A.U0 = U0; A.out = out;
     A.level = c->d_level; A.cf4 = c->d_cf4; A.ch_ebeg = c->d_ch_ebeg; A.ch_fbeg = c->d_ch_fbeg;
+    A.ch_ref = c->d_ch_ref; A.points = c->points;
     A.slot_ptr = c->d_slot_ptr; A.slots = c->d_slots; A.err = c->d_err;
-    A.n_elem = c->n; A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems;
+    A.n_elem = c->n; A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems; A.block = c->block;
     A.n_xcd = c->n_xcd;
     A.mode = mode; A.combine = combine; A.dt = dt;
     A.visc = (c->ph && c->cfg.use_visc) ? c->d_vi : NULL;

@@ -52,6 +52,17 @@ struct charm_mesh {
     uint16_t *slots;        /* local face index << 1 | side */
 };
 
+/* The chunks of a mesh cut into pieces of at most max_e leaves and max_f
+ * faces (more only where one leaf has more): the chunk arrays of a mesh, and
+ * per piece the first leaf of the chunk it was cut from. */
+typedef struct {
+    int64_t   nch, ncf;
+    int32_t  *ch_ebeg, *ch_fbeg, *ch_ref, *cf4;
+    uint16_t *slots;
+} charm_pieces_t;
+int  charm_mesh_cut(const charm_mesh_t *m, int max_e, int max_f, charm_pieces_t *out);
+void charm_pieces_free(charm_pieces_t *p);
+
 /* the forest's user pointer (the reference's charm_ctx_t) */
 struct charm_ctx {
     charm_config_t   cfg;

@@ -13,11 +13,13 @@ struct StageArgs {
     void *out;                // residual (mode 0) or updated state (mode 1)
     const uint8_t *level;
     const int4 *cf4;          // chunk face records (e0, e1, info, 0)
-    const int *ch_ebeg, *ch_fbeg, *slot_ptr;
+    const int *ch_ebeg, *ch_fbeg, *ch_ref, *slot_ptr;
     const uint16_t *slots;
     int *err;
     int64_t n_elem;
     int n_chunks, max_faces, chunk_elems;
+    int points;               // one thread per quadrature point (k_stage_pt)
+    int block;                // threads of a chunk's workgroup (128 or 256)
     int n_xcd;                // XCDs the workgroups are spread over
     int mode;                 // 0: write int_*; 1: c - dt A^-1 int
     int combine;              // 0: none, 1: w/4 + 3 u0/4, 2: 2w/3 + u0/3
@@ -196,6 +198,8 @@ const void *stage_fn_mix_ph0(int nc, int flux, int bs);
 // prec: 0 FP64, 1 FP32, 2 mixed (FP64 state, FP32 residual)
 hipError_t launch_stage(int prec, int nc, int flux, int ph, const StageArgs &A, const DevParams &P, hipStream_t st);
 size_t stage_smem_bytes(int prec, int nc, int max_faces);
+// LDS bytes of a point-kernel workgroup for chunks of at most `faces` faces and `elems` leaves
+size_t stage_points_smem_bytes(int prec, int nc, int faces, int elems);
 // host address of the stage kernel a launch with these parameters uses
 // (bs = the workgroup size: 128 or 256)
 const void *stage_kernel(int prec, int nc, int flux, int ph, int bs);

@@ -284,6 +284,12 @@ size_t stage_smem_bytes(int prec, int nc, int max_faces)
     return (size_t) max_faces * (3 * (4 + nc) * (prec ? 4 : 8) + sizeof(int));
 }
 
+size_t stage_points_smem_bytes(int prec, int nc, int faces, int elems)
+{
+    const size_t nv = 4 + nc;
+    return (9 * nv * faces + 8 * (3 * nv + 1) * elems) * (prec ? 4 : 8) + 2 * (size_t) faces * sizeof(int);
+}
+
 template <typename R, int PH>
 static hipError_t launch_limiter_r(int nc, const LimArgs &A, const DevParams &P, hipStream_t st)
 {
