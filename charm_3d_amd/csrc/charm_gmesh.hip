@@ -5,15 +5,15 @@
 //
 // Face pass, one thread per face: at its 6 points both traces (side 1 from
 // the boundary condition on a boundary face), the flux along the side-0
-// normal in the reference's face frame, and the moment sums of both sides,
-// each written to its leaf's slot for that local face, FQ[6][4V][n] (side 1
-// negated; on a conforming forest every local face of a leaf has exactly one
-// face).  Element pass, one thread per leaf: the volume integral at 8 points
-// (flux tensor against grad phi = e / dh, gravity on the momentum), its six
-// face slots (coalesced, no atomics), the full 4x4 A^-1, the update and the
-// SSP-RK combine; ahead of the limiter also the cell means of the new state.  The arithmetic is the
-// reference's Euler model (src/models/euler/charm_model.c:66-212, 215-372,
-// 402-433) with the geometry of src/charm_geom.c.
+// normal, and side 0's moment sums, FS[4V][nf].  Side 1's basis is the affine
+// image b1 = b0 r + o of side 0's, so its sums are the same image of side 0's
+// and are not stored.  Element pass, one thread per leaf: the volume integral
+// at 8 points (flux tensor against grad phi = e / dh, gravity on the
+// momentum), its six faces' sums (LF[6][n]: face << 1 | side; no atomics), the
+// full 4x4 A^-1, the update and the SSP-RK combine; ahead of the limiter also
+// the cell means of the new state.  The arithmetic is the reference's Euler
+// model (src/models/euler/charm_model.c:66-212, 215-372, 402-433) with the
+// geometry of src/charm_geom.c.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "charm_device.hpp"
@@ -111,6 +111,52 @@ static inline int64_t xcd_grid(int64_t blocks, int n_xcd)
 
 } // namespace
 
+// Flux along the unit normal n in global components.  LF, HLLC and CD are
+// linear in the tangential velocities: with tangential velocities (1, 0) and
+// (0, 1) on the two sides the tangential fluxes are the factors a, b of
+// q = q_n n + a (u_L - u_Ln n) + b (u_R - u_Rn n), and no face frame is needed.
+// The exact Riemann solver's energy takes the tangential velocities themselves:
+// it runs in the reference's frame.
+template <typename R, int NC, int FLUX>
+__device__ __forceinline__ bool flux_normal(const Prim<R, NC> &pa, const Prim<R, NC> &pb, const double nn[3],
+                                            const R n3[3], R *g)
+{
+    constexpr int NV = 4 + NC;
+    R q[NV];
+    bool ok;
+    if constexpr (FLUX == FLUX_GODUNOV) {
+        double nt[3][3];
+        ref_face_frame(nn, nt);
+        const Frame<R, NC> fa = to_frame<R, NC>(pa, R(nt[0][0]), R(nt[0][1]), R(nt[0][2]), R(nt[1][0]), R(nt[1][1]),
+                                                R(nt[1][2]), R(nt[2][0]), R(nt[2][1]), R(nt[2][2]));
+        const Frame<R, NC> fb = to_frame<R, NC>(pb, R(nt[0][0]), R(nt[0][1]), R(nt[0][2]), R(nt[1][0]), R(nt[1][1]),
+                                                R(nt[1][2]), R(nt[2][0]), R(nt[2][1]), R(nt[2][2]));
+        ok = flux_x<R, NC, FLUX>(fa, fb, q);
+        #pragma unroll
+        for (int d = 0; d < 3; d++) g[d] = q[0] * R(nt[0][d]) + q[1] * R(nt[1][d]) + q[2] * R(nt[2][d]);
+    } else {
+        Frame<R, NC> fa = frame_state(pa), fb = frame_state(pb);
+        fa.un = pa.u * n3[0] + pa.v * n3[1] + pa.w * n3[2];
+        fb.un = pb.u * n3[0] + pb.v * n3[1] + pb.w * n3[2];
+        fa.ut1 = R(1); fa.ut2 = R(0);
+        fb.ut1 = R(0); fb.ut2 = R(1);
+        ok = flux_x<R, NC, FLUX>(fa, fb, q);
+        const R qn = q[0] - q[1] * fa.un - q[2] * fb.un;
+        g[0] = qn * n3[0] + q[1] * pa.u + q[2] * pb.u;
+        g[1] = qn * n3[1] + q[1] * pa.v + q[2] * pb.v;
+        g[2] = qn * n3[2] + q[1] * pa.w + q[2] * pb.w;
+    }
+    #pragma unroll
+    for (int v = 3; v < NV; v++) g[v] = q[v];
+    return ok;
+}
+
+// Bound by HBM traffic.  Storing one side's sums (80 of the FP32 bytes per face
+// saved), no face frame and four waves per SIMD took the FP32 HLLC pass over
+// 6.3M faces from 615 to 391 us and over 0.79M from 82 to 47; FP64 6.3M faces
+// 1,668 to 763.  The element pass, which now gathers half its sums through the
+// face index, went from 390 to 379 us (FP32, 2.1M leaves) and 782 to 717 (FP64):
+// stage 5.8 TB/s of designed bytes in FP32 against 5.1 of a large copy.
 template <typename R, int NC, int FLUX>
 __global__ __launch_bounds__(256)
 void k_gface(GArgs A, DevParams P)
@@ -127,60 +173,49 @@ void k_gface(GArgs A, DevParams P)
     for (int i = 0; i < 4 * NV; i++) u0[i] = (U + i * n)[e0];
     #pragma unroll
     for (int i = 0; i < 4 * NV; i++) u1[i] = e1 >= 0 ? (U + i * n)[e1] : R(0);
-    double nn[3] = {A.fn[f], A.fn[nf + f], A.fn[2 * nf + f]}, nt[3][3];
-    ref_face_frame(nn, nt);
+    const double nn[3] = {A.fn[f], A.fn[nf + f], A.fn[2 * nf + f]};
     const R n3[3] = {R(nn[0]), R(nn[1]), R(nn[2])};
-    R s0[NV][4], s1[NV][4];
+    R s0[NV][4];
     #pragma unroll
     for (int v = 0; v < NV; v++)
         #pragma unroll
-        for (int k = 0; k < 4; k++) { s0[v][k] = R(0); s1[v][k] = R(0); }
+        for (int k = 0; k < 4; k++) s0[v][k] = R(0);
     bool ok = true;
     // side 1's basis is the affine image of side 0's: b1 = b0 r + o per axis
     const R r1[3] = {FG[18 * nf], FG[19 * nf], FG[20 * nf]}, o1[3] = {FG[21 * nf], FG[22 * nf], FG[23 * nf]};
+    // rolled (114 registers, four waves per SIMD; unrolled 171 and two), each
+    // point's basis and weight loaded one point ahead
+    R bn[4] = {FG[0], FG[nf], FG[2 * nf], FG[24 * nf]};
+    #pragma unroll 1
     for (int p = 0; p < 6; p++) {
-        const R b0[3] = {FG[(3 * p) * nf], FG[(3 * p + 1) * nf], FG[(3 * p + 2) * nf]};
-        const R b1[3] = {b0[0] * r1[0] + o1[0], b0[1] * r1[1] + o1[1], b0[2] * r1[2] + o1[2]};
-        const R wj = FG[(24 + p) * nf];
+        const R b0[3] = {bn[0], bn[1], bn[2]}, wj = bn[3];
+        const int pn = p < 5 ? p + 1 : 5;
+        bn[0] = FG[(3 * pn) * nf]; bn[1] = FG[(3 * pn + 1) * nf]; bn[2] = FG[(3 * pn + 2) * nf];
+        bn[3] = FG[(24 + pn) * nf];
         R t[NV];
         Prim<R, NC> pa, pb;
         trace_at<R, NV>(u0, b0, t);
         cons_to_prim<R, NC, 0>(P, t, pa);
         if (e1 >= 0) {
+            const R b1[3] = {b0[0] * r1[0] + o1[0], b0[1] * r1[1] + o1[1], b0[2] * r1[2] + o1[2]};
             trace_at<R, NV>(u1, b1, t);
             cons_to_prim<R, NC, 0>(P, t, pb);
         } else {
             bnd_state_n<R, NC>(P, -1 - e1, n3, pa, pb);
         }
-        const Frame<R, NC> fa = to_frame<R, NC>(pa, R(nt[0][0]), R(nt[0][1]), R(nt[0][2]), R(nt[1][0]), R(nt[1][1]),
-                                                R(nt[1][2]), R(nt[2][0]), R(nt[2][1]), R(nt[2][2]));
-        const Frame<R, NC> fb = to_frame<R, NC>(pb, R(nt[0][0]), R(nt[0][1]), R(nt[0][2]), R(nt[1][0]), R(nt[1][1]),
-                                                R(nt[1][2]), R(nt[2][0]), R(nt[2][1]), R(nt[2][2]));
-        R q[NV], g[NV];
-        ok &= flux_x<R, NC, FLUX>(fa, fb, q);
-        #pragma unroll
-        for (int d = 0; d < 3; d++) g[d] = q[0] * R(nt[0][d]) + q[1] * R(nt[1][d]) + q[2] * R(nt[2][d]);
-        #pragma unroll
-        for (int v = 3; v < NV; v++) g[v] = q[v];
+        R g[NV];
+        ok &= flux_normal<R, NC, FLUX>(pa, pb, nn, n3, g);
         const R ph0[4] = {wj, b0[0] * wj, b0[1] * wj, b0[2] * wj};
-        const R ph1[4] = {wj, b1[0] * wj, b1[1] * wj, b1[2] * wj};
         #pragma unroll
         for (int v = 0; v < NV; v++)
             #pragma unroll
-            for (int k = 0; k < 4; k++) { s0[v][k] += g[v] * ph0[k]; s1[v][k] += g[v] * ph1[k]; }
+            for (int k = 0; k < 4; k++) s0[v][k] += g[v] * ph0[k];
     }
-    R *__restrict__ FQ = reinterpret_cast<R *>(A.fq);
-    const int l0 = A.ff[f], l1 = A.ff[nf + f];
+    R *__restrict__ FS = reinterpret_cast<R *>(A.fs) + f;
     #pragma unroll
     for (int v = 0; v < NV; v++)
         #pragma unroll
-        for (int k = 0; k < 4; k++) (FQ + (int64_t) (4 * NV * l0 + 4 * v + k) * n)[e0] = s0[v][k];
-    if (e1 >= 0) {
-        #pragma unroll
-        for (int v = 0; v < NV; v++)
-            #pragma unroll
-            for (int k = 0; k < 4; k++) (FQ + (int64_t) (4 * NV * l1 + 4 * v + k) * n)[e1] = -s1[v][k];
-    }
+        for (int k = 0; k < 4; k++) FS[(int64_t) (4 * v + k) * nf] = s0[v][k];
     if (!ok) A.err[0] = 1;
 }
 
@@ -189,14 +224,18 @@ __global__ __launch_bounds__(256)
 void k_gelem(GArgs A, DevParams P)
 {
     constexpr int NV = 4 + NC;
-    const int64_t n = A.n;
-    const int64_t e = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t n = A.n, nf = A.nf;
+    const int64_t e = (int64_t) xcd_block(A.n_xcd) * blockDim.x + threadIdx.x;
     if (e >= n) return;
     const R *__restrict__ U = reinterpret_cast<const R *>(A.U);
     const R *__restrict__ LG = reinterpret_cast<const R *>(A.lg) + e;
     R u[4 * NV];
     #pragma unroll
     for (int i = 0; i < 4 * NV; i++) u[i] = (U + i * n)[e];
+    // the leaf's faces: their loads are in flight during the volume integral
+    int lf[6];
+    #pragma unroll
+    for (int d = 0; d < 6; d++) lf[d] = A.lf[d * n + e];
     R in[NV][4];
     #pragma unroll
     for (int v = 0; v < NV; v++)
@@ -229,13 +268,34 @@ void k_gelem(GArgs A, DevParams P)
             #pragma unroll
             for (int k = 0; k < 4; k++) in[d][k] -= p.r * grav[d] * phi[k];
     }
-    const R *__restrict__ FQ = reinterpret_cast<const R *>(A.fq);
-    #pragma unroll 1
-    for (int lf = 0; lf < 6; lf++)
+    const R *__restrict__ FS = reinterpret_cast<const R *>(A.fs);
+    const R *__restrict__ FG = reinterpret_cast<const R *>(A.fg);
+    #pragma unroll
+    for (int d = 0; d < 6; d++) {
+        const int64_t f = lf[d] >> 1;
+        R s[NV][4];
         #pragma unroll
         for (int v = 0; v < NV; v++)
             #pragma unroll
-            for (int k = 0; k < 4; k++) in[v][k] += (FQ + (int64_t) (4 * NV * lf + 4 * v + k) * n)[e];
+            for (int k = 0; k < 4; k++) s[v][k] = (FS + (int64_t) (4 * v + k) * nf)[f];
+        if (lf[d] & 1) {
+            // side 1: -sum g (1, b1) wj with b1 = b0 r + o
+            R r[3], o[3];
+            #pragma unroll
+            for (int k = 0; k < 3; k++) { r[k] = (FG + (18 + k) * nf)[f]; o[k] = (FG + (21 + k) * nf)[f]; }
+            #pragma unroll
+            for (int v = 0; v < NV; v++) {
+                in[v][0] -= s[v][0];
+                #pragma unroll
+                for (int k = 0; k < 3; k++) in[v][1 + k] -= s[v][1 + k] * r[k] + s[v][0] * o[k];
+            }
+        } else {
+            #pragma unroll
+            for (int v = 0; v < NV; v++)
+                #pragma unroll
+                for (int k = 0; k < 4; k++) in[v][k] += s[v][k];
+        }
+    }
     R *__restrict__ out = reinterpret_cast<R *>(A.out);
     if (A.mode == 0) {
         #pragma unroll
@@ -346,9 +406,10 @@ void k_glimiter(GArgs A, DevParams P)
 template <typename R, int NC>
 static hipError_t launch_gstage_r(int flux, const GArgs &A, const DevParams &P, hipStream_t st)
 {
-    // the face grid is a multiple of the XCD count (xcd_block's bijection);
-    // the padding blocks return
-    const dim3 block(256), gf((unsigned) xcd_grid((A.nf + 255) / 256, A.n_xcd)), ge((unsigned) ((A.n + 255) / 256));
+    // the grids are multiples of the XCD count (xcd_block's bijection); the
+    // padding blocks return
+    const dim3 block(256), gf((unsigned) xcd_grid((A.nf + 255) / 256, A.n_xcd)),
+        ge((unsigned) xcd_grid((A.n + 255) / 256, A.n_xcd));
     switch (flux) {
     case FLUX_LF: hipLaunchKernelGGL((k_gface<R, NC, FLUX_LF>), gf, block, 0, st, A, P); break;
     case FLUX_HLLC: hipLaunchKernelGGL((k_gface<R, NC, FLUX_HLLC>), gf, block, 0, st, A, P); break;

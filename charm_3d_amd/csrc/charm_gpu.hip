@@ -57,9 +57,9 @@ struct charm_gpu_ctx {
     // multi-tree mesh (charm_gpu_upload_gmesh; gm = 1): the general kernels
     int gm;
     int64_t gnf;
-    void *d_glg, *d_gfg, *d_gfq, *d_gmb;
+    void *d_glg, *d_gfg, *d_gfs, *d_gmb;
     double *d_gfn;
-    int *d_gfe, *d_gff, *d_glnb;
+    int *d_gfe, *d_glf, *d_glnb;
     const void *gmb_of;             // the state whose cell means d_gmb holds (multi-tree)
     // state
     void *B[3];
@@ -94,8 +94,8 @@ static void free_mesh(charm_gpu_ctx_t *c)
                   (void **) &c->d_stage64, (void **) &c->d_partial, (void **) &c->d_q,
                   &c->d_auxf, &c->d_vi, &c->d_auxo, &c->d_lift, (void **) &c->d_dcoef, (void **) &c->d_chem,
                   (void **) &c->d_tpt,
-                  &c->d_glg, &c->d_gfg, &c->d_gfq, &c->d_gmb, (void **) &c->d_gfn, (void **) &c->d_gfe,
-                  (void **) &c->d_gff, (void **) &c->d_glnb};
+                  &c->d_glg, &c->d_gfg, &c->d_gfs, &c->d_gmb, (void **) &c->d_gfn, (void **) &c->d_gfe,
+                  (void **) &c->d_glf, (void **) &c->d_glnb};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); i++)
         if (*p[i]) { (void) hipFree(*p[i]); *p[i] = NULL; }
     c->gm = 0; c->gnf = 0; c->gmb_of = NULL; c->temps_of = NULL;
@@ -439,6 +439,11 @@ extern "C" int charm_gpu_upload_gmesh(charm_gpu_ctx_t *c, const charm_gmesh_t *m
                             -1 - g.fe[g.nf + i]);
             return CHARM_ERR_ARG;
         }
+    if (g.nf >= ((int64_t) 1 << 30)) {
+        // a face and its side share 32 bits (the arrays of so many faces exceed the GPU's memory)
+        charm_set_error("upload_gmesh: %lld faces (at most 2^30)", (long long) g.nf);
+        return CHARM_ERR_ARG;
+    }
     HIPCHK(hipStreamSynchronize(c->st));
     free_mesh(c);
     const int64_t n = g.n, nf = g.nf;
@@ -448,18 +453,26 @@ extern "C" int charm_gpu_upload_gmesh(charm_gpu_ctx_t *c, const charm_gmesh_t *m
     DMALLOC(c->d_partial, (size_t) ((n + 255) / 256 + 1) * (c->nv + 1) * sizeof(double));
     DMALLOC(c->d_glg, (size_t) n * CHARM_GM_LEAFQ * c->esz);
     DMALLOC(c->d_gfg, (size_t) nf * CHARM_GM_FACEQ * c->esz);
-    DMALLOC(c->d_gfq, (size_t) n * 6 * 4 * c->nv * c->esz);
+    DMALLOC(c->d_gfs, (size_t) nf * 4 * c->nv * c->esz);
     DMALLOC(c->d_gmb, (size_t) n * c->nv * c->esz);
     DMALLOC(c->d_gfn, (size_t) nf * 3 * sizeof(double));
     DMALLOC(c->d_gfe, (size_t) nf * 2 * sizeof(int));
-    DMALLOC(c->d_gff, (size_t) nf * 2 * sizeof(int));
+    DMALLOC(c->d_glf, (size_t) n * 6 * sizeof(int));
     DMALLOC(c->d_glnb, (size_t) n * 6 * sizeof(int));
+    // each leaf's six faces (face << 1 | side)
+    int *lf = (int *) malloc((size_t) n * 6 * sizeof(int));
+    if (!lf) { charm_set_error("upload_gmesh: out of memory"); free_mesh(c); return CHARM_ERR_MEM; }
+    for (int64_t f = 0; f < nf; f++) {
+        lf[g.ff[f] * n + g.fe[f]] = (int) (f << 1);
+        if (g.fe[nf + f] >= 0) lf[g.ff[nf + f] * n + g.fe[nf + f]] = (int) (f << 1 | 1);
+    }
     hipError_t e = upload_real(c, c->d_glg, g.lg, (size_t) n * CHARM_GM_LEAFQ);
     if (e == hipSuccess) e = upload_real(c, c->d_gfg, g.fg, (size_t) nf * CHARM_GM_FACEQ);
     if (e == hipSuccess) e = hipMemcpy(c->d_gfn, g.fn, (size_t) nf * 3 * sizeof(double), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_gfe, g.fe, (size_t) nf * 2 * sizeof(int), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(c->d_glnb, g.lnb, (size_t) n * 6 * sizeof(int), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(c->d_gff, g.ff, (size_t) nf * 2 * sizeof(int), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(c->d_glf, lf, (size_t) n * 6 * sizeof(int), hipMemcpyHostToDevice);
+    free(lf);
     for (int i = 0; i < 3 && e == hipSuccess; i++) e = hipMemsetAsync(c->B[i], 0, ssz, c->st);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     if (e != hipSuccess) {
@@ -626,9 +639,9 @@ static hipError_t ns_prepare(charm_gpu_ctx_t *c, const void *in, void *chem_out,
 static GArgs gargs(charm_gpu_ctx_t *c, const void *U, const void *U0, void *out, int mode, int combine, double dt)
 {
     GArgs G;
-    G.U = U; G.U0 = U0; G.out = out; G.fq = c->d_gfq; G.mb = NULL;
+    G.U = U; G.U0 = U0; G.out = out; G.fs = c->d_gfs; G.mb = NULL;
     G.lg = c->d_glg; G.fg = c->d_gfg; G.fn = c->d_gfn;
-    G.fe = c->d_gfe; G.ff = c->d_gff; G.lnb = c->d_glnb;
+    G.fe = c->d_gfe; G.lf = c->d_glf; G.lnb = c->d_glnb;
     G.err = c->d_err; G.n = c->n; G.nf = c->gnf;
     G.mode = mode; G.combine = combine; G.dt = dt;
     G.n_xcd = c->n_xcd;

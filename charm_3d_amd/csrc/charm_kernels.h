@@ -86,21 +86,21 @@ struct ProjArgs {
 };
 
 // Multi-tree (general hexahedral) meshes, charm_gmesh.hip: the stage as a
-// face pass (FQ[2][4V][nf]) and an element pass; the limiter.  Geometry
+// face pass (FS[4V][nf]) and an element pass; the limiter.  Geometry
 // arrays in the state precision, layouts of charm_internal.h (CHARM_GM_*).
 struct GArgs {
     const void *U;            // stage: the state the residual is evaluated on; limiter: W
     const void *U0;           // SSP-RK combine base
     void *out;                // mode 0: the residual integrals; else the new state
-    void *fq;                 // [6][4V][n] each leaf's face sums by local face (side 1 negated)
+    void *fs;                 // [4V][nf] side 0's moment sums of each face
     void *mb;                 // [V][n] cell means of the stage output for the limiter (or null)
     const void *lg, *fg;      // [CHARM_GM_LEAFQ][n], [CHARM_GM_FACEQ][nf]
     const double *fn;         // [3][nf] side-0 outward normals (FP64: the reference's face frame)
-    const int *fe, *ff, *lnb;
+    const int *fe, *lf, *lnb; // lf [6][n]: each leaf's faces, face << 1 | side
     int *err;
     int64_t n, nf;
     int mode, combine;
-    int n_xcd;                // XCDs: the face pass and limiter give each a contiguous range
+    int n_xcd;                // XCDs: every pass gives each a contiguous range
     double dt;
 };
 hipError_t launch_gstage(int prec, int nc, int flux, const GArgs &A, const DevParams &P, hipStream_t st);
