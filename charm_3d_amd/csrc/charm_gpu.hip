@@ -842,19 +842,32 @@ extern "C" int charm_gpu_recommended_chunks(const charm_config_t *cfg, int *ce, 
         faces = (int) (budget / per_face);
         if (faces > 1024) faces = 1024;
         // at most three passes of the workgroup over the faces (a fourth,
-        // partial pass runs with most lanes idle)
+        // partial pass runs with most lanes idle); two and a half where the
+        // adjoint below does not limit them
         if (faces > 3 * bs) faces = 3 * bs;
+        if (config_physics(cfg) && faces > 640) faces = 640;
         // the FP32 stage adjoint runs on the same chunks with wider LDS
         // records: keep two of its workgroups per CU (one halves the
         // adjoint's occupancy; the forward stage time does not change
-        // between 640 and 768 faces)
-        if (cfg->precision == CHARM_FP32) {
+        // between 640 and 768 faces).  The adjoint has no Navier-Stokes,
+        // Cp(T) or chemistry terms.
+        if (cfg->precision == CHARM_FP32 && !config_physics(cfg)) {
             const int adj_faces = (int) (lds_cu / 2 / adj_chunk_smem_bytes(1, cfg->n_comp, 1));
             if (faces > adj_faces) faces = adj_faces;
         }
         // 128-thread workgroups serve chunks of at most 128 elements
         if (bs == 128 || faces / 3 > 128 || config_physics(cfg)) break;
     }
+    // Whole passes of 256 faces: a partial last pass costs its full latency.
+    // Stage, us, at the size above against this one: FP64 one species 262,144
+    // leaves LF 104 / 94, HLLC 141 / 129, exact 473 / 428 (528 / 512 faces); FP64 two
+    // species 170,248 leaves HLLC 227 / 151, exact 507 / 329 (442 / 256); FP32
+    // two species exact 102.5 / 97.1 (538 / 512); four species with transport
+    // and Cp(T) FP32 262,144 leaves 462 / 424 (417, the adjoint's limit / 512),
+    // FP64 32,768 leaves 201 / 170 (334 / 256; 262,144 leaves 1,060 / 1,072).
+    // FP32 one species runs best at its two and a half passes (640: 430; 512:
+    // 462; 768: 462 at level 7).
+    if (faces >= 256 && !(cfg->n_comp == 1 && cfg->precision != CHARM_FP64)) faces &= ~255;
     if (faces < 96) faces = 96;
     *cf = faces;
     *ce = faces / 3 > 256 ? 256 : faces / 3;
