@@ -111,7 +111,7 @@ static int64_t find_near(const charm_forest_t *f, uint64_t k, int64_t hint)
 /* ------------------------------------------------------------ host threads */
 
 /* CHARM_HOST_THREADS, else OMP_NUM_THREADS, else the online cores; [1, 64] */
-static int host_threads(void)
+int charm_host_threads(void)
 {
     const char *s = getenv("CHARM_HOST_THREADS");
     long t = s ? atol(s) : 0;
@@ -120,7 +120,7 @@ static int host_threads(void)
     return t < 1 ? 1 : (t > 64 ? 64 : (int) t);
 }
 
-typedef void (*range_fn)(void *arg, int64_t lo, int64_t hi, int part);
+typedef charm_range_fn range_fn;
 typedef struct { range_fn fn; void *arg; int64_t lo, hi; int part; } range_job_t;
 
 static void *range_run(void *p)
@@ -133,13 +133,13 @@ static void *range_run(void *p)
 /* number of contiguous parts [0, n) is split into (>= min_per_part each) */
 static int par_parts(int64_t n, int64_t min_per_part)
 {
-    int64_t t = host_threads();
+    int64_t t = charm_host_threads();
     if (n / min_per_part < t) t = n / min_per_part;
     return t < 1 ? 1 : (int) t;
 }
 
 /* fn over the `parts` contiguous ranges of [0, n), part 0 on the caller */
-static void par_for(int64_t n, int parts, range_fn fn, void *arg)
+void charm_par_for(int64_t n, int parts, range_fn fn, void *arg)
 {
     range_job_t job[64];
     pthread_t th[64];
@@ -356,7 +356,7 @@ static int forest_rebuild(charm_forest_t *f, const int8_t *act, int64_t **map_ou
     int p, parts = par_parts(f->n, 16384);
     memset(&r, 0, sizeof(r));
     r.f = f; r.act = act; r.child_code = child_code;
-    par_for(f->n, parts, rebuild_count, &r);
+    charm_par_for(f->n, parts, rebuild_count, &r);
     for (p = 0; p < parts; p++) { r.off[p] = n_new; n_new += r.cnt[p]; }
     r.q = (int32_t *) malloc((size_t) (n_new ? n_new : 1) * 4 * sizeof(int32_t));
     r.key = (uint64_t *) malloc((size_t) (n_new ? n_new : 1) * sizeof(uint64_t));
@@ -367,7 +367,7 @@ static int forest_rebuild(charm_forest_t *f, const int8_t *act, int64_t **map_ou
         charm_set_error("forest: out of memory");
         return CHARM_ERR_MEM;
     }
-    par_for(f->n, parts, rebuild_fill, &r);
+    charm_par_for(f->n, parts, rebuild_fill, &r);
     free(f->q); free(f->key);
     f->q = r.q; f->key = r.key; f->n = n_new;
     if (map_out) { *map_out = r.map; *n_map = n_new; }
@@ -470,7 +470,7 @@ static int forest_balance_map(charm_forest_t *f, int64_t **map, int8_t *fresh)
         b.fresh = fresh;
         b.act = (int8_t *) calloc((size_t) (f->n ? f->n : 1), 1);
         if (!b.act) { free(fresh); charm_set_error("forest: out of memory"); return CHARM_ERR_MEM; }
-        par_for(f->n, parts, balance_scan, &b);
+        charm_par_for(f->n, parts, balance_scan, &b);
         free(fresh);
         fresh = NULL;
         for (p = 0; p < parts; p++) any |= b.found[p];
@@ -482,7 +482,7 @@ static int forest_balance_map(charm_forest_t *f, int64_t **map, int8_t *fresh)
             if (rc) return rc;
             if (map && *map) {           /* compose maps: new -> old original */
                 compose_arg_t c = {m2, *map};
-                par_for(nm2, par_parts(nm2, 16384), compose_maps, &c);
+                charm_par_for(nm2, par_parts(nm2, 16384), compose_maps, &c);
                 free(*map);
             }
             if (map) *map = m2;
@@ -632,7 +632,7 @@ static int mesh_faces(const charm_forest_t *f, charm_mesh_t *m)
     int64_t nf = 0, o = 0;
     memset(&a, 0, sizeof(a));
     a.f = f;
-    par_for(f->n, parts, faces_scan, &a);
+    charm_par_for(f->n, parts, faces_scan, &a);
     for (p = 0; p < parts; p++) { nf += a.cnt[p]; if (a.err[p] && !err) err = a.err[p]; }
     if (!err) {
         m->f4 = (int32_t *) malloc((size_t) (nf ? nf : 1) * 4 * sizeof(int32_t));
@@ -734,20 +734,20 @@ static int mesh_neighbors(charm_mesh_t *m)
 {
     nbr_arg_t r;
     int64_t i, naux = 0;
-    int p, fparts = par_parts(m->nf, 16384), lparts = par_parts(m->n, 8192);
+    int p, fparts = par_parts(m->nf, 16384), lparts = par_parts(m->n, 4096);
     memset(&r, 0, sizeof(r));
     r.m = m;
     m->nbr = (int32_t *) malloc((size_t) (m->n ? m->n : 1) * 6 * sizeof(int32_t));
     if (!m->nbr) { charm_set_error("flatten: out of memory"); return CHARM_ERR_MEM; }
     for (i = 0; i < m->n * 6; i++) m->nbr[i] = INT32_MIN;
-    par_for(m->nf, fparts, nbr_slots, &r);
-    par_for(m->n, lparts, nbr_count, &r);
+    charm_par_for(m->nf, fparts, nbr_slots, &r);
+    charm_par_for(m->n, lparts, nbr_count, &r);
     for (p = 0; p < lparts; p++) { r.off[p] = naux; naux += r.cnt[p]; }
     m->aux = (int32_t *) malloc((size_t) (naux ? naux : 1) * 4 * sizeof(int32_t));
     if (!m->aux) { charm_set_error("flatten: out of memory"); return CHARM_ERR_MEM; }
-    par_for(m->n, lparts, nbr_number, &r);
-    par_for(m->nf, fparts, nbr_groups, &r);
-    par_for(m->n, lparts, nbr_check, &r);
+    charm_par_for(m->n, lparts, nbr_number, &r);
+    charm_par_for(m->nf, fparts, nbr_groups, &r);
+    charm_par_for(m->n, lparts, nbr_check, &r);
     for (p = 0; p < lparts; p++)
         if (r.bad[p]) { charm_set_error("flatten: an element face is not covered"); return CHARM_ERR_MESH; }
     for (i = 0; i < naux * 4; i++)
@@ -993,15 +993,15 @@ static int mesh_chunks(charm_mesh_t *m, int ch_e, int ch_f)
     if (!inc_ptr) goto done;
     {
         inc_arg_t I = {m, inc_ptr, NULL, NULL};
-        par_for(nf, par_parts(nf, 16384), inc_count, &I);
+        charm_par_for(nf, par_parts(nf, 16384), inc_count, &I);
         for (e = 0; e < n; e++) inc_ptr[e+1] += inc_ptr[e];
         inc = (int32_t *) malloc((size_t) (inc_ptr[n] + 1) * sizeof(int32_t));
         fill = (int32_t *) malloc((size_t) (n + 1) * sizeof(int32_t));
         if (!inc || !fill) goto done;
         memcpy(fill, inc_ptr, (size_t) n * sizeof(int32_t));
         I.inc = inc; I.fill = fill;
-        par_for(nf, par_parts(nf, 16384), inc_fill, &I);
-        par_for(n, par_parts(n, 8192), inc_sort, &I);
+        charm_par_for(nf, par_parts(nf, 16384), inc_fill, &I);
+        charm_par_for(n, par_parts(n, 8192), inc_sort, &I);
     }
 
     m->slot_ptr = (int32_t *) malloc((size_t) (n + 1) * sizeof(int32_t));
@@ -1019,7 +1019,7 @@ static int mesh_chunks(charm_mesh_t *m, int ch_e, int ch_f)
         goto done;
     memcpy(m->slot_ptr, inc_ptr, (size_t) (n + 1) * sizeof(int32_t));
     J.m = m; J.inc_ptr = inc_ptr; J.inc = inc; J.ch_e = ch_e; J.ch_f = ch_f; J.n = n; J.slots = m->slots;
-    par_for(nblk, par_parts(nblk, 1), chunk_blocks, &J);
+    charm_par_for(nblk, par_parts(nblk, 1), chunk_blocks, &J);
     for (b = 0; b < nblk; b++)
         if (J.err[b]) {
             rc = J.err[b];
@@ -1037,7 +1037,7 @@ static int mesh_chunks(charm_mesh_t *m, int ch_e, int ch_f)
     {
         chunk_merge_t M;
         M.m = m; M.J = &J; M.ch_off = ch_off; M.cf_off = cf_off;
-        par_for(nblk, par_parts(nblk, 1), chunk_merge, &M);
+        charm_par_for(nblk, par_parts(nblk, 1), chunk_merge, &M);
     }
     m->ch_ebeg[m->nch] = (int32_t) n;
     m->ch_fbeg[m->nch] = (int32_t) m->ncf;
@@ -1059,63 +1059,87 @@ void charm_pieces_free(charm_pieces_t *p)
     memset(p, 0, sizeof(*p));
 }
 
-/* The cut runs over contiguous chunk ranges on host threads: a counting pass,
- * then one that fills (40,000 leaves: 2.5-3.4 ms on one thread, 0.8-1.1 on
- * eight). */
+/* The cut runs over contiguous chunk ranges on host threads: a part writes its
+ * pieces from the entry of its first leaf and its faces from that leaf's first
+ * slot (every slot names a face of its piece, so the slots bound the face
+ * copies), and the parts are then moved together (40,328 leaves: 1.1 ms on one
+ * thread, 0.9 on eight). */
 typedef struct {
     const charm_mesh_t *m;
     charm_pieces_t *out;
-    int max_e, max_f, fill;
-    int64_t np[65], nf[65];            /* per part: counts, then (fill) first piece and face */
-    int32_t *mark, *rank;              /* per part, chunk_faces + 1 each */
+    int max_e, max_f;
+    int64_t np[64], nf[64];            /* per part: pieces and faces */
+    int32_t *rank;                     /* per part: chunk_faces + 1 */
+    uint64_t *bits;                    /* per part: chunk_faces / 64 + 1 */
 } cut_job_t;
+
+/* leaf e's faces into the piece's set: how many were new (a leaf that is its
+ * own periodic neighbour names one face twice) */
+static int cut_take(const charm_mesh_t *m, int64_t e, uint64_t *bits, uint16_t *fresh)
+{
+    int nnew = 0;
+    int32_t k;
+    for (k = m->slot_ptr[e]; k < m->slot_ptr[e + 1]; k++) {
+        const unsigned f = m->slots[k] >> 1;
+        const uint64_t b = (uint64_t) 1 << (f & 63);
+        if (!(bits[f >> 6] & b)) { bits[f >> 6] |= b; fresh[nnew++] = (uint16_t) f; }
+    }
+    return nnew;
+}
 
 static void cut_range(void *arg, int64_t lo, int64_t hi, int part)
 {
     cut_job_t *J = (cut_job_t *) arg;
     const charm_mesh_t *m = J->m;
     charm_pieces_t *out = J->out;
-    int32_t *mark = J->mark + (int64_t) part * (m->chunk_faces + 1);
+    uint64_t *bits = J->bits + (int64_t) part * (m->chunk_faces / 64 + 1);      /* the piece's faces */
     int32_t *rank = J->rank + (int64_t) part * (m->chunk_faces + 1);
-    int64_t c, e, k, np = J->fill ? J->np[part] : 0, ncf = J->fill ? J->nf[part] : 0;
+    const int64_t p0 = m->ch_ebeg[lo], f0 = m->slot_ptr[p0];
+    int64_t c, np = 0, ncf = 0;
+    uint16_t fresh[64];                                 /* at most 24 faces of a leaf */
     for (c = lo; c < hi; c++) {
-        const int64_t eb = m->ch_ebeg[c], ee = m->ch_ebeg[c + 1], fb = m->ch_fbeg[c], nf = m->ch_fbeg[c + 1] - fb;
-        int64_t pb = eb, f, cap = 0;
-        for (f = 0; f < nf; f++) mark[f] = -1;          /* the last piece (by its first leaf) that took the face */
+        const int64_t eb = m->ch_ebeg[c], ee = m->ch_ebeg[c + 1], fb = m->ch_fbeg[c];
+        const int64_t nw = (m->ch_fbeg[c + 1] - fb) / 64 + 1;
+        int64_t e, i, pb = eb;
+        int cap = 0, nnew = 0, j;
+        memset(bits, 0, (size_t) nw * sizeof(uint64_t));
         for (e = eb; e <= ee; e++) {
-            int64_t nnew = 0;
-            if (e < ee)
-                /* (a leaf that is its own periodic neighbour holds both sides
-                 * of the face in adjacent slots) */
-                for (k = m->slot_ptr[e]; k < m->slot_ptr[e + 1]; k++)
-                    nnew += mark[m->slots[k] >> 1] != pb &&
-                            !(k > m->slot_ptr[e] && m->slots[k - 1] >> 1 == m->slots[k] >> 1);
-            if (e == ee || (e > pb && (e - pb >= J->max_e || cap + nnew > J->max_f))) {
-                if (J->fill) {
-                    int64_t q, to = ncf;
-                    out->ch_ebeg[np] = (int32_t) pb;
-                    out->ch_fbeg[np] = (int32_t) ncf;
-                    out->ch_ref[np] = (int32_t) eb;
-                    for (f = 0; f < nf; f++)
-                        if (mark[f] == pb) {
-                            rank[f] = (int32_t) (to - ncf);
-                            memcpy(&out->cf4[4 * to], &m->cf4[4 * (fb + f)], 4 * sizeof(int32_t));
-                            to++;
-                        }
-                    for (q = m->slot_ptr[pb]; q < m->slot_ptr[e]; q++)
-                        out->slots[q] = (uint16_t) ((rank[m->slots[q] >> 1] << 1) | (m->slots[q] & 1));
-                }
+            int close = e == ee || e - pb >= J->max_e;
+            if (!close) {
+                nnew = cut_take(m, e, bits, fresh);
+                close = e > pb && cap + nnew > J->max_f;
+                if (close)
+                    for (j = 0; j < nnew; j++) bits[fresh[j] >> 6] &= ~((uint64_t) 1 << (fresh[j] & 63));
+            }
+            if (close) {
+                int64_t q, to = 0;
+                int32_t *cf = out->cf4 + 4 * (f0 + ncf);
+                out->ch_ebeg[p0 + np] = (int32_t) pb;
+                out->ch_fbeg[p0 + np] = (int32_t) ncf;
+                out->ch_ref[p0 + np] = (int32_t) eb;
                 np++;
-                ncf += cap;
+                for (i = 0; i < nw; i++) {
+                    uint64_t w = bits[i];
+                    for (; w; w &= w - 1, to++) {
+                        const int64_t f = 64 * i + __builtin_ctzll(w);
+                        rank[f] = (int32_t) (to << 1);
+                        memcpy(&cf[4 * to], &m->cf4[4 * (fb + f)], 4 * sizeof(int32_t));
+                    }
+                    bits[i] = 0;
+                }
+                ncf += to;
+                for (q = m->slot_ptr[pb]; q < m->slot_ptr[e]; q++)
+                    out->slots[q] = (uint16_t) (rank[m->slots[q] >> 1] | (m->slots[q] & 1));
+                if (e == ee) break;
                 pb = e;
                 cap = 0;
+                nnew = cut_take(m, e, bits, fresh);
             }
-            if (e < ee)
-                for (k = m->slot_ptr[e]; k < m->slot_ptr[e + 1]; k++)
-                    if (mark[m->slots[k] >> 1] != pb) { mark[m->slots[k] >> 1] = (int32_t) pb; cap++; }
+            cap += nnew;
         }
     }
-    if (!J->fill) { J->np[part] = np; J->nf[part] = ncf; }
+    J->np[part] = np;
+    J->nf[part] = ncf;
 }
 
 /* A piece's faces keep their chunk's order (by axis and kind) and a leaf its
@@ -1123,36 +1147,41 @@ static void cut_range(void *arg, int64_t lo, int64_t hi, int part)
 int charm_mesh_cut(const charm_mesh_t *m, int max_e, int max_f, charm_pieces_t *out)
 {
     cut_job_t J;
-    int p, parts = par_parts(m->n, 2048);
+    int64_t i;
+    int p, parts = par_parts(m->n, 8192);
+    if (parts > 8) parts = 8;
     if (parts > m->nch) parts = m->nch > 0 ? (int) m->nch : 1;
     memset(out, 0, sizeof(*out));
-    J.m = m; J.out = out; J.max_e = max_e; J.max_f = max_f; J.fill = 0;
-    J.mark = (int32_t *) malloc((size_t) parts * (m->chunk_faces + 1) * sizeof(int32_t));
+    J.m = m; J.out = out; J.max_e = max_e; J.max_f = max_f;
+    J.bits = (uint64_t *) malloc((size_t) parts * (m->chunk_faces / 64 + 1) * sizeof(uint64_t));
     J.rank = (int32_t *) malloc((size_t) parts * (m->chunk_faces + 1) * sizeof(int32_t));
-    if (!J.mark || !J.rank) goto nomem;
-    par_for(m->nch, parts, cut_range, &J);
-    for (p = 0; p < parts; p++) {
-        const int64_t np = J.np[p], nf = J.nf[p];
-        J.np[p] = out->nch; J.nf[p] = out->ncf;
-        out->nch += np; out->ncf += nf;
-    }
-    out->ch_ebeg = (int32_t *) malloc((size_t) (out->nch + 1) * sizeof(int32_t));
-    out->ch_fbeg = (int32_t *) malloc((size_t) (out->nch + 1) * sizeof(int32_t));
-    out->ch_ref = (int32_t *) malloc((size_t) (out->nch + 1) * sizeof(int32_t));
-    out->cf4 = (int32_t *) malloc((size_t) (out->ncf + 1) * 4 * sizeof(int32_t));
+    out->ch_ebeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->ch_fbeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->ch_ref = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+    out->cf4 = (int32_t *) malloc((size_t) (m->nslot + 1) * 4 * sizeof(int32_t));
     out->slots = (uint16_t *) malloc((size_t) (m->nslot + 1) * sizeof(uint16_t));
-    if (!out->ch_ebeg || !out->ch_fbeg || !out->ch_ref || !out->cf4 || !out->slots) goto nomem;
-    J.fill = 1;
-    par_for(m->nch, parts, cut_range, &J);
+    if (!J.bits || !J.rank || !out->ch_ebeg || !out->ch_fbeg || !out->ch_ref || !out->cf4 || !out->slots) {
+        free(J.bits); free(J.rank);
+        charm_pieces_free(out);
+        charm_set_error("mesh_cut: out of memory");
+        return CHARM_ERR_MEM;
+    }
+    charm_par_for(m->nch, parts, cut_range, &J);
+    for (p = 0; p < parts; p++) {
+        const int64_t p0 = m->ch_ebeg[m->nch * p / parts], f0 = m->slot_ptr[p0];
+        if (p) {
+            memmove(out->ch_ebeg + out->nch, out->ch_ebeg + p0, (size_t) J.np[p] * sizeof(int32_t));
+            memmove(out->ch_ref + out->nch, out->ch_ref + p0, (size_t) J.np[p] * sizeof(int32_t));
+            for (i = 0; i < J.np[p]; i++) out->ch_fbeg[out->nch + i] = (int32_t) (out->ch_fbeg[p0 + i] + out->ncf);
+            memmove(out->cf4 + 4 * out->ncf, out->cf4 + 4 * f0, (size_t) J.nf[p] * 4 * sizeof(int32_t));
+        }
+        out->nch += J.np[p];
+        out->ncf += J.nf[p];
+    }
     out->ch_ebeg[out->nch] = (int32_t) m->n;
     out->ch_fbeg[out->nch] = (int32_t) out->ncf;
-    free(J.mark); free(J.rank);
+    free(J.bits); free(J.rank);
     return CHARM_OK;
-nomem:
-    free(J.mark); free(J.rank);
-    charm_pieces_free(out);
-    charm_set_error("mesh_cut: out of memory");
-    return CHARM_ERR_MEM;
 }
 
 int charm_forest_flatten(const charm_forest_t *f, int chunk_elems, int chunk_faces,

@@ -6,6 +6,7 @@
 // the message of a failure is kept per host thread (charm_gpu_last_error).
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <pthread.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -16,6 +17,23 @@
 using namespace charm;
 
 extern "C" const char *charm_host_last_error(void);
+
+// Boundary faces of the mesh for the adjoint's boundary kernels (from the
+// neighbour table: codes -1..-6 are boundary faces): the leaves with one,
+// their face ranges, the faces (leaf * 8 + direction, ordered by leaf), and
+// the per-point scratch of their contributions.
+struct AdjBoundary {
+    int *elems, *ptr, *faces, *of;
+    void *part;
+    double *theta;
+    int n_elems, n_faces;
+};
+
+constexpr int kXferParts = 8;              // streams of a large state transfer
+constexpr size_t kPinBytes = 256 * 1024;   // pinned buffer of small transfers
+constexpr size_t kPinHead = 4096;          // error flag and reduction results ahead of it
+constexpr int kLiveBlocks = 96, kIdleBlocks = 48;
+constexpr size_t kIdleBytes = (size_t) 256 << 20;
 
 struct charm_gpu_ctx {
     charm_config_t cfg;
@@ -66,7 +84,83 @@ struct charm_gpu_ctx {
     double *d_stage64;        // FP64 staging for host transfers
     double *d_partial, *d_result;
     int *d_err;
+    // host side of the calls
+    int dev;                  // the device of the context
+    char *h_pin, *d_pin;      // pinned, mapped: flag, results, kPinBytes of small transfers (pin_mu)
+    hipStream_t xst[kXferParts];
+    AdjBoundary bnd;          // of the mesh, built by the first adjoint call on it
+    int bnd_ok;
+    // device blocks in use, and freed ones kept for the next request (mem_mu)
+    struct Block { void *p; size_t bytes; } live[kLiveBlocks], idle[kIdleBlocks];
+    int n_live, n_idle;
+    size_t idle_bytes;
+    pthread_mutex_t pin_mu, mem_mu;
 };
+
+namespace {
+struct Lock {
+    pthread_mutex_t *m;
+    explicit Lock(pthread_mutex_t *mu) : m(mu) { pthread_mutex_lock(m); }
+    ~Lock() { pthread_mutex_unlock(m); }
+};
+} // namespace
+
+// Device memory of a context.  A freed block is kept, up to kIdleBytes in
+// all, and serves the next request that fills at least half of it: a remesh
+// makes some fifteen allocations and as many frees, each a call of 5-100 us,
+// and so do the reverse stage and the point-wise fluxes.  Blocks are freed only
+// behind a synchronised stream.  The kept ones are given back before an
+// allocation fails, and with the context.
+static void idle_release(charm_gpu_ctx_t *c)
+{
+    for (int i = 0; i < c->n_idle; i++) (void) hipFree(c->idle[i].p);
+    c->n_idle = 0;
+    c->idle_bytes = 0;
+}
+
+static hipError_t dalloc(charm_gpu_ctx_t *c, void **p, size_t bytes)
+{
+    Lock lock(&c->mem_mu);
+    if (bytes < 256) bytes = 256;
+    int best = -1;
+    for (int i = 0; i < c->n_idle; i++)
+        if (c->idle[i].bytes >= bytes && c->idle[i].bytes / 2 <= bytes &&
+            (best < 0 || c->idle[i].bytes < c->idle[best].bytes)) best = i;
+    if (best >= 0 && c->n_live < kLiveBlocks) {
+        c->live[c->n_live++] = c->idle[best];
+        *p = c->idle[best].p;
+        c->idle_bytes -= c->idle[best].bytes;
+        c->idle[best] = c->idle[--c->n_idle];
+        return hipSuccess;
+    }
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && c->n_idle) {
+        (void) hipGetLastError();
+        idle_release(c);
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess && c->n_live < kLiveBlocks) { c->live[c->n_live].p = *p; c->live[c->n_live++].bytes = bytes; }
+    return e;
+}
+
+static void dfree(charm_gpu_ctx_t *c, void *p)
+{
+    if (!p) return;
+    Lock lock(&c->mem_mu);
+    for (int i = 0; i < c->n_live; i++)
+        if (c->live[i].p == p) {
+            const size_t b = c->live[i].bytes;
+            c->live[i] = c->live[--c->n_live];
+            if (c->n_idle < kIdleBlocks && b <= kIdleBytes - c->idle_bytes) {
+                c->idle[c->n_idle].p = p;
+                c->idle[c->n_idle++].bytes = b;
+                c->idle_bytes += b;
+                return;
+            }
+            break;
+        }
+    (void) hipFree(p);
+}
 
 #define HIPCHK(x)                                                                  \
     do {                                                                           \
@@ -86,8 +180,18 @@ extern "C" int charm_gpu_device_count(int *n)
     return CHARM_OK;
 }
 
+static void adj_boundary_free(charm_gpu_ctx_t *c)
+{
+    AdjBoundary &b = c->bnd;
+    void *bufs[] = {b.elems, b.ptr, b.faces, b.of, b.part, b.theta};
+    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++) dfree(c, bufs[i]);
+    memset(&b, 0, sizeof(b));
+    c->bnd_ok = 0;
+}
+
 static void free_mesh(charm_gpu_ctx_t *c)
 {
+    adj_boundary_free(c);
     void **p[] = {(void **) &c->d_level, (void **) &c->d_cf4, (void **) &c->d_aux,
                   (void **) &c->d_ch_ebeg, (void **) &c->d_ch_fbeg, (void **) &c->d_ch_ref, (void **) &c->d_slot_ptr,
                   (void **) &c->d_nbr, (void **) &c->d_slots, &c->B[0], &c->B[1], &c->B[2],
@@ -97,7 +201,7 @@ static void free_mesh(charm_gpu_ctx_t *c)
                   &c->d_glg, &c->d_gfg, &c->d_gfs, &c->d_gmb, (void **) &c->d_gfn, (void **) &c->d_gfe,
                   (void **) &c->d_glf, (void **) &c->d_glnb};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); i++)
-        if (*p[i]) { (void) hipFree(*p[i]); *p[i] = NULL; }
+        if (*p[i]) { dfree(c, *p[i]); *p[i] = NULL; }
     c->gm = 0; c->gnf = 0; c->gmb_of = NULL; c->temps_of = NULL;
     free(c->hq);
     c->hq = NULL;
@@ -143,6 +247,8 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
     if (ndev < 1) { charm_set_error("gpu_create: no HIP device"); return CHARM_ERR_HIP; }
     charm_gpu_ctx_t *c = (charm_gpu_ctx_t *) calloc(1, sizeof(charm_gpu_ctx_t));
     if (!c) { charm_set_error("gpu_create: out of memory"); return CHARM_ERR_MEM; }
+    pthread_mutex_init(&c->pin_mu, NULL);
+    pthread_mutex_init(&c->mem_mu, NULL);
     c->cfg = *cfg;
     c->prec = cfg->precision;
     c->sprec = cfg->precision == CHARM_FP32;
@@ -238,16 +344,21 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
     for (int d = 0; d < 3; d++) P.grav_f[d] = (float) P.grav[d];
     hipError_t e;
     if ((e = hipStreamCreate(&c->st)) != hipSuccess || (e = hipEventCreate(&c->ev0)) != hipSuccess ||
-        (e = hipEventCreate(&c->ev1)) != hipSuccess || (e = hipMalloc(&c->d_err, sizeof(int))) != hipSuccess ||
-        (e = hipMalloc(&c->d_result, 16 * sizeof(double))) != hipSuccess ||
+        (e = hipEventCreate(&c->ev1)) != hipSuccess || (e = hipGetDevice(&c->dev)) != hipSuccess ||
+        (e = hipHostMalloc((void **) &c->h_pin, kPinHead + kPinBytes, hipHostMallocDefault)) != hipSuccess ||
+        (e = hipHostGetDevicePointer((void **) &c->d_pin, c->h_pin, 0)) != hipSuccess ||
         (e = hipMalloc(&c->d_P, sizeof(DevParams))) != hipSuccess ||
         (e = hipMemcpyAsync(c->d_P, &c->P, sizeof(DevParams), hipMemcpyHostToDevice, c->st)) != hipSuccess ||
-        (e = hipMemsetAsync(c->d_err, 0, sizeof(int), c->st)) != hipSuccess ||
         (e = hipStreamSynchronize(c->st)) != hipSuccess) {
         charm_set_error("gpu_create: %s", hipGetErrorString(e));
         charm_gpu_destroy(c);
         return CHARM_ERR_HIP;
     }
+    // the kernels' error flag and the reductions' results are written to host
+    // memory: read after a synchronisation, without a copy (8 us each)
+    memset(c->h_pin, 0, kPinHead);
+    c->d_err = (int *) c->d_pin;
+    c->d_result = (double *) (c->d_pin + 64);
     *out = c;
     return CHARM_OK;
 }
@@ -257,12 +368,16 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
     if (!c) return CHARM_OK;
     if (c->st) (void) hipStreamSynchronize(c->st);
     free_mesh(c);
-    if (c->d_err) (void) hipFree(c->d_err);
-    if (c->d_result) (void) hipFree(c->d_result);
+    idle_release(c);
+    if (c->h_pin) (void) hipHostFree(c->h_pin);
+    for (int i = 0; i < kXferParts; i++)
+        if (c->xst[i]) (void) hipStreamDestroy(c->xst[i]);
     if (c->d_P) (void) hipFree(c->d_P);
     if (c->ev0) (void) hipEventDestroy(c->ev0);
     if (c->ev1) (void) hipEventDestroy(c->ev1);
     if (c->st) (void) hipStreamDestroy(c->st);
+    pthread_mutex_destroy(&c->pin_mu);
+    pthread_mutex_destroy(&c->mem_mu);
     free(c);
     return CHARM_OK;
 }
@@ -270,7 +385,7 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
 #define DMALLOC(ptr, bytes)                                                         \
     do {                                                                            \
         size_t b_ = (bytes) ? (bytes) : 16;                                         \
-        hipError_t e_ = hipMalloc((void **) &(ptr), b_);                            \
+        hipError_t e_ = dalloc(c, (void **) &(ptr), b_);                            \
         if (e_ != hipSuccess) {                                                     \
             charm_set_error("upload_mesh: hipMalloc(%zu) failed: %s", b_, hipGetErrorString(e_)); \
             free_mesh(c);                                                           \
@@ -317,6 +432,50 @@ struct Pieces {
     ~Pieces() { if (cut) charm_pieces_free(&p); }
 };
 
+// the mesh arrays and state buffers that the pieces do not change
+static int upload_arrays(charm_gpu_ctx_t *c, const charm_mesh_t *m)
+{
+    const size_t ssz = (size_t) m->n * 4 * c->nv * c->esz;
+    DMALLOC(c->d_level, (size_t) m->n);
+    DMALLOC(c->d_slot_ptr, (size_t) (m->n + 1) * sizeof(int));
+    DMALLOC(c->d_nbr, (size_t) m->n * 6 * sizeof(int));
+    DMALLOC(c->d_aux, (size_t) m->naux * sizeof(int4));
+    for (int i = 0; i < 3; i++) DMALLOC(c->B[i], ssz);
+    // FP64 staging: the state, or the 36 auxiliary coefficients of the
+    // Navier-Stokes test hook, whichever is larger
+    DMALLOC(c->d_stage64, (size_t) m->n * (4 * c->nv > 36 || !c->ph ? 4 * c->nv : 36) * sizeof(double));
+    DMALLOC(c->d_partial, (size_t) ((m->n + 255) / 256 + 1) * (c->nv + 1) * sizeof(double));
+    DMALLOC(c->d_q, (size_t) m->n * sizeof(int4));
+    if (c->ph) {
+        DMALLOC(c->d_auxf, (size_t) m->n * 36 * c->esz);
+        DMALLOC(c->d_vi, (size_t) m->n * 16 * c->esz);
+        if (c->cfg.use_visc && c->cfg.visc_br2_eta > 0.0) {
+            DMALLOC(c->d_auxo, (size_t) m->n * 36 * c->esz);
+            DMALLOC(c->d_lift, (size_t) m->n * kLiftSlots * kLiftFields * c->esz);
+        }
+        DMALLOC(c->d_dcoef, (size_t) m->n * c->nc * sizeof(double));
+        DMALLOC(c->d_chem, (size_t) m->n * sizeof(double));
+        if (c->P.newton_t) {
+            DMALLOC(c->d_tpt, (size_t) m->n * kMemoPlanes * kMemoRows * c->esz);
+        }
+    }
+    c->hq = (int32_t *) malloc((size_t) (m->n ? m->n : 1) * 4 * sizeof(int32_t));
+    if (!c->hq) { charm_set_error("upload_mesh: out of memory"); free_mesh(c); return CHARM_ERR_MEM; }
+    memcpy(c->hq, m->q, (size_t) m->n * 4 * sizeof(int32_t));
+    HIPCHK(hipMemcpyAsync(c->d_q, m->q, (size_t) m->n * sizeof(int4), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_level, m->level, (size_t) m->n, hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_slot_ptr, m->slot_ptr, (size_t) (m->n + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(c->d_nbr, m->nbr, (size_t) m->n * 6 * sizeof(int), hipMemcpyHostToDevice, c->st));
+    if (m->naux)
+        HIPCHK(hipMemcpyAsync(c->d_aux, m->aux, (size_t) m->naux * sizeof(int4), hipMemcpyHostToDevice, c->st));
+    for (int i = 0; i < 3; i++) HIPCHK(hipMemsetAsync(c->B[i], 0, ssz, c->st));
+    if (c->ph) {
+        HIPCHK(hipMemsetAsync(c->d_dcoef, 0, (size_t) m->n * c->nc * sizeof(double), c->st));
+        HIPCHK(hipMemsetAsync(c->d_chem, 0, (size_t) m->n * sizeof(double), c->st));
+    }
+    return CHARM_OK;
+}
+
 extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
 {
     if (!c || !m) { charm_set_error("upload_mesh: null argument"); return CHARM_ERR_ARG; }
@@ -346,56 +505,20 @@ extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
     }
     HIPCHK(hipStreamSynchronize(c->st));
     free_mesh(c);
-    const size_t ssz = (size_t) m->n * 4 * c->nv * c->esz;
     Pieces pc(c, m);
     if (pc.rc) return pc.rc;
-    DMALLOC(c->d_level, (size_t) m->n);
+    int rc = upload_arrays(c, m);
+    if (rc) return rc;
     DMALLOC(c->d_cf4, (size_t) pc.p.ncf * sizeof(int4));
     DMALLOC(c->d_ch_ebeg, (size_t) (pc.p.nch + 1) * sizeof(int));
     DMALLOC(c->d_ch_fbeg, (size_t) (pc.p.nch + 1) * sizeof(int));
     DMALLOC(c->d_ch_ref, (size_t) pc.p.nch * sizeof(int));
-    DMALLOC(c->d_slot_ptr, (size_t) (m->n + 1) * sizeof(int));
     DMALLOC(c->d_slots, (size_t) m->nslot * sizeof(uint16_t));
-    DMALLOC(c->d_nbr, (size_t) m->n * 6 * sizeof(int));
-    DMALLOC(c->d_aux, (size_t) m->naux * sizeof(int4));
-    for (int i = 0; i < 3; i++) DMALLOC(c->B[i], ssz);
-    // FP64 staging: the state, or the 36 auxiliary coefficients of the
-    // Navier-Stokes test hook, whichever is larger
-    DMALLOC(c->d_stage64, (size_t) m->n * (4 * c->nv > 36 || !c->ph ? 4 * c->nv : 36) * sizeof(double));
-    DMALLOC(c->d_partial, (size_t) ((m->n + 255) / 256 + 1) * (c->nv + 1) * sizeof(double));
-    DMALLOC(c->d_q, (size_t) m->n * sizeof(int4));
-    if (c->ph) {
-        DMALLOC(c->d_auxf, (size_t) m->n * 36 * c->esz);
-        DMALLOC(c->d_vi, (size_t) m->n * 16 * c->esz);
-        if (c->cfg.use_visc && c->cfg.visc_br2_eta > 0.0) {
-            DMALLOC(c->d_auxo, (size_t) m->n * 36 * c->esz);
-            DMALLOC(c->d_lift, (size_t) m->n * kLiftSlots * kLiftFields * c->esz);
-        }
-        DMALLOC(c->d_dcoef, (size_t) m->n * c->nc * sizeof(double));
-        DMALLOC(c->d_chem, (size_t) m->n * sizeof(double));
-        if (c->P.newton_t) {
-            DMALLOC(c->d_tpt, (size_t) m->n * kMemoPlanes * kMemoRows * c->esz);
-        }
-    }
-    c->hq = (int32_t *) malloc((size_t) (m->n ? m->n : 1) * 4 * sizeof(int32_t));
-    if (!c->hq) { charm_set_error("upload_mesh: out of memory"); free_mesh(c); return CHARM_ERR_MEM; }
-    memcpy(c->hq, m->q, (size_t) m->n * 4 * sizeof(int32_t));
-    HIPCHK(hipMemcpyAsync(c->d_q, m->q, (size_t) m->n * sizeof(int4), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_level, m->level, (size_t) m->n, hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_cf4, pc.p.cf4, (size_t) pc.p.ncf * sizeof(int4), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_ch_ebeg, pc.p.ch_ebeg, (size_t) (pc.p.nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_ch_fbeg, pc.p.ch_fbeg, (size_t) (pc.p.nch + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_ch_ref, pc.p.ch_ref, (size_t) pc.p.nch * sizeof(int), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_slot_ptr, m->slot_ptr, (size_t) (m->n + 1) * sizeof(int), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipMemcpyAsync(c->d_slots, pc.p.slots, (size_t) m->nslot * sizeof(uint16_t), hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_nbr, m->nbr, (size_t) m->n * 6 * sizeof(int), hipMemcpyHostToDevice, c->st));
-    if (m->naux)
-        HIPCHK(hipMemcpyAsync(c->d_aux, m->aux, (size_t) m->naux * sizeof(int4), hipMemcpyHostToDevice, c->st));
-    for (int i = 0; i < 3; i++) HIPCHK(hipMemsetAsync(c->B[i], 0, ssz, c->st));
-    if (c->ph) {
-        HIPCHK(hipMemsetAsync(c->d_dcoef, 0, (size_t) m->n * c->nc * sizeof(double), c->st));
-        HIPCHK(hipMemsetAsync(c->d_chem, 0, (size_t) m->n * sizeof(double), c->st));
-    }
     HIPCHK(hipStreamSynchronize(c->st));
     c->n = m->n; c->nch = pc.p.nch; c->ncf = pc.p.ncf; c->nslot = m->nslot; c->naux = m->naux;
     // the largest chunk there is sizes the workgroups and their LDS
@@ -503,23 +626,126 @@ static int need_mesh(const charm_gpu_ctx_t *c, int64_t n)
     return CHARM_OK;
 }
 
+// State transfers between host FP64 arrays [n][V][4] and a device state.  The
+// runtime copies pageable memory through its own pinned buffers on one host
+// thread, and a result array's pages are first touched there: 335 MB (2,097,152
+// leaves) take 13 ms in and 34 ms out.  From 12 MB the leaves go over in 4
+// ranges, from 64 MB in 8, a host thread and a stream each (335 MB: 7.1 and
+// 7.4 ms; 20 MB out 1.26 -> 0.57; at 5 MB the threads cost what they give).
+// Up to kPinBytes the conversion kernel works on pinned memory itself, which
+// saves the copy command (8 us).
+struct Xfer {
+    charm_gpu_ctx_t *c;
+    const void *src;
+    void *dst;
+    const double *in;
+    double *out;
+    hipError_t err[kXferParts];
+};
+
+static void xfer_part(void *arg, int64_t lo, int64_t hi, int part)
+{
+    Xfer *x = (Xfer *) arg;
+    charm_gpu_ctx_t *c = x->c;
+    const int nvk = 4 * c->nv;
+    const int64_t e0 = 64 * lo, e1 = 64 * hi < c->n ? 64 * hi : c->n;
+    const size_t bytes = (size_t) (e1 - e0) * nvk * sizeof(double);
+    double *stage = c->d_stage64 + e0 * nvk;
+    hipStream_t st = c->xst[part];
+    int dev = c->dev;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess && dev != c->dev) e = hipSetDevice(c->dev);
+    if (x->in) {
+        if (e == hipSuccess) e = hipMemcpyAsync(stage, x->in + e0 * nvk, bytes, hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = launch_convert(c->sprec, 0, c->d_stage64, x->dst, c->n, nvk, st, e0, e1);
+    } else {
+        if (e == hipSuccess) e = launch_convert(c->sprec, 1, x->src, c->d_stage64, c->n, nvk, st, e0, e1);
+        if (e == hipSuccess) e = hipMemcpyAsync(x->out + e0 * nvk, stage, bytes, hipMemcpyDeviceToHost, st);
+    }
+    const hipError_t es = hipStreamSynchronize(st);
+    if (dev != c->dev) (void) hipSetDevice(dev);
+    x->err[part] = e != hipSuccess ? e : es;
+}
+
+// ranges of a transfer (1: one copy on the context's stream), their streams made
+static int xfer_parts(charm_gpu_ctx_t *c, size_t bytes)
+{
+    int t = bytes >= ((size_t) 64 << 20) ? kXferParts : bytes >= ((size_t) 12 << 20) ? 4 : 1;
+    if (t > charm_host_threads()) t = charm_host_threads();
+    for (int i = 0; t > 1 && i < t; i++)
+        if (!c->xst[i] && hipStreamCreate(&c->xst[i]) != hipSuccess) { (void) hipGetLastError(); c->xst[i] = NULL; t = i; }
+    return t > 1 ? t : 1;
+}
+
+static hipError_t xfer(Xfer &x, int parts)
+{
+    // earlier work on the context's stream may use the staging or the state
+    hipError_t e = hipStreamSynchronize(x.c->st);
+    if (e != hipSuccess) return e;
+    charm_par_for((x.c->n + 63) / 64, parts, xfer_part, &x);
+    for (int i = 0; i < parts; i++)
+        if (x.err[i] != hipSuccess) return x.err[i];
+    return hipSuccess;
+}
+
+// u into the state dst; small arrays wait for the stream, larger ones may
+// leave the conversion on it
+static hipError_t state_in(charm_gpu_ctx_t *c, const double *u, void *dst)
+{
+    const int nvk = 4 * c->nv;
+    const size_t bytes = (size_t) c->n * nvk * sizeof(double);
+    if (bytes <= kPinBytes) {
+        Lock lock(&c->pin_mu);
+        memcpy(c->h_pin + kPinHead, u, bytes);
+        hipError_t e = launch_convert(c->sprec, 0, c->d_pin + kPinHead, dst, c->n, nvk, c->st);
+        const hipError_t es = hipStreamSynchronize(c->st);
+        return e != hipSuccess ? e : es;
+    }
+    const int parts = xfer_parts(c, bytes);
+    if (parts > 1) {
+        Xfer x = {c, NULL, dst, u, NULL, {}};
+        return xfer(x, parts);
+    }
+    const hipError_t e = hipMemcpyAsync(c->d_stage64, u, bytes, hipMemcpyHostToDevice, c->st);
+    if (e != hipSuccess) return e;
+    return launch_convert(c->sprec, 0, c->d_stage64, dst, c->n, nvk, c->st);
+}
+
+static hipError_t state_out(charm_gpu_ctx_t *c, const void *src, double *u)
+{
+    const int nvk = 4 * c->nv;
+    const size_t bytes = (size_t) c->n * nvk * sizeof(double);
+    if (bytes <= kPinBytes) {
+        Lock lock(&c->pin_mu);
+        hipError_t e = launch_convert(c->sprec, 1, src, c->d_pin + kPinHead, c->n, nvk, c->st);
+        const hipError_t es = hipStreamSynchronize(c->st);
+        if (e == hipSuccess) e = es;
+        if (e == hipSuccess) memcpy(u, c->h_pin + kPinHead, bytes);
+        return e;
+    }
+    const int parts = xfer_parts(c, bytes);
+    if (parts > 1) {
+        Xfer x = {c, src, NULL, NULL, u, {}};
+        return xfer(x, parts);
+    }
+    const hipError_t e = launch_convert(c->sprec, 1, src, c->d_stage64, c->n, nvk, c->st);
+    if (e != hipSuccess) return e;
+    return hipMemcpyAsync(u, c->d_stage64, bytes, hipMemcpyDeviceToHost, c->st);
+}
+
 extern "C" int charm_gpu_set_state(charm_gpu_ctx_t *c, const double *u, int64_t n)
 {
     int rc = need_mesh(c, n);
     if (rc) return rc;
     if (!u) { charm_set_error("set_state: null state"); return CHARM_ERR_ARG; }
-    const int64_t cnt = n * 4 * c->nv;
-    HIPCHK(hipMemcpyAsync(c->d_stage64, u, (size_t) cnt * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(launch_convert(c->sprec, 0, c->d_stage64, c->B[0], n, 4 * c->nv, c->st));
+    HIPCHK(state_in(c, u, c->B[0]));
     HIPCHK(hipStreamSynchronize(c->st));
     return CHARM_OK;
 }
 
-static int copy_out(charm_gpu_ctx_t *c, const void *src, double *u, int64_t n)
+static int copy_out(charm_gpu_ctx_t *c, const void *src, double *u)
 {
-    const int64_t cnt = n * 4 * c->nv;
-    HIPCHK(launch_convert(c->sprec, 1, src, c->d_stage64, n, 4 * c->nv, c->st));
-    HIPCHK(hipMemcpyAsync(u, c->d_stage64, (size_t) cnt * sizeof(double), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(state_out(c, src, u));
     HIPCHK(hipStreamSynchronize(c->st));
     return CHARM_OK;
 }
@@ -529,7 +755,7 @@ extern "C" int charm_gpu_get_state(charm_gpu_ctx_t *c, double *u, int64_t n)
     int rc = need_mesh(c, n);
     if (rc) return rc;
     if (!u) { charm_set_error("get_state: null state"); return CHARM_ERR_ARG; }
-    return copy_out(c, c->B[0], u, n);
+    return copy_out(c, c->B[0], u);
 }
 
 static StageArgs stage_args(charm_gpu_ctx_t *c, const void *U, const void *U0, void *out, int mode,
@@ -557,13 +783,19 @@ static LimArgs lim_args(charm_gpu_ctx_t *c, const void *W, const void *U0, void 
     return A;
 }
 
+// the kernels' error flag, cleared; behind a synchronised stream
+static int take_flag(charm_gpu_ctx_t *c)
+{
+    volatile int *f = (volatile int *) c->h_pin;
+    const int v = *f;
+    if (v) *f = 0;
+    return v;
+}
+
 static int check_flag(charm_gpu_ctx_t *c)
 {
-    int flag = 0;
-    HIPCHK(hipMemcpyAsync(&flag, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
-    if (flag) {
-        HIPCHK(hipMemsetAsync(c->d_err, 0, sizeof(int), c->st));
+    if (take_flag(c)) {
         charm_set_error("HLLC: inequality SL <= S* <= SR is FALSE (NaN or invalid state)");
         return CHARM_ERR_STATE;
     }
@@ -695,7 +927,7 @@ extern "C" int charm_gpu_residual(charm_gpu_ctx_t *c, double *out, int64_t n)
     HIPCHK(stage_launch(c, A));
     rc = check_flag(c);
     if (rc) return rc;
-    return copy_out(c, c->B[1], out, n);
+    return copy_out(c, c->B[1], out);
 }
 
 extern "C" int charm_gpu_limiter_bj(charm_gpu_ctx_t *c)
@@ -962,8 +1194,8 @@ static int reduce(charm_gpu_ctx_t *c, int mode, double *host)
     A.U = c->B[0]; A.level = c->d_level; A.partial = c->d_partial; A.result = c->d_result;
     A.n = c->n; A.mode = mode;
     HIPCHK(launch_reduce(c->sprec, c->nc, c->ph, A, c->P, c->st));
-    HIPCHK(hipMemcpyAsync(host, c->d_result, (size_t) (c->nv + 1) * sizeof(double), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    memcpy(host, c->h_pin + 64, (size_t) (c->nv + 1) * sizeof(double));
     return CHARM_OK;
 }
 
@@ -1025,9 +1257,8 @@ extern "C" int charm_gpu_conservation_sums_noalloc(charm_gpu_ctx_t *c, double *o
 extern "C" int charm_gpu_state_flag(charm_gpu_ctx_t *c, int *flag)
 {
     if (!c || !flag) { charm_set_error("state_flag: null argument"); return CHARM_ERR_ARG; }
-    HIPCHK(hipMemcpyAsync(flag, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipMemsetAsync(c->d_err, 0, sizeof(int), c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    *flag = take_flag(c);
     return CHARM_OK;
 }
 
@@ -1048,23 +1279,38 @@ extern "C" int charm_gpu_flux_batch(charm_gpu_ctx_t *c, int flux, int64_t n, con
     if (n == 0) return CHARM_OK;
     const size_t np = (size_t) n * (5 + c->nc) * sizeof(double);
     const size_t nn = (size_t) n * 3 * sizeof(double), no = (size_t) n * c->nv * sizeof(double);
-    double *dl = NULL, *dr = NULL, *dn = NULL, *dq = NULL;
-    hipError_t e = hipMalloc(&dl, np);
-    if (e == hipSuccess) e = hipMalloc(&dr, np);
-    if (e == hipSuccess) e = hipMalloc(&dn, nn);
-    if (e == hipSuccess) e = hipMalloc(&dq, no);
-    if (e == hipSuccess) e = hipMemcpyAsync(dl, prim_l, np, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) e = hipMemcpyAsync(dr, prim_r, np, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) e = hipMemcpyAsync(dn, normals, nn, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) {
-        FluxArgs A;
-        memset(&A, 0, sizeof(A));
-        A.prim_l = dl; A.prim_r = dr; A.normals = dn; A.out = dq; A.n = n;
+    FluxArgs A;
+    memset(&A, 0, sizeof(A));
+    A.n = n;
+    hipError_t e = hipSuccess;
+    if (2 * np + nn + no <= kPinBytes) {
+        // a few points: the kernel works on pinned memory (1,000 points 17 us
+        // less than four allocations, four copies and four frees)
+        Lock lock(&c->pin_mu);
+        char *h = c->h_pin + kPinHead;
+        double *d = (double *) (c->d_pin + kPinHead);
+        memcpy(h, prim_l, np); memcpy(h + np, prim_r, np); memcpy(h + 2 * np, normals, nn);
+        A.prim_l = d; A.prim_r = d + np / 8; A.normals = d + np / 4; A.out = d + np / 4 + nn / 8;
         e = launch_flux_points(c->sprec, c->nc, flux, A, c->P, c->st);
+        const hipError_t es = hipStreamSynchronize(c->st);
+        if (e == hipSuccess) e = es;
+        if (e == hipSuccess) memcpy(out, h + 2 * np + nn, no);
+    } else {
+        char *d = NULL;
+        e = dalloc(c, (void **) &d, 2 * np + nn + no);
+        if (e == hipSuccess) e = hipMemcpyAsync(d, prim_l, np, hipMemcpyHostToDevice, c->st);
+        if (e == hipSuccess) e = hipMemcpyAsync(d + np, prim_r, np, hipMemcpyHostToDevice, c->st);
+        if (e == hipSuccess) e = hipMemcpyAsync(d + 2 * np, normals, nn, hipMemcpyHostToDevice, c->st);
+        if (e == hipSuccess) {
+            A.prim_l = (double *) d; A.prim_r = (double *) (d + np); A.normals = (double *) (d + 2 * np);
+            A.out = (double *) (d + 2 * np + nn);
+            e = launch_flux_points(c->sprec, c->nc, flux, A, c->P, c->st);
+        }
+        if (e == hipSuccess) e = hipMemcpyAsync(out, A.out, no, hipMemcpyDeviceToHost, c->st);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+        if (e != hipSuccess) (void) hipStreamSynchronize(c->st);
+        dfree(c, d);
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(out, dq, no, hipMemcpyDeviceToHost, c->st);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    (void) hipFree(dl); (void) hipFree(dr); (void) hipFree(dn); (void) hipFree(dq);
     if (e != hipSuccess) { charm_set_error("flux_batch: %s", hipGetErrorString(e)); return CHARM_ERR_HIP; }
     return CHARM_OK;
 }
@@ -1085,12 +1331,12 @@ extern "C" int charm_gpu_flux_vjp_batch(charm_gpu_ctx_t *c, int flux, int64_t n,
     const size_t np = (size_t) n * (5 + c->nc) * sizeof(double);
     const size_t nn = (size_t) n * 3 * sizeof(double), nq = (size_t) n * c->nv * sizeof(double);
     double *dl = NULL, *dr = NULL, *dn = NULL, *dq = NULL, *bl = NULL, *br = NULL;
-    hipError_t e = hipMalloc(&dl, np);
-    if (e == hipSuccess) e = hipMalloc(&dr, np);
-    if (e == hipSuccess) e = hipMalloc(&dn, nn);
-    if (e == hipSuccess) e = hipMalloc(&dq, nq);
-    if (e == hipSuccess) e = hipMalloc(&bl, np);
-    if (e == hipSuccess) e = hipMalloc(&br, np);
+    hipError_t e = dalloc(c, (void **) &dl, np);
+    if (e == hipSuccess) e = dalloc(c, (void **) &dr, np);
+    if (e == hipSuccess) e = dalloc(c, (void **) &dn, nn);
+    if (e == hipSuccess) e = dalloc(c, (void **) &dq, nq);
+    if (e == hipSuccess) e = dalloc(c, (void **) &bl, np);
+    if (e == hipSuccess) e = dalloc(c, (void **) &br, np);
     if (e == hipSuccess) e = hipMemcpyAsync(dl, prim_l, np, hipMemcpyHostToDevice, c->st);
     if (e == hipSuccess) e = hipMemcpyAsync(dr, prim_r, np, hipMemcpyHostToDevice, c->st);
     if (e == hipSuccess) e = hipMemcpyAsync(dn, normals, nn, hipMemcpyHostToDevice, c->st);
@@ -1106,7 +1352,7 @@ extern "C" int charm_gpu_flux_vjp_batch(charm_gpu_ctx_t *c, int flux, int64_t n,
     if (e == hipSuccess) e = hipMemcpyAsync(prim_r_bar, br, np, hipMemcpyDeviceToHost, c->st);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     (void) hipStreamSynchronize(c->st);
-    (void) hipFree(dl); (void) hipFree(dr); (void) hipFree(dn); (void) hipFree(dq); (void) hipFree(bl); (void) hipFree(br);
+    dfree(c, dl); dfree(c, dr); dfree(c, dn); dfree(c, dq); dfree(c, bl); dfree(c, br);
     if (e != hipSuccess) { charm_set_error("flux_vjp_batch: %s", hipGetErrorString(e)); return CHARM_ERR_HIP; }
     return CHARM_OK;
 }
@@ -1196,7 +1442,7 @@ extern "C" int charm_gpu_remesh(charm_gpu_ctx_t *c, const charm_mesh_t *m, const
     hipError_t e = hipSuccess;
     rc = charm_gpu_upload_mesh(c, m);
     if (!rc) {
-        e = hipMalloc((void **) &d_map, (size_t) (m->n ? m->n : 1) * sizeof(int64_t));
+        e = dalloc(c, (void **) &d_map, (size_t) (m->n ? m->n : 1) * sizeof(int64_t));
         if (e == hipSuccess) e = hipMemcpyAsync(d_map, map, (size_t) m->n * sizeof(int64_t), hipMemcpyHostToDevice, c->st);
         if (e == hipSuccess) {
             ProjArgs A;
@@ -1207,9 +1453,9 @@ extern "C" int charm_gpu_remesh(charm_gpu_ctx_t *c, const charm_mesh_t *m, const
         if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     }
     (void) hipStreamSynchronize(c->st);
-    if (d_map) (void) hipFree(d_map);
-    (void) hipFree(u_old);
-    (void) hipFree(q_old);
+    dfree(c, d_map);
+    dfree(c, u_old);
+    dfree(c, q_old);
     if (rc) return rc;
     if (e != hipSuccess) { charm_set_error("remesh: %s", hipGetErrorString(e)); return CHARM_ERR_HIP; }
     return CHARM_OK;
@@ -1404,34 +1650,18 @@ extern "C" int charm_gpu_objective(charm_gpu_ctx_t *c, double dt, int nsteps, co
     if (!lo || !hi || !J) { charm_set_error("objective: null argument"); return CHARM_ERR_ARG; }
     const int64_t nblk = (c->n + 255) / 256;
     double *part = NULL;
-    HIPCHK(hipMalloc((void **) &part, (size_t) nsteps * nblk * sizeof(double)));
+    HIPCHK(dalloc(c, (void **) &part, (size_t) nsteps * nblk * sizeof(double)));
     rc = adj_forward(c, dt, nsteps, 1, lo, hi, NULL, NULL, part, nblk, J);
-    (void) hipFree(part);
+    (void) hipStreamSynchronize(c->st);
+    dfree(c, part);
     return rc;
 }
 
-// Boundary faces of the mesh for the adjoint's boundary kernels (from the
-// neighbour table: codes -1..-6 are boundary faces): the leaves with one,
-// their face ranges, the faces (leaf * 8 + direction, ordered by leaf), and
-// the per-point scratch of their contributions.
-struct AdjBoundary {
-    int *elems, *ptr, *faces, *of;
-    void *part;
-    double *theta;
-    int n_elems, n_faces;
-};
-
-static void adj_boundary_free(AdjBoundary &b)
+// The adjoint's boundary tables, built once per mesh.
+static int adj_boundary(charm_gpu_ctx_t *c)
 {
-    void *bufs[] = {b.elems, b.ptr, b.faces, b.of, b.part, b.theta};
-    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
-        if (bufs[i]) (void) hipFree(bufs[i]);
-    memset(&b, 0, sizeof(b));
-}
-
-static int adj_boundary(charm_gpu_ctx_t *c, AdjBoundary &b)
-{
-    memset(&b, 0, sizeof(b));
+    AdjBoundary &b = c->bnd;
+    if (c->bnd_ok) return CHARM_OK;
     const int64_t n = c->n;
     int *nbr = (int *) malloc((size_t) n * 6 * sizeof(int));
     int *elems = (int *) malloc((size_t) n * sizeof(int));
@@ -1457,25 +1687,26 @@ static int adj_boundary(charm_gpu_ctx_t *c, AdjBoundary &b)
         }
     }
     if (e == hipSuccess && ne > 0) {
-        e = hipMalloc((void **) &b.elems, (size_t) ne * sizeof(int));
-        if (e == hipSuccess) e = hipMalloc((void **) &b.ptr, ((size_t) ne + 1) * sizeof(int));
-        if (e == hipSuccess) e = hipMalloc((void **) &b.faces, (size_t) nf * sizeof(int));
-        if (e == hipSuccess) e = hipMalloc(&b.part, (size_t) nf * 6 * 4 * c->nv * c->esz);
-        if (e == hipSuccess) e = hipMalloc((void **) &b.theta, (size_t) nf * 6 * 3 * sizeof(double));
+        e = dalloc(c, (void **) &b.elems, (size_t) ne * sizeof(int));
+        if (e == hipSuccess) e = dalloc(c, (void **) &b.ptr, ((size_t) ne + 1) * sizeof(int));
+        if (e == hipSuccess) e = dalloc(c, (void **) &b.faces, (size_t) nf * sizeof(int));
+        if (e == hipSuccess) e = dalloc(c, &b.part, (size_t) nf * 6 * 4 * c->nv * c->esz);
+        if (e == hipSuccess) e = dalloc(c, (void **) &b.theta, (size_t) nf * 6 * 3 * sizeof(double));
         if (e == hipSuccess) e = hipMemcpy(b.elems, elems, (size_t) ne * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(b.ptr, ptr, ((size_t) ne + 1) * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(b.faces, faces, (size_t) nf * sizeof(int), hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = hipMalloc((void **) &b.of, (size_t) n * sizeof(int));
+        if (e == hipSuccess) e = dalloc(c, (void **) &b.of, (size_t) n * sizeof(int));
         if (e == hipSuccess) e = hipMemcpy(b.of, of, (size_t) n * sizeof(int), hipMemcpyHostToDevice);
     }
     free(nbr); free(elems); free(ptr); free(faces); free(of);
     if (e != hipSuccess) {
-        adj_boundary_free(b);
+        adj_boundary_free(c);
         charm_set_error("adjoint: %s", hipGetErrorString(e));
         return CHARM_ERR_HIP;
     }
     b.n_elems = ne;
     b.n_faces = nf;
+    c->bnd_ok = 1;
     return CHARM_OK;
 }
 
@@ -1495,22 +1726,20 @@ extern "C" int charm_gpu_stage_vjp(charm_gpu_ctx_t *c, double dt, const double *
         return CHARM_ERR_UNSUPPORTED;
     }
     if ((rc = adj_bnd_supported(c))) return rc;
-    const size_t ssz = (size_t) n * 4 * c->nv * c->esz, dsz = (size_t) n * 4 * c->nv * sizeof(double);
-    AdjBoundary bnd;
-    if ((rc = adj_boundary(c, bnd))) return rc;
+    const size_t ssz = (size_t) n * 4 * c->nv * c->esz;
+    if ((rc = adj_boundary(c))) return rc;
+    const AdjBoundary &bnd = c->bnd;
     int dev = 0, lds_max = 0;
     const bool chunked = c->sprec && hipGetDevice(&dev) == hipSuccess &&
                          hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
                          adj_chunk_smem_bytes(1, c->nc, c->max_faces) <= (size_t) lds_max;
     (void) hipGetLastError();
     char *dU = NULL, *dX = NULL, *dO = NULL;
-    hipError_t e = hipMalloc((void **) &dU, ssz);
-    if (e == hipSuccess) e = hipMalloc((void **) &dX, ssz);
-    if (e == hipSuccess) e = hipMalloc((void **) &dO, ssz);
-    if (e == hipSuccess) e = hipMemcpyAsync(c->d_stage64, u, dsz, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) e = launch_convert(c->sprec, 0, c->d_stage64, dU, n, 4 * c->nv, c->st);
-    if (e == hipSuccess) e = hipMemcpyAsync(c->d_stage64, x, dsz, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) e = launch_convert(c->sprec, 0, c->d_stage64, dX, n, 4 * c->nv, c->st);
+    hipError_t e = dalloc(c, (void **) &dU, ssz);
+    if (e == hipSuccess) e = dalloc(c, (void **) &dX, ssz);
+    if (e == hipSuccess) e = dalloc(c, (void **) &dO, ssz);
+    if (e == hipSuccess) e = state_in(c, u, dU);
+    if (e == hipSuccess) e = state_in(c, x, dX);
     if (e == hipSuccess) {
         AdjArgs A;
         memset(&A, 0, sizeof(A));
@@ -1527,14 +1756,10 @@ extern "C" int charm_gpu_stage_vjp(charm_gpu_ctx_t *c, double dt, const double *
         A.c_in = 1.0; A.c_out = 1.0; A.c_acc = 0.0; A.c_acc2 = 0.0;
         e = launch_adj_stage(c->sprec, c->nc, c->cfg.flux, A, c->P, c->st);
     }
-    if (e == hipSuccess) e = launch_convert(c->sprec, 1, dO, c->d_stage64, n, 4 * c->nv, c->st);
-    if (e == hipSuccess) e = hipMemcpyAsync(out, c->d_stage64, dsz, hipMemcpyDeviceToHost, c->st);
+    if (e == hipSuccess) e = state_out(c, dO, out);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
     (void) hipStreamSynchronize(c->st);
-    void *bufs[] = {dU, dX, dO};
-    for (size_t i = 0; i < 3; i++)
-        if (bufs[i]) (void) hipFree(bufs[i]);
-    adj_boundary_free(bnd);
+    dfree(c, dU); dfree(c, dX); dfree(c, dO);
     if (e != hipSuccess) { charm_set_error("stage_vjp: %s", hipGetErrorString(e)); return CHARM_ERR_HIP; }
     return check_flag(c);
 }
@@ -1548,7 +1773,6 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
     if (!lo || !hi || !J) { charm_set_error("adjoint: null argument"); return CHARM_ERR_ARG; }
     const int64_t n = c->n, nblk = (n + 255) / 256;
     const size_t ssz = (size_t) n * 4 * c->nv * c->esz;
-    const int64_t m = n * 4 * c->nv;
     // ckpt = 0: every stage state of the forward pass is kept (one segment
     // of nsteps steps filled by the forward pass, no recompute); else
     // checkpoints every ckpt steps and segments recomputed in two buffers
@@ -1564,8 +1788,8 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
     hipStream_t st2 = NULL;
     hipEvent_t ev_ready[2] = {NULL, NULL}, ev_done[2] = {NULL, NULL};
     double *part = NULL, *theta = NULL;
-    AdjBoundary bnd;
-    if ((rc = adj_boundary(c, bnd))) return rc;
+    if ((rc = adj_boundary(c))) return rc;
+    const AdjBoundary &bnd = c->bnd;
     // FP32: the chunked face-centric stage adjoint when its LDS fits a
     // workgroup (else, and in FP64, the element-centric one)
     int dev = 0, lds_max = 0;
@@ -1573,8 +1797,8 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
                          hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
                          adj_chunk_smem_bytes(1, c->nc, c->max_faces) <= (size_t) lds_max;
     (void) hipGetLastError();
-    hipError_t e = ncp > 1 ? hipMalloc((void **) &cp, (size_t) (ncp - 1) * ssz) : hipSuccess;
-    if (e == hipSuccess) e = hipMalloc((void **) &seg, (size_t) nseg_buf * (3 * seg_len + 1) * ssz);
+    hipError_t e = ncp > 1 ? dalloc(c, (void **) &cp, (size_t) (ncp - 1) * ssz) : hipSuccess;
+    if (e == hipSuccess) e = dalloc(c, (void **) &seg, (size_t) nseg_buf * (3 * seg_len + 1) * ssz);
     if (e == hipSuccess) e = hipStreamCreate(&st2);
     for (int i = 0; i < 2 && e == hipSuccess; i++) {
         e = hipEventCreateWithFlags(&ev_ready[i], hipEventDisableTiming);
@@ -1582,11 +1806,11 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
     }
     segb[0] = seg;
     segb[1] = (seg && nseg_buf == 2) ? seg + (size_t) (3 * seg_len + 1) * ssz : seg;
-    if (e == hipSuccess) e = hipMalloc((void **) &la, ssz);
-    if (e == hipSuccess) e = hipMalloc((void **) &lb, ssz);
-    if (e == hipSuccess) e = hipMalloc((void **) &lc, ssz);
-    if (e == hipSuccess) e = hipMalloc((void **) &part, (size_t) nsteps * nblk * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void **) &theta, (size_t) n * 3 * sizeof(double));
+    if (e == hipSuccess) e = dalloc(c, (void **) &la, ssz);
+    if (e == hipSuccess) e = dalloc(c, (void **) &lb, ssz);
+    if (e == hipSuccess) e = dalloc(c, (void **) &lc, ssz);
+    if (e == hipSuccess) e = dalloc(c, (void **) &part, (size_t) nsteps * nblk * sizeof(double));
+    if (e == hipSuccess) e = dalloc(c, (void **) &theta, (size_t) n * 3 * sizeof(double));
     float ms_f = 0.f, ms_a = 0.f;
     if (e != hipSuccess) {
         charm_set_error("adjoint: device memory: %s", hipGetErrorString(e));
@@ -1673,8 +1897,7 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
     ADJ_CHK(hipEventSynchronize(c->ev1));
     ADJ_CHK(hipEventElapsedTime(&ms_a, c->ev0, c->ev1));
     if (grad_u0) {
-        ADJ_CHK(launch_convert(c->sprec, 1, la, c->d_stage64, n, 4 * c->nv, c->st));
-        ADJ_CHK(hipMemcpyAsync(grad_u0, c->d_stage64, (size_t) m * sizeof(double), hipMemcpyDeviceToHost, c->st));
+        ADJ_CHK(state_out(c, la, grad_u0));
     }
     if (grad_theta) {
         double *h = (double *) malloc((size_t) n * 3 * sizeof(double));
@@ -1700,8 +1923,6 @@ done:
         if (ev_done[i]) (void) hipEventDestroy(ev_done[i]);
     }
     void *bufs[] = {cp, seg, la, lb, lc, part, theta};
-    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++)
-        if (bufs[i]) (void) hipFree(bufs[i]);
-    adj_boundary_free(bnd);
+    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++) dfree(c, bufs[i]);
     return rc;
 }

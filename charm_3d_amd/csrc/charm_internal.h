@@ -52,6 +52,13 @@ struct charm_mesh {
     uint16_t *slots;        /* local face index << 1 | side */
 };
 
+/* host threads: CHARM_HOST_THREADS, else OMP_NUM_THREADS, else the online
+ * cores, in [1, 64]; fn over `parts` (at most 64) contiguous ranges of [0, n),
+ * a thread each, part 0 on the caller */
+typedef void (*charm_range_fn)(void *arg, int64_t lo, int64_t hi, int part);
+int  charm_host_threads(void);
+void charm_par_for(int64_t n, int parts, charm_range_fn fn, void *arg);
+
 /* The chunks of a mesh cut into pieces of at most max_e leaves and max_f
  * faces (more only where one leaf has more): the chunk arrays of a mesh, and
  * per piece the first leaf of the chunk it was cut from. */

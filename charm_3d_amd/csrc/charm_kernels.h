@@ -220,7 +220,9 @@ hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t st)
 hipError_t launch_ns(int prec, int what, int nc, const NsArgs &A, const DevParams &P, hipStream_t st);
 hipError_t launch_amr_indicator(int prec, int nc, int ph, const AmrArgs &A, const DevParams &P, hipStream_t st);
 hipError_t launch_amr_project(int prec, const ProjArgs &A, hipStream_t st);
-hipError_t launch_convert(int prec, int to_f64, const void *src, void *dst, int64_t n, int nvk, hipStream_t st);
+// leaves [e0, e1) (all with e1 = -1) of the n
+hipError_t launch_convert(int prec, int to_f64, const void *src, void *dst, int64_t n, int nvk, hipStream_t st,
+                          int64_t e0 = 0, int64_t e1 = -1);
 // HLLC branch comparison of two FP64 states on one chunked octree mesh
 constexpr int kHllcBits = 9;
 struct FlipArgs {
