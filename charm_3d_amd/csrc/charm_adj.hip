@@ -3,16 +3,15 @@
 // linearisation of one stage S(U) = U - dt A^-1 int(U), the gradient of the
 // objective Q(U) = sum over the leaves of a box of int p, and Q itself.
 //
-// A stage adjoint is element-centric: one thread per leaf forms
+// A stage adjoint forms per leaf
 //   T = sb + (d int / d U)^T W,  W = -dt A^-1 sb,  sb = c_in X,
-// from the volume term and every point of its six face slots.  At each point
-// the pointwise numerics (cons_to_prim, boundary state, HLLC / LF) run on
-// forward-mode dual numbers whose tangents are this leaf's point values;
-// the contraction s = sum_v q_v G_v with the adjoint weights G of both sides
-// then carries d s / d u(point) in its tangents.  Every interior point is
-// evaluated from both sides, each side keeping its own derivative (no
-// atomics).  The inlet parameters (velocity x, T, p of one boundary face)
-// get their own dual pass.
+// from the volume term and every point of its six face slots: one primal
+// evaluation and one hand-written reverse sweep per point, by leaves
+// (k_adj_leaves: every interior point from both sides, each side keeping its
+// own derivative) or by chunks (k_adj_chunk: once per chunk that holds a side);
+// no atomics.  Boundary points run on forward-mode dual numbers (the boundary
+// state functions), the inlet parameters (velocity x, T, p of one boundary
+// face) in a dual pass of their own.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "charm_device.hpp"
@@ -98,16 +97,17 @@ __device__ __forceinline__ void inlet_dual(const DevParams &P, int face, const P
 
 // Volume term of a stage adjoint at leaf e (coefficients u, adjoint weights
 // w): ub += (d / d u) of sum_d sum_v cw_dv F_d,v(t) - sum_{v<3} g_v wJ w(ph) rho
-// over the 8 Gauss points, cw_dv = -(wJ / h) w[v][1 + d]
+// over the Gauss points [g0, g1) of the 8, cw_dv = -(wJ / h) w[v][1 + d]
 template <typename R, int NC>
-__device__ __forceinline__ void adj_volume(const DevParams &P, const R *u, const R *w, R h, R hinv, R *ub)
+__device__ __forceinline__ void adj_volume(const DevParams &P, const R *u, const R *w, R h, R hinv, R *ub,
+                                           int g0 = 0, int g1 = 8)
 {
     constexpr int NV = 4 + NC;
     const R gph = R(0.28867513459481288225);
     const R wj = h * h * h * R(0.125);
     const R f = -wj * hinv;
     #pragma unroll 1
-    for (int g = 0; g < 8; g++) {
+    for (int g = g0; g < g1; g++) {
         const R ph[3] = {(g & 1) ? gph : -gph, (g & 2) ? gph : -gph, (g & 4) ? gph : -gph};
         R t[NV], tb[NV];
         #pragma unroll
@@ -153,10 +153,11 @@ __device__ __forceinline__ void adj_volume(const DevParams &P, const R *u, const
 
 } // namespace
 
-// Interior part of one stage adjoint: the volume term and every interior
-// face point of leaf e, each through the hand-written reverse sweep (the
-// primal at the point, then the flux and cons_to_prim VJPs for e's side).
-// Boundary faces are added by k_adj_bnd_pts / k_adj_bnd_sum.
+// Stage adjoint of large FP64 meshes without hanging faces, one thread per
+// leaf: the volume term and every interior face point of leaf e, each through
+// the reverse sweep (the primal at the point, then the flux and cons_to_prim
+// VJPs for e's side); a leaf's state and weights are loaded once.  The boundary
+// faces' parts come from k_adj_bnd_pts.
 template <typename R, int NC, int FLUX>
 __global__ __launch_bounds__(128)
 void k_adj_stage(AdjArgs A, DevParams P)
@@ -223,15 +224,6 @@ void k_adj_stage(AdjArgs A, DevParams P)
         const R sign = (d & 1) ? R(1) : R(-1);
         const int a = d >> 1;
         if (nb >= 0) {
-            R o1 = R(0), o2 = R(0), m = R(1);
-            if (A.level[nb] != lev) {
-                // e is sub-face j of the coarser neighbour's face
-                const int4 grp = A.aux[-kNbrAuxBase - A.nbr[6 * nb + (d ^ 1)]];
-                const int j = (grp.x == e) ? 0 : ((grp.y == e) ? 1 : ((grp.z == e) ? 2 : 3));
-                o1 = (j & 1) ? R(0.25) : R(-0.25);
-                o2 = (j & 2) ? R(0.25) : R(-0.25);
-                m = R(0.5);
-            }
             R un[4 * NV], wn[4 * NV];
             load_coeffs<R, NV>(U, n, nb, un);
             adj_weights<R, NV>(A, P, X, nb, wn);
@@ -240,30 +232,29 @@ void k_adj_stage(AdjArgs A, DevParams P)
             for (int k = 0; k < 6; k++) {
                 R ps[3], pn[3];
                 face_point<R>(d, k, R(0), R(0), R(1), ps);
-                face_point<R>(d ^ 1, k, o1, o2, m, pn);
+                face_point<R>(d ^ 1, k, R(0), R(0), R(1), pn);
                 point(un, wn, a, ps, pn, wjf, sign);
-            }
-        } else if (nb <= -kNbrAuxBase) {
-            const int4 grp = A.aux[-kNbrAuxBase - nb];
-            const int q4[4] = {grp.x, grp.y, grp.z, grp.w};
-            const R wjf = R(0.25) * h * h * R(1.0 / 6.0);
-            #pragma unroll 1
-            for (int j = 0; j < 4; j++) {
-                R un[4 * NV], wn[4 * NV];
-                load_coeffs<R, NV>(U, n, q4[j], un);
-                adj_weights<R, NV>(A, P, X, q4[j], wn);
-                const R o1 = (j & 1) ? R(0.25) : R(-0.25), o2 = (j & 2) ? R(0.25) : R(-0.25);
-                #pragma unroll 1
-                for (int k = 0; k < 6; k++) {
-                    R ps[3], pn[3];
-                    face_point<R>(d, k, o1, o2, R(0.5), ps);
-                    face_point<R>(d ^ 1, k, R(0), R(0), R(1), pn);
-                    point(un, wn, a, ps, pn, wjf, sign);
-                }
             }
         }
     }
 
+    const int bi = A.bnd_of ? A.bnd_of[e] : -1;
+    if (bi >= 0) {
+        const R *__restrict__ part = reinterpret_cast<const R *>(A.bnd_part);
+        double th[3] = {0.0, 0.0, 0.0};
+        for (int p = 6 * A.bnd_ptr[bi]; p < 6 * A.bnd_ptr[bi + 1]; p++) {
+            #pragma unroll
+            for (int j = 0; j < 4 * NV; j++) ub[j] += part[(size_t) p * 4 * NV + j];
+            if (A.theta_bar) {
+                #pragma unroll
+                for (int j = 0; j < 3; j++) th[j] += A.bnd_theta[3 * (size_t) p + j];
+            }
+        }
+        if (A.theta_bar) {
+            #pragma unroll
+            for (int j = 0; j < 3; j++) A.theta_bar[3 * (size_t) e + j] += th[j];
+        }
+    }
     // not __restrict__: the last stage adjoint accumulates into its own output
     R *out = reinterpret_cast<R *>(A.OUT);
     const R *acc = reinterpret_cast<const R *>(A.ACC);
@@ -278,6 +269,231 @@ void k_adj_stage(AdjArgs A, DevParams P)
     }
 }
 
+// One side's plane of a (sub)face in its point coordinates (g1, g2), in the
+// face frame: at the side's normal coordinate pn, its tangential coordinates
+// o1 + m g1, o2 + m g2.  p: the leaf's first coefficient of the variable.
+template <typename R>
+__device__ __forceinline__ void trace_plane(const R *__restrict__ p, int64_t n, int a, int t1, int t2, R pn, R o1,
+                                            R o2, R m, R &c0, R &c1, R &c2)
+{
+    const R k1 = p[(1 + t1) * n], k2 = p[(1 + t2) * n];
+    c0 = p[0] + pn * p[(1 + a) * n] + o1 * k1 + o2 * k2;
+    c1 = m * k1;
+    c2 = m * k2;
+}
+
+// Stage adjoint leaf by leaf: a workgroup of four waves takes 32 leaves and
+// lists their interior (sub)faces, 6 a leaf and 3 more where four smaller
+// neighbours share one; a lane takes a (sub)face, its six points and the leaf's
+// side of the reverse sweep, one group of 64 lanes the leaves' volume points.
+// The direction differs between lanes, so traces are loaded in the face frame
+// by address: a plane each (value and two tangential slopes, 3 numbers per
+// variable instead of 4), the difference of the two sides' weights likewise,
+// and the gradient's moments over the points.  The moments meet in LDS; the
+// boundary faces' per-point parts (k_adj_bnd_pts, launched first) are added
+// there, every sum in a fixed order.  Bound by the latency and issue of one or
+// two waves per SIMD (the registers).  One thread per leaf, walking its faces
+// and volume points in a row, took 480 us in FP64 at 9,192 leaves; this 58.
+template <typename R, int NC, int FLUX, int WG>
+__global__ __launch_bounds__(256, WG)
+void k_adj_leaves(AdjArgs A, DevParams P)
+{
+    constexpr int NV = 4 + NC, LP = kAdjLeaves, NF = 6 * LP, VP = 64 / LP;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    R *vol = reinterpret_cast<R *>(smem_raw);                            // [4 NV][64]
+    R *mom = vol + 4 * NV * 64;                                          // [items][3][NV], frame order
+    uint16_t *list = reinterpret_cast<uint16_t *>(mom + (size_t) A.max_items * 3 * NV);
+    __shared__ uint16_t base[NF + 1];
+    __shared__ int wsum[4];
+    const R *__restrict__ U = reinterpret_cast<const R *>(A.U);
+    const R *__restrict__ X = reinterpret_cast<const R *>(A.X);
+    const int64_t n = A.n, first = (int64_t) xcd_block(A.n_xcd) * LP;
+    if (first >= n) return;                      // whole workgroup exits together
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+
+    // the list, by direction and leaf: leaf + LP direction | subface << 8
+    int nsub = 0;
+    if (tid < NF && first + tid % LP < n) {
+        const int nb = A.nbr[6 * (first + tid % LP) + tid / LP];
+        nsub = nb >= 0 ? 1 : (nb <= -kNbrAuxBase ? 4 : 0);
+    }
+    const uint64_t m1 = __ballot(nsub > 0), m4 = __ballot(nsub == 4), below = ((uint64_t) 1 << lane) - 1;
+    int at = __popcll(m1 & below) + 3 * __popcll(m4 & below);
+    if (lane == 0) wsum[wv] = __popcll(m1) + 3 * __popcll(m4);
+    __syncthreads();
+    #pragma unroll
+    for (int w = 0; w < 4; w++) at += w < wv ? wsum[w] : 0;
+    const int items = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+    if (tid < NF) {
+        base[tid] = (uint16_t) at;
+        for (int j = 0; j < nsub; j++) list[at + j] = (uint16_t) (tid | j << 8);
+    }
+    if (tid == 0) base[NF] = (uint16_t) items;
+    __syncthreads();
+
+    // groups of 64: the volume points first, then the (sub)faces
+    for (int g = wv; g <= (items + 63) / 64; g += 4) {
+        if (g == 0) {
+            const int64_t e = first + lane % LP;
+            if (e >= n) continue;
+            const int lev = A.level[e];
+            R u[4 * NV], w[4 * NV], ub[4 * NV];
+            load_coeffs<R, NV>(U, n, (int) e, u);
+            adj_weights<R, NV>(A, P, X, (int) e, w);
+            #pragma unroll
+            for (int i = 0; i < 4 * NV; i++) ub[i] = R(0);
+            const int part = lane / LP;
+            adj_volume<R, NC>(P, u, w, ldexp(R(1), -lev), ldexp(R(1), lev), ub, part * (8 / VP), (part + 1) * (8 / VP));
+            #pragma unroll
+            for (int i = 0; i < 4 * NV; i++) vol[64 * i + lane] = ub[i];
+            continue;
+        }
+        const int it = 64 * (g - 1) + lane;
+        if (it >= items) continue;
+        const int code = list[it], t = code & 255, j = code >> 8;
+        const int64_t e = first + t % LP;
+        const int d = t / LP, a = d >> 1, t1 = (a == 0) ? 1 : 0, t2 = (a == 2) ? 1 : 2;
+        const bool up = d & 1;                   // the leaf is side 0, the normal +e_a
+        const int nb = A.nbr[6 * e + d], lev = A.level[e];
+        const bool split = nb < 0;
+        int q = nb;
+        // the leaf's part (o1, o2, m) of a split face, the neighbour's (b1, b2, bm) where it is the larger
+        R o1 = R(0), o2 = R(0), m = R(1), b1 = R(0), b2 = R(0), bm = R(1);
+        if (split) {
+            const int4 grp = A.aux[-kNbrAuxBase - nb];
+            q = j == 0 ? grp.x : (j == 1 ? grp.y : (j == 2 ? grp.z : grp.w));
+            o1 = (j & 1) ? R(0.25) : R(-0.25);
+            o2 = (j & 2) ? R(0.25) : R(-0.25);
+            m = R(0.5);
+        } else if (A.level[nb] != lev) {
+            const int4 og = A.aux[-kNbrAuxBase - A.nbr[6 * (int64_t) nb + (d ^ 1)]];
+            const int s = (og.x == e) ? 0 : ((og.y == e) ? 1 : ((og.z == e) ? 2 : 3));
+            b1 = (s & 1) ? R(0.25) : R(-0.25);
+            b2 = (s & 2) ? R(0.25) : R(-0.25);
+            bm = R(0.5);
+        }
+        // weights (adj_weights) times wJ, the leaf's sign in side 0 less side 1
+        const R h = ldexp(split ? R(0.5) : R(1), -lev);
+        const R wj = (up ? R(1) : R(-1)) * h * h * R(1.0 / 6.0) * R(-A.dt) * R(A.c_in);
+        const R fe = wj * ldexp(R(1), 3 * lev), fq = -wj * ldexp(R(1), 3 * (int) A.level[q]);
+        const R a0 = cst<R>(P.ainv0[0], P.ainv0_f[0]), ax = cst<R>(P.ainv0[1], P.ainv0_f[1]);
+        const R ay = cst<R>(P.ainv0[2], P.ainv0_f[2]), az = cst<R>(P.ainv0[3], P.ainv0_f[3]);
+        const R aa = sel(a == 0, ax, sel(a == 1, ay, az)), ab = sel(a == 0, ay, ax), ac = sel(a == 2, ay, az);
+        const R pn = up ? R(0.5) : R(-0.5);
+        R L0[NV], L1[NV], L2[NV], R0[NV], R1[NV], R2[NV], G0[NV], G1[NV], G2[NV];
+        #pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const int gv = v == 0 ? a : (v == 1 ? t1 : (v == 2 ? t2 : v));
+            const R *ul = U + (int64_t) 4 * gv * n, *xl = X + (int64_t) 4 * gv * n;
+            trace_plane<R>(ul + (up ? e : q), n, a, t1, t2, R(0.5), up ? o1 : b1, up ? o2 : b2, up ? m : bm,
+                           L0[v], L1[v], L2[v]);
+            trace_plane<R>(ul + (up ? q : e), n, a, t1, t2, R(-0.5), up ? b1 : o1, up ? b2 : o2, up ? bm : m,
+                           R0[v], R1[v], R2[v]);
+            const R *we = xl + e, *wq = xl + q;
+            const R e1 = ab * fe * we[(1 + t1) * n], e2 = ac * fe * we[(1 + t2) * n];
+            const R q1 = ab * fq * wq[(1 + t1) * n], q2 = ac * fq * wq[(1 + t2) * n];
+            G0[v] = a0 * (fe * we[0] + fq * wq[0]) + pn * aa * (fe * we[(1 + a) * n] - fq * wq[(1 + a) * n]) +
+                    o1 * e1 + o2 * e2 + b1 * q1 + b2 * q2;
+            G1[v] = m * e1 + bm * q1;
+            G2[v] = m * e2 + bm * q2;
+        }
+        R S[3][NV];
+        #pragma unroll
+        for (int v = 0; v < NV; v++) S[0][v] = S[1][v] = S[2][v] = R(0);
+        #pragma unroll 1
+        for (int k = 0; k < 6; k++) {
+            const R g1 = gp_t1<R>(k), g2 = gp_t2<R>(k);
+            R tL[NV], tR[NV], qb[NV];
+            #pragma unroll
+            for (int v = 0; v < NV; v++) {
+                tL[v] = L0[v] + g1 * L1[v] + g2 * L2[v];
+                tR[v] = R0[v] + g1 * R1[v] + g2 * R2[v];
+                qb[v] = G0[v] + g1 * G1[v] + g2 * G2[v];
+            }
+            Prim<R, NC> pL, pR;
+            cons_to_prim<R, NC>(P, tL, pL);
+            cons_to_prim<R, NC>(P, tR, pR);
+            Frame<R, NC> fL, fR;
+            frame_of<R, NC>(pL, 0, fL);          // (the traces are in the face frame)
+            frame_of<R, NC>(pR, 0, fR);
+            FrameBar<R, NC> fb0, fb1;
+            zero_bar<R, NC>(fb0);
+            zero_bar<R, NC>(fb1);
+            flux_vjp<R, NC, FLUX>(fL, fR, qb, fb0, fb1);
+            // the leaf's side
+            PrimBar<R, NC> pb, pb1;
+            prim_bar_of<R, NC>(fb0, 0, pb);
+            prim_bar_of<R, NC>(fb1, 0, pb1);
+            pb.r = sel(up, pb.r, pb1.r); pb.u = sel(up, pb.u, pb1.u); pb.v = sel(up, pb.v, pb1.v);
+            pb.w = sel(up, pb.w, pb1.w); pb.e_tot = sel(up, pb.e_tot, pb1.e_tot); pb.p = sel(up, pb.p, pb1.p);
+            pb.cz = sel(up, pb.cz, pb1.cz); pb.gam = sel(up, pb.gam, pb1.gam);
+            Prim<R, NC> ps;
+            ps.r = sel(up, pL.r, pR.r); ps.u = sel(up, pL.u, pR.u); ps.v = sel(up, pL.v, pR.v);
+            ps.w = sel(up, pL.w, pR.w); ps.e = sel(up, pL.e, pR.e); ps.p = sel(up, pL.p, pR.p);
+            ps.cz = sel(up, pL.cz, pR.cz); ps.gam = sel(up, pL.gam, pR.gam);
+            #pragma unroll
+            for (int i = 0; i < NC; i++) { pb.c[i] = sel(up, pb.c[i], pb1.c[i]); ps.c[i] = sel(up, pL.c[i], pR.c[i]); }
+            R tb[NV];
+            #pragma unroll
+            for (int v = 0; v < NV; v++) tL[v] = sel(up, tL[v], tR[v]);
+            cons_to_prim_vjp<R, NC>(P, tL, ps, pb, tb);
+            #pragma unroll
+            for (int v = 0; v < NV; v++) { S[0][v] += tb[v]; S[1][v] += tb[v] * g1; S[2][v] += tb[v] * g2; }
+        }
+        R *to = mom + (size_t) it * 3 * NV;
+        #pragma unroll
+        for (int k = 0; k < 3; k++)
+            #pragma unroll
+            for (int v = 0; v < NV; v++) to[k * NV + v] = S[k][v];
+    }
+    __syncthreads();
+
+    // not __restrict__: the last stage adjoint accumulates into its own output
+    R *out = reinterpret_cast<R *>(A.OUT);
+    const R *acc = reinterpret_cast<const R *>(A.ACC);
+    const R *acc2 = reinterpret_cast<const R *>(A.ACC2);
+    for (int o = tid; o < 4 * NV * LP; o += 256) {
+        const int l = o % LP, i = o / LP, v = i >> 2, k = i & 3;
+        const int64_t e = first + l;
+        if (e >= n) continue;
+        R ub = R(0);
+        #pragma unroll
+        for (int s = 0; s < VP; s++) ub += vol[64 * i + s * LP + l];
+        for (int d = 0; d < 6; d++) {
+            const int b0 = base[d * LP + l], cnt = base[d * LP + l + 1] - b0;
+            const int a = d >> 1, t1 = (a == 0) ? 1 : 0;
+            const int vf = v > 2 ? v : (v == a ? 0 : (v == t1 ? 1 : 2));
+            for (int j = 0; j < cnt; j++) {
+                const R *from = mom + (size_t) (b0 + j) * 3 * NV + vf;
+                const R s0 = from[0];
+                if (k == 0) ub += s0;
+                else if (k - 1 == a) ub += ((d & 1) ? R(0.5) : R(-0.5)) * s0;
+                else {
+                    const bool first_t = k - 1 == t1;
+                    const R m = cnt == 4 ? R(0.5) : R(1);
+                    const R off = cnt == 4 ? ((j & (first_t ? 1 : 2)) ? R(0.25) : R(-0.25)) : R(0);
+                    ub += off * s0 + m * from[first_t ? NV : 2 * NV];
+                }
+            }
+        }
+        const int bi = A.bnd_of ? A.bnd_of[e] : -1;
+        if (bi >= 0) {
+            const R *__restrict__ bp = reinterpret_cast<const R *>(A.bnd_part);
+            double th = 0.0;
+            for (int p = 6 * A.bnd_ptr[bi]; p < 6 * A.bnd_ptr[bi + 1]; p++) {
+                ub += bp[(size_t) p * 4 * NV + i];
+                if (A.theta_bar && i < 3) th += A.bnd_theta[3 * (size_t) p + i];
+            }
+            if (A.theta_bar && i < 3) A.theta_bar[3 * e + i] += th;
+        }
+        const R sb = R(A.c_in) * (X + i * n)[e];
+        R r = R(A.c_out) * (sb + ub);
+        if (acc) r += R(A.c_acc) * (acc + i * n)[e];
+        if (acc2) r += R(A.c_acc2) * (acc2 + i * n)[e];
+        (out + i * n)[e] = r;
+    }
+}
+
 // One interior face of a chunk, both sides at once: at each of the six
 // points one primal evaluation and one reverse sweep of
 //   s = wJ sum_v q_v(t0, t1) (w0_v(p0) - w1_v(p1))
@@ -285,32 +501,50 @@ void k_adj_stage(AdjArgs A, DevParams P)
 // the adjoint weights of side s at its point) give d s / d t0 and d s / d t1;
 // out[side][m][v] = sum over the points of (d s / d t_side)_v g_m,
 // g = (1, t1 coordinate, t2 coordinate) of the small face's point.
-// The face's normal axis AX is a template argument, so that every
-// coefficient and velocity component is picked at compile time.
-template <typename R, int NC, int FLUX, int AX>
+// One path for the three axes, the traces loaded in the face frame by address
+// (with the axis a template argument a wave that holds faces of two axes ran
+// both versions: 64 us a stage adjoint at 32,768 leaves, 52 so; 73 and 43 at
+// 4,096).  The variables of out are in the face frame's order.
+template <typename R, int NC, int FLUX>
 __device__ __forceinline__ void adj_face(const AdjArgs &A, const DevParams &P, const R *__restrict__ U,
                                          const R *__restrict__ X, int4 rec, R *out)
 {
     constexpr int NV = 4 + NC;
-    constexpr int a = AX, t1 = (AX == 0) ? 1 : 0, t2 = (AX == 2) ? 1 : 2;
     const int64_t n = A.n;
     const int info = rec.z;
     const int dir0 = info & 7, kind = (info >> 3) & 3, sub = (info >> 5) & 3;
+    const int a = dir0 >> 1, t1 = (a == 0) ? 1 : 0, t2 = (a == 2) ? 1 : 2;
     const R s = (dir0 & 1) ? R(1) : R(-1);
-    const int lown = A.level[rec.x] + (kind == FACE_HANG1 ? 1 : 0);
-    const R h = ldexp(R(1), -lown);
-    const R wj = h * h * R(1.0 / 6.0);
+    const int lev0 = A.level[rec.x], lev1 = A.level[rec.y];
+    const R h = ldexp(R(1), -(lev0 + (kind == FACE_HANG1 ? 1 : 0)));
+    const R wj = h * h * R(1.0 / 6.0) * R(-A.dt) * R(A.c_in);
     const R pa0 = R(0.5) * s, pa1 = -pa0;
     const R d1 = (sub & 1) ? R(0.25) : R(-0.25), d2 = (sub & 2) ? R(0.25) : R(-0.25);
     const bool big0 = kind == FACE_HANG1, big1 = kind == FACE_HANG0;
     const R m0 = big0 ? R(0.5) : R(1), m1 = big1 ? R(0.5) : R(1);
     const R o01 = big0 ? d1 : R(0), o02 = big0 ? d2 : R(0);
     const R o11 = big1 ? d1 : R(0), o12 = big1 ? d2 : R(0);
-    R u0[4 * NV], u1[4 * NV], w0[4 * NV], w1[4 * NV];
-    load_coeffs<R, NV>(U, n, rec.x, u0);
-    load_coeffs<R, NV>(U, n, rec.y, u1);
-    adj_weights<R, NV>(A, P, X, rec.x, w0);
-    adj_weights<R, NV>(A, P, X, rec.y, w1);
+    const R f0 = wj * ldexp(R(1), 3 * lev0), f1 = -wj * ldexp(R(1), 3 * lev1);
+    const R i0 = cst<R>(P.ainv0[0], P.ainv0_f[0]), ix = cst<R>(P.ainv0[1], P.ainv0_f[1]);
+    const R iy = cst<R>(P.ainv0[2], P.ainv0_f[2]), iz = cst<R>(P.ainv0[3], P.ainv0_f[3]);
+    const R ia = sel(a == 0, ix, sel(a == 1, iy, iz)), i1 = sel(a == 0, iy, ix), i2 = sel(a == 2, iy, iz);
+    R L0[NV], L1[NV], L2[NV], R0[NV], R1[NV], R2[NV], G0[NV], G1[NV], G2[NV];
+    #pragma unroll
+    for (int v = 0; v < NV; v++) {
+        const int gv = v == 0 ? a : (v == 1 ? t1 : (v == 2 ? t2 : v));
+        const R *u = U + (int64_t) 4 * gv * n, *x = X + (int64_t) 4 * gv * n;
+        trace_plane<R>(u + rec.x, n, a, t1, t2, pa0, o01, o02, m0, L0[v], L1[v], L2[v]);
+        trace_plane<R>(u + rec.y, n, a, t1, t2, pa1, o11, o12, m1, R0[v], R1[v], R2[v]);
+        const R *x0 = x + rec.x, *x1 = x + rec.y;
+        const R e1 = i1 * f0 * x0[(1 + t1) * n], e2 = i2 * f0 * x0[(1 + t2) * n];
+        const R q1 = i1 * f1 * x1[(1 + t1) * n], q2 = i2 * f1 * x1[(1 + t2) * n];
+        // component 0 along s e_a: the flux's normal momentum
+        const R sg = v == 0 ? s : R(1);
+        G0[v] = sg * (i0 * (f0 * x0[0] + f1 * x1[0]) + pa0 * ia * (f0 * x0[(1 + a) * n] - f1 * x1[(1 + a) * n]) +
+                      o01 * e1 + o02 * e2 + o11 * q1 + o12 * q2);
+        G1[v] = sg * (m0 * e1 + m1 * q1);
+        G2[v] = sg * (m0 * e2 + m1 * q2);
+    }
     R M0[3][NV], M1[3][NV];
     #pragma unroll
     for (int m = 0; m < 3; m++)
@@ -319,28 +553,20 @@ __device__ __forceinline__ void adj_face(const AdjArgs &A, const DevParams &P, c
     #pragma unroll 1
     for (int k = 0; k < 6; k++) {
         const R g1 = gp_t1<R>(k), g2 = gp_t2<R>(k);
-        const R q01 = o01 + m0 * g1, q02 = o02 + m0 * g2;     // side 0 tangential coordinates
-        const R q11 = o11 + m1 * g1, q12 = o12 + m1 * g2;     // side 1
-        R tL[NV], tR[NV], G[NV];
+        R tL[NV], tR[NV], qb[NV];
         #pragma unroll
         for (int v = 0; v < NV; v++) {
-            tL[v] = u0[4*v] + pa0 * u0[4*v+1+a] + q01 * u0[4*v+1+t1] + q02 * u0[4*v+1+t2];
-            tR[v] = u1[4*v] + pa1 * u1[4*v+1+a] + q11 * u1[4*v+1+t1] + q12 * u1[4*v+1+t2];
-            const R wl = w0[4*v] + pa0 * w0[4*v+1+a] + q01 * w0[4*v+1+t1] + q02 * w0[4*v+1+t2];
-            const R wr = w1[4*v] + pa1 * w1[4*v+1+a] + q11 * w1[4*v+1+t1] + q12 * w1[4*v+1+t2];
-            G[v] = wj * (wl - wr);
+            tL[v] = L0[v] + g1 * L1[v] + g2 * L2[v];
+            tR[v] = R0[v] + g1 * R1[v] + g2 * R2[v];
+            qb[v] = G0[v] + g1 * G1[v] + g2 * G2[v];
         }
         Prim<R, NC> pL, pR;
         cons_to_prim<R, NC>(P, tL, pL);
         cons_to_prim<R, NC>(P, tR, pR);
         Frame<R, NC> fL, fR;
-        frame_of<R, NC>(pL, a, fL);
-        frame_of<R, NC>(pR, a, fR);
+        frame_of<R, NC>(pL, 0, fL);              // (the traces are in the face frame)
+        frame_of<R, NC>(pR, 0, fR);
         fL.un *= s; fR.un *= s;
-        R qb[NV];
-        qb[0] = s * G[a]; qb[1] = G[t1]; qb[2] = G[t2];
-        #pragma unroll
-        for (int v = 3; v < NV; v++) qb[v] = G[v];
         FrameBar<R, NC> b0, b1;
         zero_bar<R, NC>(b0);
         zero_bar<R, NC>(b1);
@@ -348,11 +574,11 @@ __device__ __forceinline__ void adj_face(const AdjArgs &A, const DevParams &P, c
         b0.un *= s; b1.un *= s;
         PrimBar<R, NC> pb;
         R tb[NV];
-        prim_bar_of<R, NC>(b0, a, pb);
+        prim_bar_of<R, NC>(b0, 0, pb);
         cons_to_prim_vjp<R, NC>(P, tL, pL, pb, tb);
         #pragma unroll
         for (int v = 0; v < NV; v++) { M0[0][v] += tb[v]; M0[1][v] += tb[v] * g1; M0[2][v] += tb[v] * g2; }
-        prim_bar_of<R, NC>(b1, a, pb);
+        prim_bar_of<R, NC>(b1, 0, pb);
         cons_to_prim_vjp<R, NC>(P, tR, pR, pb, tb);
         #pragma unroll
         for (int v = 0; v < NV; v++) { M1[0][v] += tb[v]; M1[1][v] += tb[v] * g1; M1[2][v] += tb[v] * g2; }
@@ -390,12 +616,7 @@ void k_adj_chunk(AdjArgs A, DevParams P)
     for (int f = fb + (int) threadIdx.x; f < fe; f += BS) {
         const int4 rec = A.cf4[f];
         if (((rec.z >> 3) & 3) != FACE_BND) {
-            // faces of a chunk are sorted by axis, so the branch is mostly wave-uniform
-            R *dst = mom + (size_t) (f - fb) * 6 * NV;
-            const int ax = (rec.z & 7) >> 1;
-            if (ax == 0) adj_face<R, NC, FLUX, 0>(A, P, U, X, rec, dst);
-            else if (ax == 1) adj_face<R, NC, FLUX, 1>(A, P, U, X, rec, dst);
-            else adj_face<R, NC, FLUX, 2>(A, P, U, X, rec, dst);
+            adj_face<R, NC, FLUX>(A, P, U, X, rec, mom + (size_t) (f - fb) * 6 * NV);
         }
         finfo[f - fb] = rec.z;
     }
@@ -427,7 +648,9 @@ void k_adj_chunk(AdjArgs A, DevParams P)
         const R *m = mom + (size_t) fl * 6 * NV + (size_t) side * 3 * NV;
         #pragma unroll
         for (int v = 0; v < NV; v++) {
-            const R S0 = m[v], S1 = m[NV + v], S2 = m[2 * NV + v];
+            // the variable in the face frame's order
+            const int vf = v > 2 ? v : (v == ax ? 0 : (v == (ax == 0 ? 1 : 0) ? 1 : 2));
+            const R S0 = m[vf], S1 = m[NV + vf], S2 = m[2 * NV + vf];
             // (normal, t1, t2) parts spread onto (x, y, z)
             const R cn = pa * S0, c1 = mu * S1 + d1 * S0, c2 = mu * S2 + d2 * S0;
             ub[4*v+0] += S0;
@@ -473,8 +696,7 @@ void k_adj_chunk(AdjArgs A, DevParams P)
 // the point's contribution phi_k (d s / d t) to the leaf's coefficient
 // gradient (and, on the inlet face of the parameters, d s / d theta) is
 // written to its own slot of a scratch array, summed per leaf in a fixed
-// order by k_adj_bnd_sum (element-centric path) or by phase 2 of
-// k_adj_chunk.
+// order by k_adj_leaves or by phase 2 of k_adj_chunk.
 template <typename R, int NC, int FLUX>
 __global__ __launch_bounds__(64)
 void k_adj_bnd_pts(AdjArgs A, DevParams P)
@@ -539,40 +761,6 @@ void k_adj_bnd_pts(AdjArgs A, DevParams P)
     }
 }
 
-// per boundary leaf: OUT += c_out * (sum over its boundary faces and their
-// points, in list order), theta_bar += the same sum of the parameter parts
-template <typename R, int NV>
-__global__ __launch_bounds__(128)
-void k_adj_bnd_sum(AdjArgs A)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.n_bnd) return;
-    const int e = A.bnd_elems[i];
-    const int f0 = A.bnd_ptr[i], f1 = A.bnd_ptr[i + 1];
-    const R *__restrict__ part = reinterpret_cast<const R *>(A.bnd_part);
-    R acc[4 * NV];
-    #pragma unroll
-    for (int j = 0; j < 4 * NV; j++) acc[j] = R(0);
-    double th[3] = {0.0, 0.0, 0.0};
-    for (int p = 6 * f0; p < 6 * f1; p++) {
-        #pragma unroll
-        for (int j = 0; j < 4 * NV; j++) acc[j] += part[(size_t) p * 4 * NV + j];
-        if (A.theta_bar) {
-            #pragma unroll
-            for (int j = 0; j < 3; j++) th[j] += A.bnd_theta[3 * (size_t) p + j];
-        }
-    }
-    R *out = reinterpret_cast<R *>(A.OUT);
-    const int64_t n = A.n;
-    #pragma unroll
-    for (int j = 0; j < 4 * NV; j++) (out + j * n)[e] += R(A.c_out) * acc[j];
-    if (A.theta_bar) {
-        A.theta_bar[3 * e + 0] += th[0];
-        A.theta_bar[3 * e + 1] += th[1];
-        A.theta_bar[3 * e + 2] += th[2];
-    }
-}
-
 template <typename R, int NC>
 static hipError_t launch_adj_bnd_pts(int flux, const AdjArgs &A, const DevParams &P, hipStream_t st)
 {
@@ -583,19 +771,6 @@ static hipError_t launch_adj_bnd_pts(int flux, const AdjArgs &A, const DevParams
     case FLUX_HLLC: hipLaunchKernelGGL((k_adj_bnd_pts<R, NC, FLUX_HLLC>), gp, bp, 0, st, A, P); break;
     default: hipLaunchKernelGGL((k_adj_bnd_pts<R, NC, FLUX_CD>), gp, bp, 0, st, A, P); break;
     }
-    return hipGetLastError();
-}
-
-// element-centric path: boundary points after the interior kernel, then the
-// per-leaf sum into OUT
-template <typename R, int NC>
-static hipError_t launch_adj_bnd(int flux, const AdjArgs &A, const DevParams &P, hipStream_t st)
-{
-    if (A.n_bnd <= 0) return hipSuccess;
-    hipError_t err = launch_adj_bnd_pts<R, NC>(flux, A, P, st);
-    if (err != hipSuccess) return err;
-    const dim3 gs((unsigned) ((A.n_bnd + 127) / 128)), bs(128);
-    hipLaunchKernelGGL((k_adj_bnd_sum<R, 4 + NC>), gs, bs, 0, st, A);
     return hipGetLastError();
 }
 
@@ -681,30 +856,54 @@ static hipError_t launch_adj_chunk(const AdjArgs &A, const DevParams &P, hipStre
                                : launch_adj_chunk_bs<R, NC, FLUX, 128>(A, P, st);
 }
 
+template <typename R, int NC, int FLUX, int WG>
+static hipError_t launch_adj_leaves(const AdjArgs &A, const DevParams &P, hipStream_t st)
+{
+    const size_t sh = ((size_t) 4 * 64 + (size_t) 3 * A.max_items) * (4 + NC) * sizeof(R) + (size_t) A.max_items * sizeof(uint16_t);
+    const void *fn = reinterpret_cast<const void *>(&k_adj_leaves<R, NC, FLUX, WG>);
+    hipError_t err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int) sh);
+    if (err != hipSuccess) return err;
+    const int64_t blocks = (A.n + kAdjLeaves - 1) / kAdjLeaves;
+    const dim3 grid((unsigned) ((blocks + A.n_xcd - 1) / A.n_xcd * A.n_xcd)), block(256);
+    hipLaunchKernelGGL((k_adj_leaves<R, NC, FLUX, WG>), grid, block, sh, st, A, P);
+    return hipGetLastError();
+}
+
+// Stage adjoint with its boundary points and launch gaps, us, at 512 / 4,096 /
+// 9,192 (hanging) / 32,768 / 262,144 leaves, HLLC one species: FP32 by chunks 39
+// / 43 / 45 / 52 / 175, by leaves 35 / 34 / 40 / 59 / 305: leaves up to 12,000
+// (19,104: 52 both).  FP64 by leaves with one workgroup per CU and no spills 46
+// / 43 / 70 / 123 / 818, with two and 100 spilled registers 51 / 50 / 73 / 112 /
+// 717: two beyond 24,000 (40,328 hanging: 162 and 165).  One thread per leaf 118
+// / 118 / 506 / 125 / 439, 86,864 with hanging faces 493 against 281 by leaves:
+// it keeps the meshes without hanging faces beyond 65,536.
+template <typename R, int NC, int FLUX>
+static hipError_t launch_adj_flux(const AdjArgs &A, const DevParams &P, hipStream_t st)
+{
+    if constexpr (sizeof(R) == 4) {
+        if (A.cf4 && A.n > 12000) return launch_adj_chunk<R, NC, FLUX>(A, P, st);
+        return launch_adj_leaves<R, NC, FLUX, 2>(A, P, st);
+    } else {
+        if (A.n > 65536 && !A.hanging) {
+            const dim3 grid((unsigned) ((A.n + 127) / 128)), block(128);
+            hipLaunchKernelGGL((k_adj_stage<R, NC, FLUX>), grid, block, 0, st, A, P);
+            return hipGetLastError();
+        }
+        return A.n > 24000 ? launch_adj_leaves<R, NC, FLUX, 2>(A, P, st) : launch_adj_leaves<R, NC, FLUX, 1>(A, P, st);
+    }
+}
+
 template <typename R, int NC>
 static hipError_t launch_adj_nc(int flux, const AdjArgs &A, const DevParams &P, hipStream_t st)
 {
-    if (sizeof(R) == 4 && A.cf4) {
-        hipError_t err = launch_adj_bnd_pts<R, NC>(flux, A, P, st);
-        if (err != hipSuccess) return err;
-        switch (flux) {
-        case FLUX_LF: err = launch_adj_chunk<R, NC, FLUX_LF>(A, P, st); break;
-        case FLUX_HLLC: err = launch_adj_chunk<R, NC, FLUX_HLLC>(A, P, st); break;
-        case FLUX_CD: err = launch_adj_chunk<R, NC, FLUX_CD>(A, P, st); break;
-        default: return hipErrorInvalidValue;
-        }
-        return err;
-    }
-    const dim3 grid((unsigned) ((A.n + 127) / 128)), block(128);
-    switch (flux) {
-    case FLUX_LF: hipLaunchKernelGGL((k_adj_stage<R, NC, FLUX_LF>), grid, block, 0, st, A, P); break;
-    case FLUX_HLLC: hipLaunchKernelGGL((k_adj_stage<R, NC, FLUX_HLLC>), grid, block, 0, st, A, P); break;
-    case FLUX_CD: hipLaunchKernelGGL((k_adj_stage<R, NC, FLUX_CD>), grid, block, 0, st, A, P); break;
-    default: return hipErrorInvalidValue;
-    }
-    hipError_t err = hipGetLastError();
+    hipError_t err = launch_adj_bnd_pts<R, NC>(flux, A, P, st);
     if (err != hipSuccess) return err;
-    return launch_adj_bnd<R, NC>(flux, A, P, st);
+    switch (flux) {
+    case FLUX_LF: return launch_adj_flux<R, NC, FLUX_LF>(A, P, st);
+    case FLUX_HLLC: return launch_adj_flux<R, NC, FLUX_HLLC>(A, P, st);
+    case FLUX_CD: return launch_adj_flux<R, NC, FLUX_CD>(A, P, st);
+    }
+    return hipErrorInvalidValue;
 }
 
 template <typename R>

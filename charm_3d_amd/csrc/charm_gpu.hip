@@ -27,6 +27,7 @@ struct AdjBoundary {
     void *part;
     double *theta;
     int n_elems, n_faces;
+    int max_items;            // most interior (sub)faces of a workgroup of k_adj_leaves
 };
 
 constexpr int kXferParts = 8;              // streams of a large state transfer
@@ -1675,7 +1676,7 @@ static int adj_boundary(charm_gpu_ctx_t *c)
     }
     hipError_t e = hipMemcpyAsync(nbr, c->d_nbr, (size_t) n * 6 * sizeof(int), hipMemcpyDeviceToHost, c->st);
     if (e == hipSuccess) e = hipStreamSynchronize(c->st);
-    int ne = 0, nf = 0;
+    int ne = 0, nf = 0, items = 0;
     if (e == hipSuccess) {
         ptr[0] = 0;
         for (int64_t i = 0; i < n; i++) {
@@ -1683,6 +1684,9 @@ static int adj_boundary(charm_gpu_ctx_t *c)
             for (int d = 0; d < 6; d++)
                 if (nbr[6 * i + d] < 0 && nbr[6 * i + d] > -8) faces[nf++] = (int) (i * 8 + d);
             of[i] = -1;
+            if (i % kAdjLeaves == 0) items = 0;
+            for (int d = 0; d < 6; d++) items += nbr[6 * i + d] >= 0 ? 1 : (nbr[6 * i + d] <= -8 ? 4 : 0);
+            if (items > b.max_items) b.max_items = items;
             if (nf > f0) { of[i] = ne; elems[ne] = (int) i; ptr[++ne] = nf; }
         }
     }
@@ -1751,7 +1755,7 @@ extern "C" int charm_gpu_stage_vjp(charm_gpu_ctx_t *c, double dt, const double *
         A.ch_ebeg = c->d_ch_ebeg; A.ch_fbeg = c->d_ch_fbeg; A.slot_ptr = c->d_slot_ptr; A.slots = c->d_slots;
         A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems;
         A.n_xcd = c->n_xcd;
-        A.bnd_of = chunked ? bnd.of : NULL;
+        A.bnd_of = bnd.of; A.max_items = bnd.max_items; A.hanging = c->naux > 0;
         A.U = dU; A.X = dX; A.ACC = NULL; A.ACC2 = NULL; A.OUT = dO;
         A.c_in = 1.0; A.c_out = 1.0; A.c_acc = 0.0; A.c_acc2 = 0.0;
         e = launch_adj_stage(c->sprec, c->nc, c->cfg.flux, A, c->P, c->st);
@@ -1791,7 +1795,7 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
     if ((rc = adj_boundary(c))) return rc;
     const AdjBoundary &bnd = c->bnd;
     // FP32: the chunked face-centric stage adjoint when its LDS fits a
-    // workgroup (else, and in FP64, the element-centric one)
+    // workgroup (else, on small meshes and in FP64, the one by leaves)
     int dev = 0, lds_max = 0;
     const bool chunked = c->sprec && hipGetDevice(&dev) == hipSuccess &&
                          hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
@@ -1880,7 +1884,7 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
             A.ch_ebeg = c->d_ch_ebeg; A.ch_fbeg = c->d_ch_fbeg; A.slot_ptr = c->d_slot_ptr; A.slots = c->d_slots;
             A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems;
             A.n_xcd = c->n_xcd;
-            A.bnd_of = chunked ? bnd.of : NULL;
+            A.bnd_of = bnd.of; A.max_items = bnd.max_items; A.hanging = c->naux > 0;
             // l3 = S^T(2/3 l); l2 = S^T(1/4 l3); l = S^T(l2) + l / 3 + 3/4 l3
             A.U = u2; A.X = la; A.ACC = NULL; A.ACC2 = NULL; A.OUT = lb;
             A.c_in = 2.0 / 3.0; A.c_out = 1.0; A.c_acc = 0.0; A.c_acc2 = 0.0;

@@ -140,6 +140,7 @@ struct NsArgs {
 // adjoint of one SSP-RK stage (one thread per leaf):
 // OUT = c_out (sb + (d int / d U)^T W) + c_acc ACC + c_acc2 ACC2,  sb = c_in X,
 // W = -dt A^-1 sb
+constexpr int kAdjLeaves = 32;   // leaves of a workgroup of k_adj_leaves
 struct AdjArgs {
     const void *U, *X, *ACC, *ACC2;
     void *OUT;
@@ -157,7 +158,7 @@ struct AdjArgs {
     void *bnd_part;           // [n_bface][6][4 V] point contributions (state type)
     double *bnd_theta;        // [n_bface][6][3] parameter contributions
     // chunked face-centric variant (chunks as for the stage kernel; null
-    // cf4: the element-centric kernel)
+    // cf4: the kernel by leaves)
     const int4 *cf4;
     const int *ch_ebeg, *ch_fbeg, *slot_ptr;
     const uint16_t *slots;
@@ -165,6 +166,8 @@ struct AdjArgs {
     // chunked variant: per leaf its index in bnd_elems (or -1); the chunk
     // kernel then adds the boundary parts itself (k_adj_bnd_pts runs first)
     const int *bnd_of;
+    int max_items;            // kernel by leaves: most interior (sub)faces of a workgroup
+    int hanging;              // the mesh has hanging faces
 };
 
 // objective over a box of leaves: mode 0 per-block partial sums of
