@@ -1146,23 +1146,44 @@ static void cut_range(void *arg, int64_t lo, int64_t hi, int part)
  * slot order, so the sums of a leaf run as in the chunk. */
 int charm_mesh_cut(const charm_mesh_t *m, int max_e, int max_f, charm_pieces_t *out)
 {
+    charm_cut_buf_t b;
+    int rc;
+    memset(&b, 0, sizeof(b));
+    rc = charm_mesh_cut_buf(m, max_e, max_f, &b);
+    *out = b.p;
+    return rc;
+}
+
+void charm_cut_buf_free(charm_cut_buf_t *b)
+{
+    charm_pieces_free(&b->p);
+    b->cap_n = b->cap_s = 0;
+}
+
+int charm_mesh_cut_buf(const charm_mesh_t *m, int max_e, int max_f, charm_cut_buf_t *buf)
+{
+    charm_pieces_t *out = &buf->p;
     cut_job_t J;
     int64_t i;
     int p, parts = par_parts(m->n, 8192);
     if (parts > 8) parts = 8;
     if (parts > m->nch) parts = m->nch > 0 ? (int) m->nch : 1;
-    memset(out, 0, sizeof(*out));
     J.m = m; J.out = out; J.max_e = max_e; J.max_f = max_f;
     J.bits = (uint64_t *) malloc((size_t) parts * (m->chunk_faces / 64 + 1) * sizeof(uint64_t));
     J.rank = (int32_t *) malloc((size_t) parts * (m->chunk_faces + 1) * sizeof(int32_t));
-    out->ch_ebeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
-    out->ch_fbeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
-    out->ch_ref = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
-    out->cf4 = (int32_t *) malloc((size_t) (m->nslot + 1) * 4 * sizeof(int32_t));
-    out->slots = (uint16_t *) malloc((size_t) (m->nslot + 1) * sizeof(uint16_t));
+    if (buf->cap_n < m->n || buf->cap_s < m->nslot) {
+        charm_cut_buf_free(buf);
+        out->ch_ebeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+        out->ch_fbeg = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+        out->ch_ref = (int32_t *) malloc((size_t) (m->n + 1) * sizeof(int32_t));
+        out->cf4 = (int32_t *) malloc((size_t) (m->nslot + 1) * 4 * sizeof(int32_t));
+        out->slots = (uint16_t *) malloc((size_t) (m->nslot + 1) * sizeof(uint16_t));
+        buf->cap_n = m->n; buf->cap_s = m->nslot;
+    }
+    out->nch = out->ncf = 0;
     if (!J.bits || !J.rank || !out->ch_ebeg || !out->ch_fbeg || !out->ch_ref || !out->cf4 || !out->slots) {
         free(J.bits); free(J.rank);
-        charm_pieces_free(out);
+        charm_cut_buf_free(buf);
         charm_set_error("mesh_cut: out of memory");
         return CHARM_ERR_MEM;
     }

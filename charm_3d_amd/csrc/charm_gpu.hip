@@ -91,6 +91,7 @@ struct charm_gpu_ctx {
     hipStream_t xst[kXferParts];
     AdjBoundary bnd;          // of the mesh, built by the first adjoint call on it
     int bnd_ok;
+    charm_cut_buf_t cut;      // host buffers of the piece cut (meshes of at most 49,152 leaves)
     // device blocks in use, and freed ones kept for the next request (mem_mu)
     struct Block { void *p; size_t bytes; } live[kLiveBlocks], idle[kIdleBlocks];
     int n_live, n_idle;
@@ -370,6 +371,7 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
     if (c->st) (void) hipStreamSynchronize(c->st);
     free_mesh(c);
     idle_release(c);
+    charm_cut_buf_free(&c->cut);
     if (c->h_pin) (void) hipHostFree(c->h_pin);
     for (int i = 0; i < kXferParts; i++)
         if (c->xst[i]) (void) hipStreamDestroy(c->xst[i]);
@@ -404,16 +406,16 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
 //     4,096 leaves FP32 21 -> 11, four species 64 -> 47;
 //   up to 12,000 (exact Riemann solver: 24,000), pieces of 16 on k_stage_pt:
 //     9,192 leaves FP64 37 -> 27, exact solver 54 -> 22;
-//   else, one to three species of constant cp: FP32 up to 65,536 pieces of 64
+//   else, one to three species of constant cp: FP32 up to 49,152 pieces of 64
 //     on 256 threads (40,328 leaves 32 -> 25, exact solver 59 -> 44; 86,864
-//     37 -> 36), FP64 up to 24,000 pieces of 48 (19,104 leaves 37 -> 30;
+//     37 -> 36, and the cut adds 0.45 ms to an upload of 53,768), FP64 up to 24,000 pieces of 48 (19,104 leaves 37 -> 30;
 //     at 32,768 the pieces lose, 34 -> 40).
 // A viscous or real-gas mesh beyond the point kernel's sizes stays uncut (104
 // and 105 at 32,768 leaves).
 struct Pieces {
     charm_pieces_t p;
     int rc, cut, points;
-    Pieces(const charm_gpu_ctx_t *c, const charm_mesh_t *m) : rc(CHARM_OK), cut(0), points(0)
+    Pieces(charm_gpu_ctx_t *c, const charm_mesh_t *m) : rc(CHARM_OK), cut(0), points(0)
     {
         const bool fp64 = c->prec == CHARM_FP64;
         int e = 0, f = 0;
@@ -421,16 +423,19 @@ struct Pieces {
         else if (m->n <= 12000 || (m->n <= 24000 && c->cfg.flux == CHARM_FLUX_GODUNOV)) { e = 16; f = 80; points = 1; }
         if (points && stage_points_smem_bytes(c->prec, c->nc, f, e) > 65536) { e = f = points = 0; }
         if (!points && !c->ph) {
-            if (!fp64 && m->n <= 65536) { e = 64; f = 256; }
+            if (!fp64 && m->n <= 49152) { e = 64; f = 256; }
             if (fp64 && m->n <= 24000) { e = 48; f = 192; }
         }
         cut = e && (m->chunk_elems > e || m->chunk_faces > f);
         memset(&p, 0, sizeof(p));
-        if (cut) { rc = charm_mesh_cut(m, e, f, &p); return; }
+        if (cut) {
+            rc = charm_mesh_cut_buf(m, e, f, &c->cut);
+            p = c->cut.p;
+            return;
+        }
         p.nch = m->nch; p.ncf = m->ncf;
         p.ch_ebeg = m->ch_ebeg; p.ch_fbeg = m->ch_fbeg; p.ch_ref = m->ch_ebeg; p.cf4 = m->cf4; p.slots = m->slots;
     }
-    ~Pieces() { if (cut) charm_pieces_free(&p); }
 };
 
 // the mesh arrays and state buffers that the pieces do not change

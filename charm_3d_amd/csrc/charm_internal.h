@@ -69,6 +69,14 @@ typedef struct {
 } charm_pieces_t;
 int  charm_mesh_cut(const charm_mesh_t *m, int max_e, int max_f, charm_pieces_t *out);
 void charm_pieces_free(charm_pieces_t *p);
+/* the same into buffers kept from cut to cut: their pages, first touched anew,
+ * cost as much as the cut itself (7 MB at 40,000 leaves) */
+typedef struct {
+    charm_pieces_t p;
+    int64_t cap_n, cap_s;
+} charm_cut_buf_t;
+int  charm_mesh_cut_buf(const charm_mesh_t *m, int max_e, int max_f, charm_cut_buf_t *b);
+void charm_cut_buf_free(charm_cut_buf_t *b);
 
 /* the forest's user pointer (the reference's charm_ctx_t) */
 struct charm_ctx {
