@@ -87,8 +87,8 @@ struct charm_gpu_ctx {
     int *d_err;
     // host side of the calls
     int dev;                  // the device of the context
+    int pooled;               // holds a reference to the transfer streams
     char *h_pin, *d_pin;      // pinned, mapped: flag, results, kPinBytes of small transfers (pin_mu)
-    hipStream_t xst[kXferParts];
     AdjBoundary bnd;          // of the mesh, built by the first adjoint call on it
     int bnd_ok;
     charm_cut_buf_t cut;      // host buffers of the piece cut (meshes of at most 49,152 leaves)
@@ -106,6 +106,62 @@ struct Lock {
     ~Lock() { pthread_mutex_unlock(m); }
 };
 } // namespace
+
+// The streams of large transfers, kXferParts on each of up to eight devices,
+// shared by the contexts of the process: a stream's first copy of pageable
+// memory makes the runtime's staging for it, which cost a new context with
+// streams of its own 2-3 ms.  One transfer at a time holds a device's streams
+// (another one meanwhile takes its context's own stream); the last context
+// gives them back.
+struct XferStreams {
+    hipStream_t s[kXferParts];
+    int dev, n, busy;
+};
+static struct {
+    pthread_mutex_t mu;
+    int refs, n;
+    XferStreams d[8];
+} xfer_pool = {PTHREAD_MUTEX_INITIALIZER, 0, 0, {}};
+
+static void xfer_pool_ref(int by)
+{
+    Lock lock(&xfer_pool.mu);
+    xfer_pool.refs += by;
+    if (xfer_pool.refs > 0) return;
+    for (int i = 0; i < xfer_pool.n; i++)
+        for (int k = 0; k < xfer_pool.d[i].n; k++) (void) hipStreamDestroy(xfer_pool.d[i].s[k]);
+    xfer_pool.n = 0;
+}
+
+// the streams of a device, at least two and up to `want`, or NULL
+static XferStreams *xfer_acquire(int dev, int want)
+{
+    Lock lock(&xfer_pool.mu);
+    XferStreams *x = NULL;
+    for (int i = 0; i < xfer_pool.n; i++)
+        if (xfer_pool.d[i].dev == dev) x = &xfer_pool.d[i];
+    if (!x) {
+        if (xfer_pool.n == (int) (sizeof(xfer_pool.d) / sizeof(xfer_pool.d[0]))) return NULL;
+        x = &xfer_pool.d[xfer_pool.n++];
+        x->dev = dev;
+        x->n = x->busy = 0;
+    }
+    if (x->busy) return NULL;
+    int cur = dev;
+    if (hipGetDevice(&cur) != hipSuccess || (cur != dev && hipSetDevice(dev) != hipSuccess)) { (void) hipGetLastError(); return NULL; }
+    while (x->n < want && hipStreamCreate(&x->s[x->n]) == hipSuccess) x->n++;
+    if (x->n < want) (void) hipGetLastError();
+    if (cur != dev) (void) hipSetDevice(cur);
+    if (x->n < 2) return NULL;
+    x->busy = 1;
+    return x;
+}
+
+static void xfer_release(XferStreams *x)
+{
+    Lock lock(&xfer_pool.mu);
+    x->busy = 0;
+}
 
 // Device memory of a context.  A freed block is kept, up to kIdleBytes in
 // all, and serves the next request that fills at least half of it: a remesh
@@ -359,6 +415,8 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
     // the kernels' error flag and the reductions' results are written to host
     // memory: read after a synchronisation, without a copy (8 us each)
     memset(c->h_pin, 0, kPinHead);
+    xfer_pool_ref(1);
+    c->pooled = 1;
     c->d_err = (int *) c->d_pin;
     c->d_result = (double *) (c->d_pin + 64);
     *out = c;
@@ -373,8 +431,7 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
     idle_release(c);
     charm_cut_buf_free(&c->cut);
     if (c->h_pin) (void) hipHostFree(c->h_pin);
-    for (int i = 0; i < kXferParts; i++)
-        if (c->xst[i]) (void) hipStreamDestroy(c->xst[i]);
+    if (c->pooled) xfer_pool_ref(-1);
     if (c->d_P) (void) hipFree(c->d_P);
     if (c->ev0) (void) hipEventDestroy(c->ev0);
     if (c->ev1) (void) hipEventDestroy(c->ev1);
@@ -646,6 +703,7 @@ struct Xfer {
     void *dst;
     const double *in;
     double *out;
+    XferStreams *streams;
     hipError_t err[kXferParts];
 };
 
@@ -657,7 +715,7 @@ static void xfer_part(void *arg, int64_t lo, int64_t hi, int part)
     const int64_t e0 = 64 * lo, e1 = 64 * hi < c->n ? 64 * hi : c->n;
     const size_t bytes = (size_t) (e1 - e0) * nvk * sizeof(double);
     double *stage = c->d_stage64 + e0 * nvk;
-    hipStream_t st = c->xst[part];
+    hipStream_t st = x->streams->s[part];
     int dev = c->dev;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess && dev != c->dev) e = hipSetDevice(c->dev);
@@ -673,25 +731,23 @@ static void xfer_part(void *arg, int64_t lo, int64_t hi, int part)
     x->err[part] = e != hipSuccess ? e : es;
 }
 
-// ranges of a transfer (1: one copy on the context's stream), their streams made
-static int xfer_parts(charm_gpu_ctx_t *c, size_t bytes)
+// ranges a transfer of so many bytes runs as (1: one copy on the context's stream)
+static int xfer_parts(size_t bytes)
 {
-    int t = bytes >= ((size_t) 64 << 20) ? kXferParts : bytes >= ((size_t) 12 << 20) ? 4 : 1;
-    if (t > charm_host_threads()) t = charm_host_threads();
-    for (int i = 0; t > 1 && i < t; i++)
-        if (!c->xst[i] && hipStreamCreate(&c->xst[i]) != hipSuccess) { (void) hipGetLastError(); c->xst[i] = NULL; t = i; }
-    return t > 1 ? t : 1;
+    const int t = bytes >= ((size_t) 64 << 20) ? kXferParts : bytes >= ((size_t) 12 << 20) ? 4 : 1;
+    return t > charm_host_threads() ? charm_host_threads() : t;
 }
 
+// the ranges of x on the streams taken, which are given back
 static hipError_t xfer(Xfer &x, int parts)
 {
+    if (parts > x.streams->n) parts = x.streams->n;
     // earlier work on the context's stream may use the staging or the state
     hipError_t e = hipStreamSynchronize(x.c->st);
-    if (e != hipSuccess) return e;
-    charm_par_for((x.c->n + 63) / 64, parts, xfer_part, &x);
-    for (int i = 0; i < parts; i++)
-        if (x.err[i] != hipSuccess) return x.err[i];
-    return hipSuccess;
+    if (e == hipSuccess) charm_par_for((x.c->n + 63) / 64, parts, xfer_part, &x);
+    for (int i = 0; i < parts && e == hipSuccess; i++) e = x.err[i];
+    xfer_release(x.streams);
+    return e;
 }
 
 // u into the state dst; small arrays wait for the stream, larger ones may
@@ -707,9 +763,9 @@ static hipError_t state_in(charm_gpu_ctx_t *c, const double *u, void *dst)
         const hipError_t es = hipStreamSynchronize(c->st);
         return e != hipSuccess ? e : es;
     }
-    const int parts = xfer_parts(c, bytes);
-    if (parts > 1) {
-        Xfer x = {c, NULL, dst, u, NULL, {}};
+    const int parts = xfer_parts(bytes);
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
+        Xfer x = {c, NULL, dst, u, NULL, s, {}};
         return xfer(x, parts);
     }
     const hipError_t e = hipMemcpyAsync(c->d_stage64, u, bytes, hipMemcpyHostToDevice, c->st);
@@ -729,9 +785,9 @@ static hipError_t state_out(charm_gpu_ctx_t *c, const void *src, double *u)
         if (e == hipSuccess) memcpy(u, c->h_pin + kPinHead, bytes);
         return e;
     }
-    const int parts = xfer_parts(c, bytes);
-    if (parts > 1) {
-        Xfer x = {c, src, NULL, NULL, u, {}};
+    const int parts = xfer_parts(bytes);
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
+        Xfer x = {c, src, NULL, NULL, u, s, {}};
         return xfer(x, parts);
     }
     const hipError_t e = launch_convert(c->sprec, 1, src, c->d_stage64, c->n, nvk, c->st);

@@ -45,6 +45,29 @@ def test_state_round_trip(level, n, precision):
         np.testing.assert_array_equal(ctx.get_state(), want)
 
 
+def test_contexts_share_the_transfer_streams():
+    """several threads, a context each, and contexts that come and go"""
+    f = mesh_of(80000, 5)
+    cfg = CA.make_config(flux="HLLC", precision=CA.FP64)
+    mesh = f.flatten(*CA.recommended_chunks(cfg))
+
+    def run(seed):
+        u = np.random.default_rng(seed).normal(size=(f.n, 5, 4))
+        for _ in range(2):
+            ctx = CA.GpuContext(cfg)
+            ctx.upload_mesh(mesh)
+            for _ in range(3):
+                ctx.set_state(u)
+                if not np.array_equal(ctx.get_state(), u):
+                    return False
+            ctx.close()
+        return True
+
+    with ThreadPoolExecutor(3) as ex:
+        assert all(ex.map(run, range(3)))
+    assert run(9)
+
+
 def points(n, seed):
     rng = np.random.default_rng(seed)
     r, p = rng.uniform(0.5, 2, n), rng.uniform(0.5, 2, n)
