@@ -980,6 +980,7 @@ extern "C" int charm_gpu_residual(charm_gpu_ctx_t *c, double *out, int64_t n)
 {
     int rc = need_mesh(c, n);
     if (rc) return rc;
+    if (!out) { charm_set_error("residual: null output"); return CHARM_ERR_ARG; }
     if (c->ph && c->cfg.model == CHARM_MODEL_NS && c->cfg.use_visc) {
         // viscous passes on the current state, without the chemistry
         HIPCHK(ns_temps(c, c->B[0]));

@@ -1,0 +1,62 @@
+"""The host side of the GPU entry points on the CPU, over a stand-in for the
+HIP calls (host_hip.c, loaded ahead of the library in a process of its own):
+what they refuse, what they leave queued, allocated and changed."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+def hip():
+    h = C.CDLL(os.environ["HOST_HIP"], mode=C.RTLD_GLOBAL)
+    h.hh_limit.argtypes, h.hh_live.restype = [C.c_size_t], C.c_size_t
+    return h
+
+
+def context(level, precision=0, flux="HLLC", chunks=(128, 512), mesh=None):
+    import charm_3d_amd as CA
+    ctx = CA.GpuContext(CA.make_config(precision=precision, flux=flux))
+    ctx.upload_mesh(mesh or CA.Forest.uniform(level).flatten(*chunks))
+    return ctx
+
+
+def null_arrays():
+    """a null state is an argument error at every size of transfer"""
+    import charm_3d_amd as CA
+    L = CA.lib()
+    for level in (1, 4, 6):              # pinned, one copy, ranges
+        ctx = context(level)
+        for fn in (L.charm_gpu_set_state, L.charm_gpu_get_state, L.charm_gpu_residual):
+            assert fn(ctx.h, None, ctx.n) == -1, fn.__name__
+            assert b"null" in L.charm_gpu_last_error()
+        ctx.close()
+
+
+CASES = {f.__name__: f for f in (null_arrays,)}
+
+
+@pytest.fixture(scope="module")
+def host_hip(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "host_hip.so")
+    subprocess.run(["gcc", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-pthread", "-o", so,
+                    os.path.join(HERE, "host_hip.c")], check=True)
+    return so
+
+
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_host_side(case, host_hip):
+    env = dict(os.environ, HOST_HIP=host_hip, CHARM_HOST_THREADS="4")
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), case], env=env, capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+if __name__ == "__main__":
+    sys.path[:0] = [HERE, os.path.dirname(HERE)]
+    HIP = hip()
+    CASES[sys.argv[1]]()
