@@ -49,6 +49,7 @@ struct charm_gpu_ctx {
     float last_ms;
     // mesh
     int64_t n, nch, ncf, nslot, naux;
+    int64_t fl_nch, fl_ncf;   // chunks and chunk faces of the flattening (nch, ncf: of its pieces)
     int max_faces, chunk_elems;
     int n_xcd;
     uint8_t *d_level;
@@ -584,6 +585,7 @@ extern "C" int charm_gpu_upload_mesh(charm_gpu_ctx_t *c, const charm_mesh_t *m)
     HIPCHK(hipMemcpyAsync(c->d_slots, pc.p.slots, (size_t) m->nslot * sizeof(uint16_t), hipMemcpyHostToDevice, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     c->n = m->n; c->nch = pc.p.nch; c->ncf = pc.p.ncf; c->nslot = m->nslot; c->naux = m->naux;
+    c->fl_nch = m->nch; c->fl_ncf = m->ncf;
     // the largest chunk there is sizes the workgroups and their LDS
     c->max_faces = c->chunk_elems = 1;
     for (int64_t i = 0; i < c->nch; i++) {
@@ -1218,8 +1220,9 @@ extern "C" int charm_gpu_hllc_branch_flips(charm_gpu_ctx_t *a, charm_gpu_ctx_t *
     if ((rc = need_mesh(b, -1))) return rc;
     if ((rc = need_octree(a, "hllc_branch_flips")) || (rc = need_octree(b, "hllc_branch_flips"))) return rc;
     if (!points || !flips) { charm_set_error("hllc_branch_flips: null output"); return CHARM_ERR_ARG; }
+    // (the pieces a context cuts depend on its flux; a's serve both)
     if (a->prec != CHARM_FP64 || b->prec != CHARM_FP64 || a->ph || b->ph || a->nc != b->nc || a->n != b->n ||
-        a->nch != b->nch || a->ncf != b->ncf) {
+        a->fl_nch != b->fl_nch || a->fl_ncf != b->fl_ncf) {
         charm_set_error("hllc_branch_flips: two FP64 constant-cp contexts on the same mesh");
         return CHARM_ERR_ARG;
     }

@@ -96,3 +96,21 @@ def test_small_mesh_viscous_residual(mesh, make):
     sim = OL.OracleSim(oracle_cfg(cfg), leaves)
     sim.set_state(u)
     assert var_err(got, sim.ns_residual()) <= 1e-11
+
+
+def test_branch_flips_between_fluxes():
+    """contexts whose fluxes cut one mesh into other pieces: every interior
+    (sub)face once, from either context"""
+    leaves = shell(4, 1)
+    assert 12000 < len(leaves) <= 24000
+    print(f"[gpu] n={len(leaves)} branch flips", flush=True)
+    mesh = CA.Forest.from_leaves(leaves).flatten(170, 512)
+    u = state(len(leaves), 1)
+    ctx = []
+    for flux in ("GODUNOV", "LF"):
+        ctx.append(CA.GpuContext(CA.make_config(precision=CA.FP64, flux=flux)))
+        ctx[-1].upload_mesh(mesh)
+        ctx[-1].set_state(u)
+    interior = int((mesh.faces()[:, 1] >= 0).sum())
+    for a, b in (ctx, ctx[::-1]):
+        assert a.hllc_branch_flips(b) == (6 * interior, 0)

@@ -37,7 +37,23 @@ def null_arrays():
         ctx.close()
 
 
-CASES = {f.__name__: f for f in (null_arrays,)}
+def branch_flips_across_fluxes():
+    """two contexts on one mesh of 13,824 leaves, which the exact solver's and
+    the other fluxes' contexts cut into other pieces; other leaves, and the
+    same leaves flattened otherwise, are refused"""
+    import charm_3d_amd as CA
+    lv = CA.Forest.uniform(4)
+    lv.adapt((np.arange(lv.n) % 3 == 0).astype(np.int8), 5)
+    assert 12000 < lv.n < 24000, lv.n
+    mesh = lv.flatten(170, 512)
+    a, b = (context(0, flux=f, mesh=mesh) for f in ("GODUNOV", "HLLC"))
+    assert a.hllc_branch_flips(b) == (0, 0) and b.hllc_branch_flips(a) == (0, 0)
+    for other in (context(4), context(0, mesh=lv.flatten(100, 300))):
+        with pytest.raises(CA.CharmError, match="same mesh"):
+            a.hllc_branch_flips(other)
+
+
+CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes)}
 
 
 @pytest.fixture(scope="module")
