@@ -248,8 +248,11 @@ static void adj_boundary_free(charm_gpu_ctx_t *c)
     c->bnd_ok = 0;
 }
 
+// The mesh's blocks, behind the work queued on them: an upload that fails
+// half way has fills and copies under way.
 static void free_mesh(charm_gpu_ctx_t *c)
 {
+    if (c->st) (void) hipStreamSynchronize(c->st);
     adj_boundary_free(c);
     void **p[] = {(void **) &c->d_level, (void **) &c->d_cf4, (void **) &c->d_aux,
                   (void **) &c->d_ch_ebeg, (void **) &c->d_ch_fbeg, (void **) &c->d_ch_ref, (void **) &c->d_slot_ptr,
@@ -427,7 +430,6 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
 extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
 {
     if (!c) return CHARM_OK;
-    if (c->st) (void) hipStreamSynchronize(c->st);
     free_mesh(c);
     idle_release(c);
     charm_cut_buf_free(&c->cut);

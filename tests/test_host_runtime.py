@@ -53,7 +53,33 @@ def branch_flips_across_fluxes():
             a.hllc_branch_flips(other)
 
 
-CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes)}
+def failed_uploads():
+    """an upload that runs out of device memory at any of its allocations
+    leaves no work queued on the blocks it gives back, and no mesh"""
+    import charm_3d_amd as CA
+    mesh = CA.Forest.uniform(3).flatten(128, 512)
+    ctx = context(3)
+    used = HIP.hh_live()
+    ctx.close()
+    failed = 0
+    for limit in range(used // 40, used, used // 40):
+        ctx = CA.GpuContext(CA.make_config(precision=CA.FP64))
+        HIP.hh_limit(limit)
+        try:
+            ctx.upload_mesh(mesh)
+        except CA.CharmError as e:
+            failed += 1
+            assert "hipMalloc" in str(e) and HIP.hh_queued() == 0, HIP.hh_queued()
+            with pytest.raises(CA.CharmError, match="no mesh"):
+                ctx.run(0.1, 1)
+        HIP.hh_limit(1 << 32)
+        ctx.upload_mesh(mesh)
+        ctx.run(0.1, 1)
+        ctx.close()
+    assert failed > 30 and HIP.hh_live() == 0
+
+
+CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads)}
 
 
 @pytest.fixture(scope="module")
