@@ -1509,6 +1509,11 @@ extern "C" int charm_gpu_remesh(charm_gpu_ctx_t *c, const charm_mesh_t *m, const
     int64_t *d_map = NULL;
     hipError_t e = hipSuccess;
     rc = charm_gpu_upload_mesh(c, m);
+    if (rc && c->n) {                // refused: the context keeps its mesh and state
+        c->B[0] = u_old;
+        c->d_q = q_old;
+        return rc;
+    }
     if (!rc) {
         e = dalloc(c, (void **) &d_map, (size_t) (m->n ? m->n : 1) * sizeof(int64_t));
         if (e == hipSuccess) e = hipMemcpyAsync(d_map, map, (size_t) m->n * sizeof(int64_t), hipMemcpyHostToDevice, c->st);

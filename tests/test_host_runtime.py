@@ -79,7 +79,18 @@ def failed_uploads():
     assert failed > 30 and HIP.hh_live() == 0
 
 
-CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads)}
+def refused_remesh():
+    """a mesh that remesh refuses leaves the context its mesh and state"""
+    import charm_3d_amd as CA
+    ctx = context(3)
+    n = ctx.n
+    with pytest.raises(CA.CharmError, match="LDS"):
+        ctx.remesh(CA.Forest.uniform(3).flatten(170, 1000), np.arange(n))
+    assert ctx.n == n
+    ctx.adjoint(0.1, 1, [0.0] * 3, [1.0] * 3, ckpt=0)    # copies the state
+
+
+CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads, refused_remesh)}
 
 
 @pytest.fixture(scope="module")
