@@ -98,6 +98,7 @@ struct charm_gpu_ctx {
     int n_live, n_idle;
     size_t idle_bytes;
     pthread_mutex_t pin_mu, mem_mu;
+    charm_gpu_ctx *next;      // list of the process's contexts (ctx_list)
 };
 
 namespace {
@@ -168,36 +169,68 @@ static void xfer_release(XferStreams *x)
 // all, and serves the next request that fills at least half of it: a remesh
 // makes some fifteen allocations and as many frees, each a call of 5-100 us,
 // and so do the reverse stage and the point-wise fluxes.  Blocks are freed only
-// behind a synchronised stream.  The kept ones are given back before an
-// allocation fails, and with the context.
+// behind a synchronised stream.  The kept ones of every context on the device
+// are given back before an allocation fails, and a context's own with it.
+static struct {
+    pthread_mutex_t mu;       // taken ahead of a context's mem_mu
+    charm_gpu_ctx_t *head;
+} ctx_list = {PTHREAD_MUTEX_INITIALIZER, NULL};
+
+static void ctx_list_add(charm_gpu_ctx_t *c)
+{
+    Lock lock(&ctx_list.mu);
+    c->next = ctx_list.head;
+    ctx_list.head = c;
+}
+
+static void ctx_list_remove(charm_gpu_ctx_t *c)
+{
+    Lock lock(&ctx_list.mu);
+    for (charm_gpu_ctx_t **p = &ctx_list.head; *p; p = &(*p)->next)
+        if (*p == c) { *p = c->next; return; }
+}
+
 static void idle_release(charm_gpu_ctx_t *c)
 {
+    Lock lock(&c->mem_mu);
     for (int i = 0; i < c->n_idle; i++) (void) hipFree(c->idle[i].p);
     c->n_idle = 0;
     c->idle_bytes = 0;
 }
 
+// hipMalloc, once more after the kept blocks of the device went back
+static hipError_t device_malloc(int dev, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void) hipGetLastError();
+    {
+        Lock lock(&ctx_list.mu);
+        for (charm_gpu_ctx_t *x = ctx_list.head; x; x = x->next)
+            if (x->dev == dev) idle_release(x);
+    }
+    return hipMalloc(p, bytes);
+}
+
 static hipError_t dalloc(charm_gpu_ctx_t *c, void **p, size_t bytes)
 {
-    Lock lock(&c->mem_mu);
     if (bytes < 256) bytes = 256;
-    int best = -1;
-    for (int i = 0; i < c->n_idle; i++)
-        if (c->idle[i].bytes >= bytes && c->idle[i].bytes / 2 <= bytes &&
-            (best < 0 || c->idle[i].bytes < c->idle[best].bytes)) best = i;
-    if (best >= 0 && c->n_live < kLiveBlocks) {
-        c->live[c->n_live++] = c->idle[best];
-        *p = c->idle[best].p;
-        c->idle_bytes -= c->idle[best].bytes;
-        c->idle[best] = c->idle[--c->n_idle];
-        return hipSuccess;
+    {
+        Lock lock(&c->mem_mu);
+        int best = -1;
+        for (int i = 0; i < c->n_idle; i++)
+            if (c->idle[i].bytes >= bytes && c->idle[i].bytes / 2 <= bytes &&
+                (best < 0 || c->idle[i].bytes < c->idle[best].bytes)) best = i;
+        if (best >= 0 && c->n_live < kLiveBlocks) {
+            c->live[c->n_live++] = c->idle[best];
+            *p = c->idle[best].p;
+            c->idle_bytes -= c->idle[best].bytes;
+            c->idle[best] = c->idle[--c->n_idle];
+            return hipSuccess;
+        }
     }
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess && c->n_idle) {
-        (void) hipGetLastError();
-        idle_release(c);
-        e = hipMalloc(p, bytes);
-    }
+    const hipError_t e = device_malloc(c->dev, p, bytes);
+    Lock lock(&c->mem_mu);
     if (e == hipSuccess && c->n_live < kLiveBlocks) { c->live[c->n_live].p = *p; c->live[c->n_live++].bytes = bytes; }
     return e;
 }
@@ -409,7 +442,7 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
         (e = hipEventCreate(&c->ev1)) != hipSuccess || (e = hipGetDevice(&c->dev)) != hipSuccess ||
         (e = hipHostMalloc((void **) &c->h_pin, kPinHead + kPinBytes, hipHostMallocDefault)) != hipSuccess ||
         (e = hipHostGetDevicePointer((void **) &c->d_pin, c->h_pin, 0)) != hipSuccess ||
-        (e = hipMalloc(&c->d_P, sizeof(DevParams))) != hipSuccess ||
+        (e = device_malloc(c->dev, (void **) &c->d_P, sizeof(DevParams))) != hipSuccess ||
         (e = hipMemcpyAsync(c->d_P, &c->P, sizeof(DevParams), hipMemcpyHostToDevice, c->st)) != hipSuccess ||
         (e = hipStreamSynchronize(c->st)) != hipSuccess) {
         charm_set_error("gpu_create: %s", hipGetErrorString(e));
@@ -420,6 +453,7 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
     // memory: read after a synchronisation, without a copy (8 us each)
     memset(c->h_pin, 0, kPinHead);
     xfer_pool_ref(1);
+    ctx_list_add(c);
     c->pooled = 1;
     c->d_err = (int *) c->d_pin;
     c->d_result = (double *) (c->d_pin + 64);
@@ -430,6 +464,7 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
 extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
 {
     if (!c) return CHARM_OK;
+    ctx_list_remove(c);
     free_mesh(c);
     idle_release(c);
     charm_cut_buf_free(&c->cut);
@@ -1230,7 +1265,7 @@ extern "C" int charm_gpu_hllc_branch_flips(charm_gpu_ctx_t *a, charm_gpu_ctx_t *
     }
     unsigned long long host[2 + kHllcBits] = {0}, *dev = NULL;
     HIPCHK(hipStreamSynchronize(b->st));
-    HIPCHK(hipMalloc((void **) &dev, sizeof(host)));
+    HIPCHK(device_malloc(a->dev, (void **) &dev, sizeof(host)));
     FlipArgs F;
     F.Ua = (const double *) a->B[0]; F.Ub = (const double *) b->B[0];
     F.cf4 = a->d_cf4; F.ch_ebeg = a->d_ch_ebeg; F.ch_fbeg = a->d_ch_fbeg;

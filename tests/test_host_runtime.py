@@ -90,7 +90,25 @@ def refused_remesh():
     ctx.adjoint(0.1, 1, [0.0] * 3, [1.0] * 3, ckpt=0)    # copies the state
 
 
-CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads, refused_remesh)}
+def blocks_kept_by_other_contexts():
+    """an allocation that would fail is served from what other contexts keep
+    of freed blocks, and a context that is gone is not asked"""
+    import charm_3d_amd as CA
+    gone, a, b = context(4), context(5), context(1)
+    gone.close()
+    a.upload_mesh(CA.Forest.uniform(1).flatten())        # level 5's blocks are free now
+    HIP.hh_limit(HIP.hh_live() + 65536)
+    b.upload_mesh(CA.Forest.uniform(5).flatten(128, 512))
+    with pytest.raises(CA.CharmError, match="out of memory"):
+        a.upload_mesh(CA.Forest.uniform(5).flatten(128, 512))
+    HIP.hh_limit(1 << 32)
+    a.close()
+    b.close()
+    assert HIP.hh_live() == 0
+
+
+CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads, refused_remesh,
+                                 blocks_kept_by_other_contexts)}
 
 
 @pytest.fixture(scope="module")
