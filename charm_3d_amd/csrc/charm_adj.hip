@@ -764,7 +764,7 @@ void k_adj_bnd_pts(AdjArgs A, DevParams P)
 template <typename R, int NC>
 static hipError_t launch_adj_bnd_pts(int flux, const AdjArgs &A, const DevParams &P, hipStream_t st)
 {
-    if (A.n_bnd <= 0) return hipSuccess;
+    if (A.n_bface <= 0) return hipSuccess;
     const dim3 gp((unsigned) ((6 * (int64_t) A.n_bface + 63) / 64)), bp(64);
     switch (flux) {
     case FLUX_LF: hipLaunchKernelGGL((k_adj_bnd_pts<R, NC, FLUX_LF>), gp, bp, 0, st, A, P); break;

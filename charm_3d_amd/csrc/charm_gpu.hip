@@ -19,14 +19,15 @@ using namespace charm;
 extern "C" const char *charm_host_last_error(void);
 
 // Boundary faces of the mesh for the adjoint's boundary kernels (from the
-// neighbour table: codes -1..-6 are boundary faces): the leaves with one,
-// their face ranges, the faces (leaf * 8 + direction, ordered by leaf), and
-// the per-point scratch of their contributions.
+// neighbour table: codes -1..-6 are boundary faces): the face ranges of the
+// leaves with one, the faces (leaf * 8 + direction, ordered by leaf), each
+// leaf's index among the ranges, and the per-point scratch of the faces'
+// contributions.
 struct AdjBoundary {
-    int *elems, *ptr, *faces, *of;
+    int *ptr, *faces, *of;
     void *part;
     double *theta;
-    int n_elems, n_faces;
+    int n_faces;
     int max_items;            // most interior (sub)faces of a workgroup of k_adj_leaves
 };
 
@@ -275,7 +276,7 @@ extern "C" int charm_gpu_device_count(int *n)
 static void adj_boundary_free(charm_gpu_ctx_t *c)
 {
     AdjBoundary &b = c->bnd;
-    void *bufs[] = {b.elems, b.ptr, b.faces, b.of, b.part, b.theta};
+    void *bufs[] = {b.ptr, b.faces, b.of, b.part, b.theta};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); i++) dfree(c, bufs[i]);
     memset(&b, 0, sizeof(b));
     c->bnd_ok = 0;
@@ -1772,12 +1773,11 @@ static int adj_boundary(charm_gpu_ctx_t *c)
     if (c->bnd_ok) return CHARM_OK;
     const int64_t n = c->n;
     int *nbr = (int *) malloc((size_t) n * 6 * sizeof(int));
-    int *elems = (int *) malloc((size_t) n * sizeof(int));
     int *ptr = (int *) malloc(((size_t) n + 1) * sizeof(int));
     int *faces = (int *) malloc((size_t) n * 6 * sizeof(int));
     int *of = (int *) malloc((size_t) (n ? n : 1) * sizeof(int));
-    if (!nbr || !elems || !ptr || !faces || !of) {
-        free(nbr); free(elems); free(ptr); free(faces); free(of);
+    if (!nbr || !ptr || !faces || !of) {
+        free(nbr); free(ptr); free(faces); free(of);
         charm_set_error("adjoint: out of memory");
         return CHARM_ERR_MEM;
     }
@@ -1794,28 +1794,25 @@ static int adj_boundary(charm_gpu_ctx_t *c)
             if (i % kAdjLeaves == 0) items = 0;
             for (int d = 0; d < 6; d++) items += nbr[6 * i + d] >= 0 ? 1 : (nbr[6 * i + d] <= -8 ? 4 : 0);
             if (items > b.max_items) b.max_items = items;
-            if (nf > f0) { of[i] = ne; elems[ne] = (int) i; ptr[++ne] = nf; }
+            if (nf > f0) { of[i] = ne; ptr[++ne] = nf; }
         }
     }
     if (e == hipSuccess && ne > 0) {
-        e = dalloc(c, (void **) &b.elems, (size_t) ne * sizeof(int));
-        if (e == hipSuccess) e = dalloc(c, (void **) &b.ptr, ((size_t) ne + 1) * sizeof(int));
+        e = dalloc(c, (void **) &b.ptr, ((size_t) ne + 1) * sizeof(int));
         if (e == hipSuccess) e = dalloc(c, (void **) &b.faces, (size_t) nf * sizeof(int));
         if (e == hipSuccess) e = dalloc(c, &b.part, (size_t) nf * 6 * 4 * c->nv * c->esz);
         if (e == hipSuccess) e = dalloc(c, (void **) &b.theta, (size_t) nf * 6 * 3 * sizeof(double));
-        if (e == hipSuccess) e = hipMemcpy(b.elems, elems, (size_t) ne * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(b.ptr, ptr, ((size_t) ne + 1) * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(b.faces, faces, (size_t) nf * sizeof(int), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = dalloc(c, (void **) &b.of, (size_t) n * sizeof(int));
         if (e == hipSuccess) e = hipMemcpy(b.of, of, (size_t) n * sizeof(int), hipMemcpyHostToDevice);
     }
-    free(nbr); free(elems); free(ptr); free(faces); free(of);
+    free(nbr); free(ptr); free(faces); free(of);
     if (e != hipSuccess) {
         adj_boundary_free(c);
         charm_set_error("adjoint: %s", hipGetErrorString(e));
         return CHARM_ERR_HIP;
     }
-    b.n_elems = ne;
     b.n_faces = nf;
     c->bnd_ok = 1;
     return CHARM_OK;
@@ -1856,8 +1853,8 @@ extern "C" int charm_gpu_stage_vjp(charm_gpu_ctx_t *c, double dt, const double *
         memset(&A, 0, sizeof(A));
         A.level = c->d_level; A.nbr = c->d_nbr; A.aux = c->d_aux; A.n = n; A.dt = dt;
         A.theta_bar = NULL; A.theta_face = -1;
-        A.bnd_elems = bnd.elems; A.bnd_ptr = bnd.ptr; A.bnd_faces = bnd.faces;
-        A.n_bnd = bnd.n_elems; A.n_bface = bnd.n_faces; A.bnd_part = bnd.part; A.bnd_theta = bnd.theta;
+        A.bnd_ptr = bnd.ptr; A.bnd_faces = bnd.faces;
+        A.n_bface = bnd.n_faces; A.bnd_part = bnd.part; A.bnd_theta = bnd.theta;
         A.cf4 = chunked ? c->d_cf4 : NULL;
         A.ch_ebeg = c->d_ch_ebeg; A.ch_fbeg = c->d_ch_fbeg; A.slot_ptr = c->d_slot_ptr; A.slots = c->d_slots;
         A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems;
@@ -1985,8 +1982,8 @@ extern "C" int charm_gpu_adjoint(charm_gpu_ctx_t *c, double dt, int nsteps, int 
             AdjArgs A;
             A.level = c->d_level; A.nbr = c->d_nbr; A.aux = c->d_aux; A.n = n; A.dt = dt;
             A.theta_bar = theta_face >= 0 ? theta : NULL; A.theta_face = theta_face;
-            A.bnd_elems = bnd.elems; A.bnd_ptr = bnd.ptr; A.bnd_faces = bnd.faces;
-            A.n_bnd = bnd.n_elems; A.n_bface = bnd.n_faces; A.bnd_part = bnd.part; A.bnd_theta = bnd.theta;
+            A.bnd_ptr = bnd.ptr; A.bnd_faces = bnd.faces;
+            A.n_bface = bnd.n_faces; A.bnd_part = bnd.part; A.bnd_theta = bnd.theta;
             A.cf4 = chunked ? c->d_cf4 : NULL;
             A.ch_ebeg = c->d_ch_ebeg; A.ch_fbeg = c->d_ch_fbeg; A.slot_ptr = c->d_slot_ptr; A.slots = c->d_slots;
             A.n_chunks = (int) c->nch; A.max_faces = c->max_faces; A.chunk_elems = c->chunk_elems;

@@ -137,7 +137,7 @@ struct NsArgs {
     const DevParams *prm;     // the context's constants in device memory (read by every NS kernel)
 };
 
-// adjoint of one SSP-RK stage (one thread per leaf):
+// adjoint of one SSP-RK stage:
 // OUT = c_out (sb + (d int / d U)^T W) + c_acc ACC + c_acc2 ACC2,  sb = c_in X,
 // W = -dt A^-1 sb
 constexpr int kAdjLeaves = 32;   // leaves of a workgroup of k_adj_leaves
@@ -151,10 +151,9 @@ struct AdjArgs {
     double *theta_bar;        // [n][3] += d/d(inlet u, T, p) (or null)
     int theta_face;           // the inlet face of the parameters (-1: none)
     int64_t n;
-    const int *bnd_elems;     // leaves with at least one boundary face
-    const int *bnd_ptr;       // [n_bnd + 1]: their ranges in bnd_faces
+    const int *bnd_ptr;       // per leaf with a boundary face: its range in bnd_faces
     const int *bnd_faces;     // boundary faces, leaf * 8 + direction, by leaf
-    int n_bnd, n_bface;
+    int n_bface;
     void *bnd_part;           // [n_bface][6][4 V] point contributions (state type)
     double *bnd_theta;        // [n_bface][6][3] parameter contributions
     // chunked face-centric variant (chunks as for the stage kernel; null
@@ -163,8 +162,8 @@ struct AdjArgs {
     const int *ch_ebeg, *ch_fbeg, *slot_ptr;
     const uint16_t *slots;
     int n_chunks, max_faces, chunk_elems, n_xcd;
-    // chunked variant: per leaf its index in bnd_elems (or -1); the chunk
-    // kernel then adds the boundary parts itself (k_adj_bnd_pts runs first)
+    // per leaf its index in bnd_ptr (or -1; null: no boundary face); the stage
+    // kernels add the boundary parts (k_adj_bnd_pts runs first)
     const int *bnd_of;
     int max_items;            // kernel by leaves: most interior (sub)faces of a workgroup
     int hanging;              // the mesh has hanging faces

@@ -315,7 +315,7 @@ __device__ __forceinline__ bool face_record(const DevParams &P, const S *__restr
 // -g_v sum_gp rho phi_k wJ.
 // volume_terms: the fluxes F_d at one Gauss point (signs of g) and the density
 // there.  DEV: u holds deviation coefficients and F is F - F(U_r), the
-// momentum, energy and mass fluxes along each axis as in dev_phys; the gravity
+// momentum, energy and mass fluxes along each axis as in phys_dev; the gravity
 // term takes the full density.
 // tk (PH = 1, may be null): the point's EOS closure, its planes kMemoRows * ts
 // apart
