@@ -413,14 +413,14 @@ def bench_hot_spot(CA, W):
 
 def gmesh_stage_bytes(nv, real_bytes, faces_per_leaf):
     """HBM bytes per leaf of one multi-tree stage (face pass + element pass)
-    by design: per face the 30 basis / weight words, the FP64 normal, two
+    by design: per face the 33 basis / weight words, the FP64 normal, two
     leaf indices, both sides' states and the face sums written; per leaf its
     54 geometry words (51 and the 3 basis means), the state read and written,
-    its six face indices and face sums, side 1's 6 basis words of each face
-    where it is side 1, and its cell means for the limiter."""
+    its six face indices and face sums, 3 basis words of each face where it is
+    side 0 and 6 where it is side 1, and its cell means for the limiter."""
     s = real_bytes * 4 * nv
-    face = real_bytes * 30 + 8 * 3 + 4 * 2 + 3 * s
-    leaf = real_bytes * 54 + 2 * s + 6 * (s + 4) + (6 - faces_per_leaf) * real_bytes * 6 + real_bytes * nv
+    face = real_bytes * 33 + 8 * 3 + 4 * 2 + 3 * s
+    leaf = real_bytes * 54 + 2 * s + 6 * (s + 4) + (faces_per_leaf * 3 + (6 - faces_per_leaf) * 6) * real_bytes + real_bytes * nv
     return faces_per_leaf * face + leaf
 
 

@@ -5,10 +5,10 @@
 //
 // Face pass, one thread per face: at its 6 points both traces (side 1 from
 // the boundary condition on a boundary face), the flux along the side-0
-// normal, and side 0's moment sums, FS[4V][nf].  Side 1's basis is the affine
-// image b1 = b0 r + o of side 0's, so its sums are the same image of side 0's
-// and are not stored.  Element pass, one thread per leaf: the volume integral
-// at 8 points (flux tensor against grad phi = e / dh, gravity on the
+// normal, and its moment sums about the face's middle, FS[4V][nf], in side 0's
+// units.  Both sides' bases are affine in its offsets d from there (b0 = c + d,
+// b1 = o + d r), and so are both sides' sums, which are not stored.  Element
+// pass, one thread per leaf: the volume integral at 8 points (flux tensor against grad phi = e / dh, gravity on the
 // momentum), its six faces' sums (LF[6][n]: face << 1 | side; no atomics), the
 // full 4x4 A^-1, the update and the SSP-RK combine; ahead of the limiter also
 // the cell means of the new state.  The arithmetic is the reference's Euler
@@ -115,6 +115,7 @@ static inline int64_t xcd_grid(int64_t blocks, int n_xcd)
 // linear in the tangential velocities: with tangential velocities (1, 0) and
 // (0, 1) on the two sides the tangential fluxes are the factors a, b of
 // q = q_n n + a (u_L - u_Ln n) + b (u_R - u_Rn n), and no face frame is needed.
+// (Summed as written: q_n less a u_Ln and b u_Rn ahead of n rounds more.)
 // The exact Riemann solver's energy takes the tangential velocities themselves:
 // it runs in the reference's frame.
 template <typename R, int NC, int FLUX>
@@ -141,10 +142,9 @@ __device__ __forceinline__ bool flux_normal(const Prim<R, NC> &pa, const Prim<R,
         fa.ut1 = R(1); fa.ut2 = R(0);
         fb.ut1 = R(0); fb.ut2 = R(1);
         ok = flux_x<R, NC, FLUX>(fa, fb, q);
-        const R qn = q[0] - q[1] * fa.un - q[2] * fb.un;
-        g[0] = qn * n3[0] + q[1] * pa.u + q[2] * pb.u;
-        g[1] = qn * n3[1] + q[1] * pa.v + q[2] * pb.v;
-        g[2] = qn * n3[2] + q[1] * pa.w + q[2] * pb.w;
+        g[0] = q[0] * n3[0] + q[1] * (pa.u - fa.un * n3[0]) + q[2] * (pb.u - fb.un * n3[0]);
+        g[1] = q[0] * n3[1] + q[1] * (pa.v - fa.un * n3[1]) + q[2] * (pb.v - fb.un * n3[1]);
+        g[2] = q[0] * n3[2] + q[1] * (pa.w - fa.un * n3[2]) + q[2] * (pb.w - fb.un * n3[2]);
     }
     #pragma unroll
     for (int v = 3; v < NV; v++) g[v] = q[v];
@@ -155,10 +155,15 @@ __device__ __forceinline__ bool flux_normal(const Prim<R, NC> &pa, const Prim<R,
 // saved), no face frame and four waves per SIMD took the FP32 HLLC pass over
 // 6.3M faces from 615 to 391 us and over 0.79M from 82 to 47; FP64 6.3M faces
 // 1,668 to 763.  The element pass, which now gathers half its sums through the
-// face index, went from 390 to 379 us (FP32, 2.1M leaves) and 782 to 717 (FP64):
-// stage 5.8 TB/s of designed bytes in FP32 against 5.1 of a large copy.
+// face index, went from 390 to 379 us (FP32, 2.1M leaves) and 782 to 717 (FP64).
+// The face's middle as the moments' origin costs 3 words per face more than
+// side 0's centre (stage 754 -> 770 us in FP32 and 1,457 -> 1,535 in FP64 at 2.1M
+// leaves) and takes the FP32 rounding between neighbours of extents 1 : 10 from
+// 9.7-13 units of the last place of a face's flux to 4.3-7.
+// Two waves per SIMD in FP64 with one and two species (HLLC and two species
+// took 258 registers and ran at one: stage at 262,144 leaves 287 us, 232 so).
 template <typename R, int NC, int FLUX>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(256, sizeof(R) == 8 && NC <= 2 && FLUX != FLUX_GODUNOV ? 2 : 1)
 void k_gface(GArgs A, DevParams P)
 {
     constexpr int NV = 4 + NC;
@@ -181,23 +186,24 @@ void k_gface(GArgs A, DevParams P)
         #pragma unroll
         for (int k = 0; k < 4; k++) s0[v][k] = R(0);
     bool ok = true;
-    // side 1's basis is the affine image of side 0's: b1 = b0 r + o per axis
-    const R r1[3] = {FG[18 * nf], FG[19 * nf], FG[20 * nf]}, o1[3] = {FG[21 * nf], FG[22 * nf], FG[23 * nf]};
+    const R c0[3] = {FG[0], FG[nf], FG[2 * nf]};
+    const R r1[3] = {FG[21 * nf], FG[22 * nf], FG[23 * nf]}, o1[3] = {FG[24 * nf], FG[25 * nf], FG[26 * nf]};
     // rolled (114 registers, four waves per SIMD; unrolled 171 and two), each
     // point's basis and weight loaded one point ahead
-    R bn[4] = {FG[0], FG[nf], FG[2 * nf], FG[24 * nf]};
+    R bn[4] = {FG[3 * nf], FG[4 * nf], FG[5 * nf], FG[27 * nf]};
     #pragma unroll 1
     for (int p = 0; p < 6; p++) {
-        const R b0[3] = {bn[0], bn[1], bn[2]}, wj = bn[3];
+        const R d[3] = {bn[0], bn[1], bn[2]}, wj = bn[3];
         const int pn = p < 5 ? p + 1 : 5;
-        bn[0] = FG[(3 * pn) * nf]; bn[1] = FG[(3 * pn + 1) * nf]; bn[2] = FG[(3 * pn + 2) * nf];
-        bn[3] = FG[(24 + pn) * nf];
+        bn[0] = FG[(3 * pn + 3) * nf]; bn[1] = FG[(3 * pn + 4) * nf]; bn[2] = FG[(3 * pn + 5) * nf];
+        bn[3] = FG[(27 + pn) * nf];
         R t[NV];
         Prim<R, NC> pa, pb;
+        const R b0[3] = {c0[0] + d[0], c0[1] + d[1], c0[2] + d[2]};
         trace_at<R, NV>(u0, b0, t);
         cons_to_prim<R, NC, 0>(P, t, pa);
         if (e1 >= 0) {
-            const R b1[3] = {b0[0] * r1[0] + o1[0], b0[1] * r1[1] + o1[1], b0[2] * r1[2] + o1[2]};
+            const R b1[3] = {d[0] * r1[0] + o1[0], d[1] * r1[1] + o1[1], d[2] * r1[2] + o1[2]};
             trace_at<R, NV>(u1, b1, t);
             cons_to_prim<R, NC, 0>(P, t, pb);
         } else {
@@ -205,7 +211,7 @@ void k_gface(GArgs A, DevParams P)
         }
         R g[NV];
         ok &= flux_normal<R, NC, FLUX>(pa, pb, nn, n3, g);
-        const R ph0[4] = {wj, b0[0] * wj, b0[1] * wj, b0[2] * wj};
+        const R ph0[4] = {wj, d[0] * wj, d[1] * wj, d[2] * wj};
         #pragma unroll
         for (int v = 0; v < NV; v++)
             #pragma unroll
@@ -279,10 +285,10 @@ void k_gelem(GArgs A, DevParams P)
             #pragma unroll
             for (int k = 0; k < 4; k++) s[v][k] = (FS + (int64_t) (4 * v + k) * nf)[f];
         if (lf[d] & 1) {
-            // side 1: -sum g (1, b1) wj with b1 = b0 r + o
+            // side 1: -sum g (1, o + d r) wj
             R r[3], o[3];
             #pragma unroll
-            for (int k = 0; k < 3; k++) { r[k] = (FG + (18 + k) * nf)[f]; o[k] = (FG + (21 + k) * nf)[f]; }
+            for (int k = 0; k < 3; k++) { r[k] = (FG + (21 + k) * nf)[f]; o[k] = (FG + (24 + k) * nf)[f]; }
             #pragma unroll
             for (int v = 0; v < NV; v++) {
                 in[v][0] -= s[v][0];
@@ -290,10 +296,16 @@ void k_gelem(GArgs A, DevParams P)
                 for (int k = 0; k < 3; k++) in[v][1 + k] -= s[v][1 + k] * r[k] + s[v][0] * o[k];
             }
         } else {
+            // side 0: sum g (1, c + d) wj
+            R c[3];
             #pragma unroll
-            for (int v = 0; v < NV; v++)
+            for (int k = 0; k < 3; k++) c[k] = (FG + k * nf)[f];
+            #pragma unroll
+            for (int v = 0; v < NV; v++) {
+                in[v][0] += s[v][0];
                 #pragma unroll
-                for (int k = 0; k < 4; k++) in[v][k] += s[v][k];
+                for (int k = 0; k < 3; k++) in[v][1 + k] += s[v][1 + k] + s[v][0] * c[k];
+            }
         }
     }
     R *__restrict__ out = reinterpret_cast<R *>(A.out);

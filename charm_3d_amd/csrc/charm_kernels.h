@@ -92,7 +92,7 @@ struct GArgs {
     const void *U;            // stage: the state the residual is evaluated on; limiter: W
     const void *U0;           // SSP-RK combine base
     void *out;                // mode 0: the residual integrals; else the new state
-    void *fs;                 // [4V][nf] side 0's moment sums of each face
+    void *fs;                 // [4V][nf] moment sums of each face about its middle
     void *mb;                 // [V][n] cell means of the stage output for the limiter (or null)
     const void *lg, *fg;      // [CHARM_GM_LEAFQ][n], [CHARM_GM_FACEQ][nf]
     const double *fn;         // [3][nf] side-0 outward normals (FP64: the reference's face frame)

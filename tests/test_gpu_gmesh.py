@@ -205,3 +205,39 @@ def test_octree_entry_points_refuse_a_multi_tree_context():
     ctx2 = CA.GpuContext(cfg2)
     with pytest.raises(CA.CharmError, match="multi-tree"):
         ctx2.upload_gmesh(CA.GMesh(v, t2v, tb, 0))
+
+
+@pytest.mark.parametrize("mach", [1.0, 10.0])
+@pytest.mark.parametrize("flux", ["LF", "HLLC", "CD", "GODUNOV"])
+def test_gmesh_fp32_rounding_of_stretched_neighbours(flux, mach):
+    """FP32 against FP64 where neighbours' extents differ by 10 and the stream
+    carries most of the flux, in units of 2^-24 of the leaf's largest face
+    times the flux.  A face point's flux takes some 20 roundings of at most half
+    a unit, 2 in the mean; both sides' momentum, energy and mass integrals add
+    at most six such faces, of which two are as large: 3 in the mean, and 9 is
+    three times that over the 6,144 integrals.  The bases of the small leaf must
+    not be formed as differences of the large one's: that gave 9.7 to 13."""
+    worst = 0.0
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        v, t2v, tb = W.distorted_box_trees(4, 0.0)
+        idx = np.rint(4 * v).astype(int)
+        v = np.array([0.0, 1, 11, 12, 22])[idx] + np.where((idx > 0) & (idx < 4), 0.1 * rng.uniform(-1, 1, v.shape), 0)
+        n = 512
+        rho, p = 1 + 0.05 * rng.uniform(-1, 1, (2, n))
+        vel = 1.183 * mach * np.array([0.6, 0.64, 0.48]) * (1 + 0.01 * rng.normal(size=(n, 3)))
+        u = np.zeros((n, 5, 4))
+        u[:, :, 0] = W.prim_to_cons(rho, vel, p)
+        u[:, :, 1:] = 0.001 * rng.normal(size=(n, 5, 3)) * u[:, :, :1]
+        u = u.astype(np.float32).astype(np.float64)
+        res = {}
+        for prec in (CA.FP64, CA.FP32):
+            ctx, gm = gdevice(CA.make_config(precision=prec, flux=flux), v, t2v, tb, 1, u)
+            res[prec] = ctx.residual()
+        dh = gm.geometry()["dh"]
+        area = (dh.prod(1, keepdims=True) / dh).max(1)
+        q, speed, pm = u[:, :, 0].max(0), np.sqrt((vel ** 2).sum(1)).max(), p.max()
+        f = np.array([pm + q[4] * speed ** 2] * 3 + [(q[3] + pm) * speed, q[4] * speed])
+        worst = max(worst, (np.abs(res[CA.FP32] - res[CA.FP64]).max(2) / (area[:, None] * f)).max() * 2.0 ** 24)
+    print(f"[gmesh] {flux} M {mach}: {worst:.2f}", flush=True)
+    assert worst <= 9.0, worst
