@@ -869,19 +869,25 @@ static hipError_t launch_adj_leaves(const AdjArgs &A, const DevParams &P, hipStr
     return hipGetLastError();
 }
 
-// Stage adjoint with its boundary points and launch gaps, us, at 512 / 4,096 /
-// 9,192 (hanging) / 32,768 / 262,144 leaves, HLLC one species: FP32 by chunks 39
-// / 43 / 45 / 52 / 175, by leaves 35 / 34 / 40 / 59 / 305: leaves up to 12,000
-// (19,104: 52 both).  FP64 by leaves with one workgroup per CU and no spills 46
-// / 43 / 70 / 123 / 818, with two and 100 spilled registers 51 / 50 / 73 / 112 /
-// 717: two beyond 24,000 (40,328 hanging: 162 and 165).  One thread per leaf 118
-// / 118 / 506 / 125 / 439, 86,864 with hanging faces 493 against 281 by leaves:
-// it keeps the meshes without hanging faces beyond 65,536.
+// The rules of launch_adj_flux; stage adjoint with its boundary points and
+// launch gaps, us, at 4,096 / 8,800 (hanging) / 17,928 (hanging) / 32,768 leaves:
+//   FP32 by chunks against by leaves: HLLC 41 43 50 51 and 33 40 50 61, LF 40
+//     40 45 45 and 30 38 45 52 (CD as LF): leaves up to 12,000; two species HLLC
+//     52 52 63 64 and 37 45 57 68, LF 49 48 57 58 and 34 42 52 61: up to 24,000.
+//     At 262,144 by chunks 175, by leaves 307.
+//   FP64 by leaves with one workgroup per CU and no spills against two with
+//     spilled registers: HLLC 41 65 91 122 and 50 67 95 112, two species LF 46
+//     71 100 134 and 52 72 100 116: two beyond 24,000; LF 37 57 79 105 and 39 50
+//     70 83 (CD as LF): beyond 6,000; two species HLLC 51 82 116 155 and 69 97 149
+//     169 (37,472 hanging: 194 and 247; 83,672: 367 and 454): never.
+//   FP64, one thread per leaf without hanging faces: HLLC 105 at 4,096, 111 at
+//     32,768 and 445 at 262,144 leaves, where leaves take 738 (LF 330 and 491,
+//     two species HLLC 717 and 1,083): beyond 65,536.
 template <typename R, int NC, int FLUX>
 static hipError_t launch_adj_flux(const AdjArgs &A, const DevParams &P, hipStream_t st)
 {
     if constexpr (sizeof(R) == 4) {
-        if (A.cf4 && A.n > 12000) return launch_adj_chunk<R, NC, FLUX>(A, P, st);
+        if (A.cf4 && A.n > (NC == 1 ? 12000 : 24000)) return launch_adj_chunk<R, NC, FLUX>(A, P, st);
         return launch_adj_leaves<R, NC, FLUX, 2>(A, P, st);
     } else {
         if (A.n > 65536 && !A.hanging) {
@@ -889,7 +895,10 @@ static hipError_t launch_adj_flux(const AdjArgs &A, const DevParams &P, hipStrea
             hipLaunchKernelGGL((k_adj_stage<R, NC, FLUX>), grid, block, 0, st, A, P);
             return hipGetLastError();
         }
-        return A.n > 24000 ? launch_adj_leaves<R, NC, FLUX, 2>(A, P, st) : launch_adj_leaves<R, NC, FLUX, 1>(A, P, st);
+        if constexpr (FLUX != FLUX_HLLC || NC == 1) {
+            if (A.n > (FLUX != FLUX_HLLC && NC == 1 ? 6000 : 24000)) return launch_adj_leaves<R, NC, FLUX, 2>(A, P, st);
+        }
+        return launch_adj_leaves<R, NC, FLUX, 1>(A, P, st);
     }
 }
 

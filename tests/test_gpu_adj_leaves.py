@@ -1,7 +1,8 @@
 """The stage VJP at the sizes where its kernels change (by leaves up to 12,000
-leaves in FP32 and everywhere in FP64, there with two workgroups per CU beyond
-24,000, and a thread per leaf beyond 65,536 without hanging faces; by chunks
-beyond 12,000 in FP32): <S_u^T x, v> in FP64 against the
+leaves in FP32, 24,000 with two species, by chunks beyond; by leaves in FP64,
+but for HLLC with two species with two workgroups per CU beyond 24,000, LF and
+CD with one species beyond 6,000, and a thread per leaf beyond 65,536 without
+hanging faces): <S_u^T x, v> in FP64 against the
 central difference of <x, S(u)> to 1e-7, one leaf to 32,768, hanging faces, a
 leaf that is its own periodic neighbour; FP32 against FP64 to 1e-5."""
 import numpy as np
