@@ -32,6 +32,7 @@ struct AdjBoundary {
 };
 
 constexpr int kXferParts = 8;              // streams of a large state transfer
+constexpr size_t kXferMake = (size_t) 96 << 20;
 constexpr size_t kPinBytes = 256 * 1024;   // pinned buffer of small transfers
 constexpr size_t kPinHead = 4096;          // error flag and reduction results ahead of it
 constexpr int kLiveBlocks = 96, kIdleBlocks = 48;
@@ -89,7 +90,6 @@ struct charm_gpu_ctx {
     int *d_err;
     // host side of the calls
     int dev;                  // the device of the context
-    int pooled;               // holds a reference to the transfer streams
     char *h_pin, *d_pin;      // pinned, mapped: flag, results, kPinBytes of small transfers (pin_mu)
     AdjBoundary bnd;          // of the mesh, built by the first adjoint call on it
     int bnd_ok;
@@ -110,34 +110,29 @@ struct Lock {
 };
 } // namespace
 
-// The streams of large transfers, kXferParts on each of up to eight devices,
-// shared by the contexts of the process: a stream's first copy of pageable
-// memory makes the runtime's staging for it, which cost a new context with
-// streams of its own 2-3 ms.  One transfer at a time holds a device's streams
-// (another one meanwhile takes its context's own stream); the last context
-// gives them back.
+// The streams of large transfers, up to kXferParts on each of up to eight
+// devices, shared by the contexts of the process.  Four of them with the
+// runtime's staging for pageable memory, made by a stream's first copies, take
+// 3-4 ms, what they save over 60-100 MB: they are made by the transfer with
+// which a device's come to kXferMake bytes, and kept from then on, beyond the
+// context (a program that has one context at a time would make them again for
+// each).  One transfer at a time holds a device's streams; another one
+// meanwhile takes its context's own stream.  They are given back when the
+// device runs out of memory.
 struct XferStreams {
     hipStream_t s[kXferParts];
     int dev, n, busy;
+    size_t seen;              // bytes of the transfers so far
 };
 static struct {
     pthread_mutex_t mu;
-    int refs, n;
+    int n;
     XferStreams d[8];
-} xfer_pool = {PTHREAD_MUTEX_INITIALIZER, 0, 0, {}};
+} xfer_pool = {PTHREAD_MUTEX_INITIALIZER, 0, {}};
 
-static void xfer_pool_ref(int by)
-{
-    Lock lock(&xfer_pool.mu);
-    xfer_pool.refs += by;
-    if (xfer_pool.refs > 0) return;
-    for (int i = 0; i < xfer_pool.n; i++)
-        for (int k = 0; k < xfer_pool.d[i].n; k++) (void) hipStreamDestroy(xfer_pool.d[i].s[k]);
-    xfer_pool.n = 0;
-}
-
-// the streams of a device, at least two and up to `want`, or NULL
-static XferStreams *xfer_acquire(int dev, int want)
+// the streams of a device for a transfer of so many bytes, at least two and up
+// to `want`, or NULL
+static XferStreams *xfer_acquire(int dev, int want, size_t bytes)
 {
     Lock lock(&xfer_pool.mu);
     XferStreams *x = NULL;
@@ -148,8 +143,10 @@ static XferStreams *xfer_acquire(int dev, int want)
         x = &xfer_pool.d[xfer_pool.n++];
         x->dev = dev;
         x->n = x->busy = 0;
+        x->seen = 0;
     }
-    if (x->busy) return NULL;
+    if (x->seen < kXferMake) x->seen += bytes;
+    if (x->busy || x->seen < kXferMake) return NULL;
     int cur = dev;
     if (hipGetDevice(&cur) != hipSuccess || (cur != dev && hipSetDevice(dev) != hipSuccess)) { (void) hipGetLastError(); return NULL; }
     while (x->n < want && hipStreamCreate(&x->s[x->n]) == hipSuccess) x->n++;
@@ -158,6 +155,17 @@ static XferStreams *xfer_acquire(int dev, int want)
     if (x->n < 2) return NULL;
     x->busy = 1;
     return x;
+}
+
+static void xfer_give_back(int dev)
+{
+    Lock lock(&xfer_pool.mu);
+    for (int i = 0; i < xfer_pool.n; i++) {
+        XferStreams &x = xfer_pool.d[i];
+        if (x.dev != dev || x.busy) continue;
+        while (x.n > 0) (void) hipStreamDestroy(x.s[--x.n]);
+        x.seen = 0;
+    }
 }
 
 static void xfer_release(XferStreams *x)
@@ -199,7 +207,7 @@ static void idle_release(charm_gpu_ctx_t *c)
     c->idle_bytes = 0;
 }
 
-// hipMalloc, once more after the kept blocks of the device went back
+// hipMalloc, once more after the device's kept blocks and streams went back
 static hipError_t device_malloc(int dev, void **p, size_t bytes)
 {
     hipError_t e = hipMalloc(p, bytes);
@@ -210,6 +218,7 @@ static hipError_t device_malloc(int dev, void **p, size_t bytes)
         for (charm_gpu_ctx_t *x = ctx_list.head; x; x = x->next)
             if (x->dev == dev) idle_release(x);
     }
+    xfer_give_back(dev);
     return hipMalloc(p, bytes);
 }
 
@@ -453,9 +462,7 @@ extern "C" int charm_gpu_create(const charm_config_t *cfg, charm_gpu_ctx_t **out
     // the kernels' error flag and the reductions' results are written to host
     // memory: read after a synchronisation, without a copy (8 us each)
     memset(c->h_pin, 0, kPinHead);
-    xfer_pool_ref(1);
     ctx_list_add(c);
-    c->pooled = 1;
     c->d_err = (int *) c->d_pin;
     c->d_result = (double *) (c->d_pin + 64);
     *out = c;
@@ -470,7 +477,6 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
     idle_release(c);
     charm_cut_buf_free(&c->cut);
     if (c->h_pin) (void) hipHostFree(c->h_pin);
-    if (c->pooled) xfer_pool_ref(-1);
     if (c->d_P) (void) hipFree(c->d_P);
     if (c->ev0) (void) hipEventDestroy(c->ev0);
     if (c->ev1) (void) hipEventDestroy(c->ev1);
@@ -804,7 +810,7 @@ static hipError_t state_in(charm_gpu_ctx_t *c, const double *u, void *dst)
         return e != hipSuccess ? e : es;
     }
     const int parts = xfer_parts(bytes);
-    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts, bytes) : NULL) {
         Xfer x = {c, NULL, dst, u, NULL, s, {}};
         return xfer(x, parts);
     }
@@ -826,7 +832,7 @@ static hipError_t state_out(charm_gpu_ctx_t *c, const void *src, double *u)
         return e;
     }
     const int parts = xfer_parts(bytes);
-    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts, bytes) : NULL) {
         Xfer x = {c, src, NULL, NULL, u, s, {}};
         return xfer(x, parts);
     }

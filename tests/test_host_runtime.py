@@ -107,8 +107,34 @@ def blocks_kept_by_other_contexts():
     assert HIP.hh_live() == 0
 
 
+def transfer_streams():
+    """streams for large transfers are made once a process has moved 96 MB,
+    are kept across contexts, are shared, and go back when memory runs out"""
+    import charm_3d_amd as CA
+    mesh = CA.Forest.uniform(6).flatten(170, 512)        # a state of 42 MB
+    ctx = context(0, mesh=mesh)
+    u = np.zeros((ctx.n, 5, 4))
+    made = []
+    for _ in range(4):
+        ctx.set_state(u)
+        made.append(HIP.hh_streams() - 1)
+    assert made == [0, 0, 4, 4], made
+    ctx.close()
+    assert HIP.hh_streams() == 4
+    a, b = context(0, mesh=mesh), context(0, mesh=mesh)
+    a.set_state(u)
+    b.set_state(u)
+    assert HIP.hh_streams() == 4 + 2
+    HIP.hh_limit(HIP.hh_live())
+    with pytest.raises(CA.CharmError, match="out of memory"):
+        a.objective(0.1, 1000, [0.0] * 3, [1.0] * 3)
+    assert HIP.hh_streams() == 2
+    HIP.hh_limit(1 << 32)
+    np.testing.assert_array_equal(a.get_state(), u)
+
+
 CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads, refused_remesh,
-                                 blocks_kept_by_other_contexts)}
+                                 blocks_kept_by_other_contexts, transfer_streams)}
 
 
 @pytest.fixture(scope="module")
