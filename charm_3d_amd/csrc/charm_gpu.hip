@@ -1200,15 +1200,26 @@ extern "C" int charm_gpu_recommended_chunks(const charm_config_t *cfg, int *ce, 
         if (bs == 128 || faces / 3 > 128 || config_physics(cfg)) break;
     }
     // Whole passes of 256 faces: a partial last pass costs its full latency.
-    // Stage, us, at the size above against this one: FP64 one species 262,144
-    // leaves LF 104 / 94, HLLC 141 / 129, exact 473 / 428 (528 / 512 faces); FP64 two
-    // species 170,248 leaves HLLC 227 / 151, exact 507 / 329 (442 / 256); FP32
-    // two species exact 102.5 / 97.1 (538 / 512); four species with transport
-    // and Cp(T) FP32 262,144 leaves 462 / 424 (417, the adjoint's limit / 512),
-    // FP64 32,768 leaves 201 / 170 (334 / 256; 262,144 leaves 1,060 / 1,072).
+    // Stage at 262,144 leaves, us, at the size above against this one: FP64 one
+    // species LF 105 / 98, HLLC 144 / 131, exact 630 / 562 (528 / 512 faces), two
+    // species LF 220 / 158, HLLC 289 / 203, exact 1,069 / 677 (442 / 256, also by
+    // 128 threads); FP32 two species LF 68 / 63, HLLC 83 / 76, exact 185 / 163 (538
+    // / 512); Cp(T) and transport: one species FP64 538 / 501 (528 / 512), FP32 232 /
+    // 223 (660 / 640), two species FP32 340 / 329 (553 / 512), four FP32 462 / 427
+    // (417, the adjoint's limit / 512) and FP64 1,061 / 1,075 (334 / 256; 32,768
+    // leaves 201 / 170).  Not where it takes more than a quarter of the faces of a
+    // 256-thread workgroup: two species with Cp(T), FP64, 442 / 256, 645 / 738.
     // FP32 one species runs best at its two and a half passes (640: 430; 512:
-    // 462; 768: 462 at level 7).
-    if (faces >= 256 && !(cfg->n_comp == 1 && cfg->precision != CHARM_FP64)) faces &= ~255;
+    // 462; 768: 462 at level 7).  FP32 arithmetic with three and four species: two
+    // passes, three workgroups per CU (465 or 409 / 512 / 256 faces: LF 90 / 77 / 79
+    // and 111 / 85 / 91, HLLC 112 / 90 / 94 and 128 / 97 / 104, exact 184 / 181 /
+    // 194 and 324 / 187 / 202).
+    const int whole = faces & ~255;
+    if (cfg->precision != CHARM_FP64 && !config_physics(cfg)) {
+        if (cfg->n_comp > 1) faces = cfg->n_comp > 2 ? 512 : (whole ? whole : faces);
+    } else if (whole && (!config_physics(cfg) || 4 * whole >= 3 * faces)) {
+        faces = whole;
+    }
     if (faces < 96) faces = 96;
     *cf = faces;
     *ce = faces / 3 > 256 ? 256 : faces / 3;
