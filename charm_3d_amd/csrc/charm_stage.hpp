@@ -440,16 +440,22 @@ __device__ __forceinline__ DevRef chunk_ref(const StageArgs &A, const DevParams 
 // The FP32 deviation-form instances are held to at most 168 VGPRs (three
 // waves per SIMD) so that a change of the code cannot drop them below the
 // occupancy their LDS allows; with the rolled point loop they need 114, and
-// four 40 KB workgroups share a CU.  The FP64 ones are held to two waves (the
-// exact Riemann solver with two species took 264 registers and ran at one).
+// four 40 KB workgroups share a CU.  The FP64 ones are held to two waves, but
+// for the exact Riemann solver with several species, which takes 264-308
+// registers and spills 10-75 of them under that bound: stage with 85-leaf chunks
+// at 32,768 / 83,672 / 262,144 leaves with one and two waves, us, two species
+// 133 318 818 and 198 330 677, three 145 333 873 and 212 379 895, four 143 350
+// 897 and 226 423 1,020.  Two species run a two-wave instance beyond 100,000
+// leaves (launch_stage_bs).
 template <typename R, int NC, int FLUX, int PH>
 constexpr int stage_min_waves()
 {
-    return uses_dev<R, NC, FLUX, PH>() ? 3 : (sizeof(R) == 8 && PH == 0 ? 2 : 1);
+    return uses_dev<R, NC, FLUX, PH>() ? 3
+           : (sizeof(R) == 8 && PH == 0 && (FLUX != FLUX_GODUNOV || NC == 1) ? 2 : 1);
 }
 
-template <typename S, typename R, int NC, int FLUX, int BS, int PH>
-__global__ __launch_bounds__(BS, (stage_min_waves<R, NC, FLUX, PH>()))
+template <typename S, typename R, int NC, int FLUX, int BS, int PH, int WAVES = stage_min_waves<R, NC, FLUX, PH>()>
+__global__ __launch_bounds__(BS, WAVES)
 void k_stage(StageArgs A, DevParams Pv)
 {
     const DevParams &P = stage_params<PH>(A, Pv);
@@ -747,7 +753,15 @@ static hipError_t launch_stage_bs(int flux, const StageArgs &A, const DevParams 
     switch (flux) {
     case FLUX_LF: hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_LF, BS, PH>), grid, block, sh, st, A, P); break;
     case FLUX_HLLC: hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_HLLC, BS, PH>), grid, block, sh, st, A, P); break;
-    case FLUX_GODUNOV: hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_GODUNOV, BS, PH>), grid, block, sh, st, A, P); break;
+    case FLUX_GODUNOV:
+        if constexpr (sizeof(R) == 8 && NC == 2 && PH == 0) {
+            if (A.n_elem > 100000) {
+                hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_GODUNOV, BS, PH, 2>), grid, block, sh, st, A, P);
+                break;
+            }
+        }
+        hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_GODUNOV, BS, PH>), grid, block, sh, st, A, P);
+        break;
     case FLUX_CD: hipLaunchKernelGGL((k_stage<S, R, NC, FLUX_CD, BS, PH>), grid, block, sh, st, A, P); break;
     default: return hipErrorInvalidValue;
     }
