@@ -1210,16 +1210,13 @@ extern "C" int charm_gpu_recommended_chunks(const charm_config_t *cfg, int *ce, 
     // leaves 201 / 170).  Not where it takes more than a quarter of the faces of a
     // 256-thread workgroup: two species with Cp(T), FP64, 442 / 256, 645 / 738.
     // FP32 one species runs best at its two and a half passes (640: 430; 512:
-    // 462; 768: 462 at level 7).  FP32 arithmetic with three and four species: two
-    // passes, three workgroups per CU (465 or 409 / 512 / 256 faces: LF 90 / 77 / 79
-    // and 111 / 85 / 91, HLLC 112 / 90 / 94 and 128 / 97 / 104, exact 184 / 181 /
-    // 194 and 324 / 187 / 202).
+    // 462; 768: 462 at level 7); FP32 arithmetic with three species, but for the
+    // exact solver, at two passes and three workgroups per CU (465 / 512 / 256
+    // faces: LF 90 / 77 / 79, HLLC 112 / 90 / 94).
     const int whole = faces & ~255;
-    if (cfg->precision != CHARM_FP64 && !config_physics(cfg)) {
-        if (cfg->n_comp > 1) faces = cfg->n_comp > 2 ? 512 : (whole ? whole : faces);
-    } else if (whole && (!config_physics(cfg) || 4 * whole >= 3 * faces)) {
-        faces = whole;
-    }
+    const bool fp64 = cfg->precision == CHARM_FP64;
+    if (!fp64 && !config_physics(cfg) && cfg->n_comp == 3 && cfg->flux != CHARM_FLUX_GODUNOV) faces = 512;
+    else if (whole && (fp64 || cfg->n_comp > 1) && (!config_physics(cfg) || 4 * whole >= 3 * faces)) faces = whole;
     if (faces < 96) faces = 96;
     *cf = faces;
     *ce = faces / 3 > 256 ? 256 : faces / 3;
