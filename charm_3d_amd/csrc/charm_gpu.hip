@@ -501,19 +501,26 @@ extern "C" int charm_gpu_destroy(charm_gpu_ctx_t *c)
 // The chunks a context runs a mesh on.  With the flattening's chunks, sized
 // for meshes of many, a small mesh would occupy a few of the 256 CUs and a
 // stage would last as long as one workgroup's serial passes, so its chunks
-// are cut into pieces; every piece keeps its chunk's reference leaf, so the
-// cut changes no bit of the FP32 deviation form.  Stage times (us), uncut and
-// as chosen:
-//   up to 6,000 leaves, pieces of 8 on k_stage_pt: 512 leaves FP64 22 -> 8,
-//     4,096 leaves FP32 21 -> 11, four species 64 -> 47;
-//   up to 12,000 (exact Riemann solver: 24,000), pieces of 16 on k_stage_pt:
-//     9,192 leaves FP64 37 -> 27, exact solver 54 -> 22;
-//   else, one to three species of constant cp: FP32 up to 49,152 pieces of 64
-//     on 256 threads (40,328 leaves 32 -> 25, exact solver 59 -> 44; 86,864
-//     37 -> 36, and the cut adds 0.45 ms to an upload of 53,768), FP64 up to 24,000 pieces of 48 (19,104 leaves 37 -> 30;
-//     at 32,768 the pieces lose, 34 -> 40).
-// A viscous or real-gas mesh beyond the point kernel's sizes stays uncut (104
-// and 105 at 32,768 leaves).
+// are cut into pieces; every piece keeps its chunk's reference leaf.  Stage
+// times, us, uncut / as chosen, at 3,872 / 8,800 / 17,928 / 32,768 (uniform) /
+// 37,472 leaves:
+//   FP32 LF one species 24 25 25 22 26 / 12 18 19 19 22, HLLC 26 28 30 26 31 / 13
+//     19 22 22 26 (mixed 27 28 30 27 32 / 13 23 23 24 27), two species 28 27 27 23
+//     34 / 14 22 24 26 30, three 29 29 30 32 34 / 15 23 26 27 33; exact solver 58 59
+//     62 59 65 / 15 22 34 42 46, two species 56 50 53 52 63 / 16 25 35 49 55;
+//     uncut beyond 49,152 (83,672: pieces of 64 leaves 36 for 34).
+//   FP64 LF 25 24 24 / 15 25 23, HLLC 33 31 32 / 17 28 30, two species 42 43 54 / 20
+//     34 50, four 56 53 75 / 30 46 66; exact solver 120 127 108 / 40 83 102, two
+//     species 137 127 127 / 44 85 127, uncut beyond 12,000 (pieces of 48: 187);
+//     uncut beyond 24,000 (32,768: pieces of 48 40 for 29).
+//   Cp(T) and transport: one species FP64 91 102 / 62 91, FP32 79 93 / 51 76, two
+//     species FP64 107 124 / 85 120, four FP32 140 162 / 102 147 and FP64 163 186 /
+//     136 185; uncut beyond 12,000.
+// Up to 6,000 leaves pieces of 8 on k_stage_pt, up to 12,000 (exact solver in
+// FP32: 24,000) of 16; beyond, pieces of 64 on 256 threads in FP32, of 48 in
+// FP64.  The cut adds 0.05 / 0.14 / 0.25 / 0.4 / 0.5 ms to an upload, what 1-5
+// steps give back up to 8,800 leaves, 10-40 (HLLC) and 3-9 (exact solver) at
+// 17,928 and 25-40 and 8-26 at 37,472.
 struct Pieces {
     charm_pieces_t p;
     int rc, cut, points;
@@ -521,12 +528,13 @@ struct Pieces {
     {
         const bool fp64 = c->prec == CHARM_FP64;
         int e = 0, f = 0;
+        const bool exact = c->cfg.flux == CHARM_FLUX_GODUNOV;
         if (m->n <= 6000) { e = 8; f = 48; points = 1; }
-        else if (m->n <= 12000 || (m->n <= 24000 && c->cfg.flux == CHARM_FLUX_GODUNOV)) { e = 16; f = 80; points = 1; }
+        else if (m->n <= 12000 || (m->n <= 24000 && exact && !fp64)) { e = 16; f = 80; points = 1; }
         if (points && stage_points_smem_bytes(c->prec, c->nc, f, e) > 65536) { e = f = points = 0; }
         if (!points && !c->ph) {
             if (!fp64 && m->n <= 49152) { e = 64; f = 256; }
-            if (fp64 && m->n <= 24000) { e = 48; f = 192; }
+            if (fp64 && m->n <= 24000 && (!exact || c->nc == 1)) { e = 48; f = 192; }
         }
         cut = e && (m->chunk_elems > e || m->chunk_faces > f);
         memset(&p, 0, sizeof(p));

@@ -104,11 +104,12 @@ def test_branch_flips_between_fluxes():
     leaves = shell(4, 1)
     assert 12000 < len(leaves) <= 24000
     print(f"[gpu] n={len(leaves)} branch flips", flush=True)
-    mesh = CA.Forest.from_leaves(leaves).flatten(170, 512)
-    u = state(len(leaves), 1)
+    mesh = CA.Forest.from_leaves(leaves).flatten(85, 256)
+    u = state(len(leaves), 2)
     ctx = []
     for flux in ("GODUNOV", "LF"):
-        ctx.append(CA.GpuContext(CA.make_config(precision=CA.FP64, flux=flux)))
+        ctx.append(CA.GpuContext(CA.make_config(precision=CA.FP64, flux=flux, eos="MIX",
+                                                comp_m=(CA.GAS_R, 0.5 * CA.GAS_R), comp_cp=(3.5, 5.0))))
         ctx[-1].upload_mesh(mesh)
         ctx[-1].set_state(u)
     interior = int((mesh.faces()[:, 1] >= 0).sum())

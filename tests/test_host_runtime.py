@@ -18,9 +18,9 @@ def hip():
     return h
 
 
-def context(level, precision=0, flux="HLLC", chunks=(128, 512), mesh=None):
+def context(level, precision=0, flux="HLLC", chunks=(128, 512), mesh=None, **kw):
     import charm_3d_amd as CA
-    ctx = CA.GpuContext(CA.make_config(precision=precision, flux=flux))
+    ctx = CA.GpuContext(CA.make_config(precision=precision, flux=flux, **kw))
     ctx.upload_mesh(mesh or CA.Forest.uniform(level).flatten(*chunks))
     return ctx
 
@@ -38,17 +38,18 @@ def null_arrays():
 
 
 def branch_flips_across_fluxes():
-    """two contexts on one mesh of 13,824 leaves, which the exact solver's and
-    the other fluxes' contexts cut into other pieces; other leaves, and the
-    same leaves flattened otherwise, are refused"""
+    """two contexts on one mesh of some 13,700 leaves, which the exact solver's
+    and the other fluxes' contexts of two species cut into other pieces; other
+    leaves, and the same leaves flattened otherwise, are refused"""
     import charm_3d_amd as CA
     lv = CA.Forest.uniform(4)
     lv.adapt((np.arange(lv.n) % 3 == 0).astype(np.int8), 5)
     assert 12000 < lv.n < 24000, lv.n
-    mesh = lv.flatten(170, 512)
-    a, b = (context(0, flux=f, mesh=mesh) for f in ("GODUNOV", "HLLC"))
+    mesh = lv.flatten(85, 256)
+    kw = dict(eos="MIX", comp_m=(CA.GAS_R, 0.5 * CA.GAS_R), comp_cp=(3.5, 5.0))
+    a, b = (context(0, flux=f, mesh=mesh, **kw) for f in ("GODUNOV", "HLLC"))
     assert a.hllc_branch_flips(b) == (0, 0) and b.hllc_branch_flips(a) == (0, 0)
-    for other in (context(4), context(0, mesh=lv.flatten(100, 300))):
+    for other in (context(4, **kw), context(0, mesh=lv.flatten(100, 300), **kw)):
         with pytest.raises(CA.CharmError, match="same mesh"):
             a.hllc_branch_flips(other)
 
