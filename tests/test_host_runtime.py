@@ -49,7 +49,7 @@ def branch_flips_across_fluxes():
     kw = dict(eos="MIX", comp_m=(CA.GAS_R, 0.5 * CA.GAS_R), comp_cp=(3.5, 5.0))
     a, b = (context(0, flux=f, mesh=mesh, **kw) for f in ("GODUNOV", "HLLC"))
     assert a.hllc_branch_flips(b) == (0, 0) and b.hllc_branch_flips(a) == (0, 0)
-    for other in (context(4, **kw), context(0, mesh=lv.flatten(100, 300), **kw)):
+    for other in (context(4, chunks=(85, 256), **kw), context(0, mesh=lv.flatten(100, 300), **kw)):
         with pytest.raises(CA.CharmError, match="same mesh"):
             a.hllc_branch_flips(other)
 
