@@ -111,9 +111,9 @@ __device__ __forceinline__ void load_dev(const S *__restrict__ U, int64_t n, int
 }
 
 // The pointwise functions below spell out their fused multiply-adds and let
-// the compiler form no others: the result of a point then does not depend on
-// the kernel it is inlined into, and a mesh gives the same bits however its
-// chunks are cut and whichever kernel runs them.
+// the compiler form no others, so that the result of a point from its traces
+// does not depend on the kernel it is inlined into.  (The traces at volume
+// points, the sums over points and faces and the update are the compiler's.)
 
 // state at a point from its deviation trace t = (dm[3], dE, drho); x = dE less
 // the kinetic-energy deviation, dp = (gamma - 1) x

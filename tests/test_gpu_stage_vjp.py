@@ -7,8 +7,9 @@ forward is the device stage itself.
   outlet and wall faces, for HLLC and LF (FP64);
 * <S_u^T x, v> equals the central difference of <x, S(u)> along v (random
   x, v), 1e-7 relative;
-* the FP32 stage VJP (chunked face-centric kernel) is within 1e-5 of the
-  FP64 one (element-centric kernel)."""
+* the FP32 stage VJP is within 1e-5 of the FP64 one (both by leaves at this
+  size; test_gpu_adj_leaves.py has the chunked kernel and the one with a thread
+  per leaf)."""
 import numpy as np
 import pytest
 import torch
