@@ -8,12 +8,13 @@
 // normal, and its moment sums about the face's middle, FS[4V][nf], in side 0's
 // units.  Both sides' bases are affine in its offsets d from there (b0 = c + d,
 // b1 = o + d r), and so are both sides' sums, which are not stored.  Element
-// pass, one thread per leaf: the volume integral at 8 points (flux tensor against grad phi = e / dh, gravity on the
-// momentum), its six faces' sums (LF[6][n]: face << 1 | side; no atomics), the
-// full 4x4 A^-1, the update and the SSP-RK combine; ahead of the limiter also
-// the cell means of the new state.  The arithmetic is the reference's Euler
-// model (src/models/euler/charm_model.c:66-212, 215-372, 402-433) with the
-// geometry of src/charm_geom.c.
+// pass, one thread per leaf: the volume integral at 8 points (flux tensor
+// against grad phi = e / dh, gravity on the momentum), its six faces' sums
+// (LF[6][n]: face << 1 | side; no atomics), the full 4x4 A^-1, the update and
+// the SSP-RK combine; ahead of the limiter also the cell means of the new
+// state.  The arithmetic is the reference's Euler model
+// (src/models/euler/charm_model.c:66-212, 215-372, 402-433) with the geometry
+// of src/charm_geom.c.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "charm_device.hpp"

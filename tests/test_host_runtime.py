@@ -109,17 +109,18 @@ def blocks_kept_by_other_contexts():
 
 
 def transfer_streams():
-    """streams for large transfers are made once a process has moved 96 MB,
-    are kept across contexts, are shared, and go back when memory runs out"""
+    """streams for large transfers are made by a transfer in once a process has
+    moved 256 MB, or one out at 512, are kept across contexts, are shared, and go
+    back when memory runs out"""
     import charm_3d_amd as CA
     mesh = CA.Forest.uniform(6).flatten(170, 512)        # a state of 42 MB
     ctx = context(0, mesh=mesh)
     u = np.zeros((ctx.n, 5, 4))
     made = []
-    for _ in range(4):
-        ctx.set_state(u)
+    for move in 2 * [lambda: ctx.set_state(u)] + 6 * [ctx.get_state] + 2 * [lambda: ctx.set_state(u)]:
+        move()
         made.append(HIP.hh_streams() - 1)
-    assert made == [0, 0, 4, 4], made
+    assert made == 8 * [0] + [4, 4], made
     ctx.close()
     assert HIP.hh_streams() == 4
     a, b = context(0, mesh=mesh), context(0, mesh=mesh)
@@ -131,7 +132,9 @@ def transfer_streams():
         a.objective(0.1, 1000, [0.0] * 3, [1.0] * 3)
     assert HIP.hh_streams() == 2
     HIP.hh_limit(1 << 32)
-    np.testing.assert_array_equal(a.get_state(), u)
+    for k in range(13):                                  # counted anew, outwards
+        np.testing.assert_array_equal(a.get_state(), u)
+        assert HIP.hh_streams() == (6 if k == 12 else 2), k
 
 
 CASES = {f.__name__: f for f in (null_arrays, branch_flips_across_fluxes, failed_uploads, refused_remesh,
