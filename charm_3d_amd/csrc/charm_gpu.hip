@@ -32,7 +32,6 @@ struct AdjBoundary {
 };
 
 constexpr int kXferParts = 8;              // streams of a large state transfer
-constexpr size_t kXferMake = (size_t) 256 << 20;
 constexpr size_t kPinBytes = 256 * 1024;   // pinned buffer of small transfers
 constexpr size_t kPinHead = 4096;          // error flag and reduction results ahead of it
 constexpr int kLiveBlocks = 96, kIdleBlocks = 48;
@@ -111,21 +110,19 @@ struct Lock {
 } // namespace
 
 // The streams of large transfers, up to kXferParts on each of up to eight
-// devices, shared by the contexts of the process.  Four of them, with the
-// hardware queues behind them, take 15-20 ms to make in a fresh process, what
-// they save over some 250 MB (a state of 42 MB in and out into fresh pages 13.3
-// ms on the context's stream, 8.0 in ranges): they are made by the transfer with
-// which a device's come to kXferMake bytes, and kept from then on, beyond the
-// context (a program that has one context at a time would make them again for
-// each, 4 ms).  A transfer in makes them: streams whose first copies go out run
-// 12% slower both ways from then on (30.8 MB in 0.92 ms against 0.81), so one
-// out makes them only at twice the bytes.  One transfer at a time holds a
-// device's streams; another one meanwhile takes its context's own stream.  They
-// are given back when the device runs out of memory.
+// devices, shared by the contexts of the process.  Four of them with the
+// hardware queues behind them take 15-20 ms to make in a fresh process and 4
+// when it makes them again, and save 1.5 ms of a 13 MB state's way in and out
+// into fresh pages, 5 ms at 42 MB: the first transfer of 12 MB makes them, and
+// they are kept beyond the context (a program that has one context at a time
+// made them again for each).  Made later, by the transfer that has earned them,
+// they cost a short program nothing but ran up to 12% slower from then on in
+// most processes (30.8 MB in 0.92 ms against 0.81).  One transfer at a time holds a device's streams;
+// another one meanwhile takes its context's own stream.  They are given back
+// when the device runs out of memory.
 struct XferStreams {
     hipStream_t s[kXferParts];
     int dev, n, busy;
-    size_t seen;              // bytes of the transfers so far
 };
 static struct {
     pthread_mutex_t mu;
@@ -133,9 +130,8 @@ static struct {
     XferStreams d[8];
 } xfer_pool = {PTHREAD_MUTEX_INITIALIZER, 0, {}};
 
-// the streams of a device for a transfer of so many bytes in or out, at least
-// two and up to `want`, or NULL
-static XferStreams *xfer_acquire(int dev, int want, size_t bytes, bool in)
+// the streams of a device, at least two and up to `want`, or NULL
+static XferStreams *xfer_acquire(int dev, int want)
 {
     Lock lock(&xfer_pool.mu);
     XferStreams *x = NULL;
@@ -146,10 +142,8 @@ static XferStreams *xfer_acquire(int dev, int want, size_t bytes, bool in)
         x = &xfer_pool.d[xfer_pool.n++];
         x->dev = dev;
         x->n = x->busy = 0;
-        x->seen = 0;
     }
-    if (x->seen < 2 * kXferMake) x->seen += bytes;
-    if (x->busy || (x->n < 2 && x->seen < (in ? 1 : 2) * kXferMake)) return NULL;
+    if (x->busy) return NULL;
     int cur = dev;
     if (hipGetDevice(&cur) != hipSuccess || (cur != dev && hipSetDevice(dev) != hipSuccess)) { (void) hipGetLastError(); return NULL; }
     while (x->n < want && hipStreamCreate(&x->s[x->n]) == hipSuccess) x->n++;
@@ -167,7 +161,6 @@ static void xfer_give_back(int dev)
         XferStreams &x = xfer_pool.d[i];
         if (x.dev != dev || x.busy) continue;
         while (x.n > 0) (void) hipStreamDestroy(x.s[--x.n]);
-        x.seen = 0;
     }
 }
 
@@ -821,7 +814,7 @@ static hipError_t state_in(charm_gpu_ctx_t *c, const double *u, void *dst)
         return e != hipSuccess ? e : es;
     }
     const int parts = xfer_parts(bytes);
-    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts, bytes, true) : NULL) {
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
         Xfer x = {c, NULL, dst, u, NULL, s, {}};
         return xfer(x, parts);
     }
@@ -843,7 +836,7 @@ static hipError_t state_out(charm_gpu_ctx_t *c, const void *src, double *u)
         return e;
     }
     const int parts = xfer_parts(bytes);
-    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts, bytes, false) : NULL) {
+    if (XferStreams *s = parts > 1 ? xfer_acquire(c->dev, parts) : NULL) {
         Xfer x = {c, src, NULL, NULL, u, s, {}};
         return xfer(x, parts);
     }
